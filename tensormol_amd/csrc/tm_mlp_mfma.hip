@@ -19,7 +19,18 @@
 // derivative of its features stays in its registers from the forward to the
 // backward pass; only activations / upstream gradients cross waves, through
 // two LDS ping-pong buffers.  The descriptor block streams through LDS in
-// 64-feature chunks, converted from FP32 on the fly.
+// 128-feature chunks, converted from FP32 on the fly, each loaded while the
+// one before it is multiplied.
+//
+// What bounds it: a 64-row tile runs its matrix instructions in 60 % (split
+// mode, D 256) and 44 % (FP16, D 768) of its cycles, the rest being the layer
+// epilogues that the second wave of a SIMD cannot cover, the descriptor reads
+// and the dG writes; at that load the card lowers its clock.  A 32-row tile is
+// bound by the weight fragments, which one CU reads at 40-55 bytes a cycle.
+// Weight fragments as a register ring, streamed descriptors and priorities
+// took the 12,288-atom box from 149 to 130 us (bf16x3f), the 24,000-atom
+// sphere from 244 to 220 us (FP16), a 2,139-atom batch from 78 to 63 us and
+// 192 atoms from 51 to 41 us (bf16x3f).
 //
 // Modes: 0 bf16, 1 fp16 (operands rounded once, FP32 accumulation),
 // 2 bf16 hi/lo split: x = hi + lo for weights and activations and
@@ -34,6 +45,8 @@
 // adds up over a system; rounding activations gives an unbiased error that is
 // decorrelated across atoms, so it averages out over large systems but not
 // over a small molecule: modes 3 and 4 remove the first, mode 5 both.
+#include <type_traits>
+
 #include "tm_common.h"
 
 namespace {
@@ -41,6 +54,16 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef unsigned uint4v __attribute__((ext_vector_type(4)));
+
+// f(0), f(1), ..., f(N - 1) with the index a compile-time constant
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void unroll(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>());
+    unroll<N, I + 1>(f);
+  }
+}
 
 constexpr int NW = 8;       // waves per workgroup
 constexpr int FT = 4;       // 16-feature tiles per wave (64 features)
@@ -102,7 +125,7 @@ struct Ty<0> {
   static __device__ __forceinline__ float back(unsigned short b) {
     return (float)__builtin_bit_cast(__bf16, b);
   }
-  static __device__ __forceinline__ floatx4 mma(const uint4& a, const uint4& b, floatx4 c) {
+  static __device__ __forceinline__ floatx4 mma(const uint4v& a, const uint4v& b, floatx4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
                                                    __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
   }
@@ -115,7 +138,7 @@ struct Ty<1> {
   static __device__ __forceinline__ float back(unsigned short b) {
     return (float)__builtin_bit_cast(_Float16, b);
   }
-  static __device__ __forceinline__ floatx4 mma(const uint4& a, const uint4& b, floatx4 c) {
+  static __device__ __forceinline__ floatx4 mma(const uint4v& a, const uint4v& b, floatx4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
                                                   __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
   }
@@ -150,6 +173,14 @@ __device__ __forceinline__ void act_pair(float z, const ActConst& c, float& act,
   const float r = __builtin_amdgcn_rcpf(1.0f + e);
   act = fmaxf(z, 0.f) + __builtin_amdgcn_logf(1.0f + e) * c.k_log;
   dact = z >= 0.f ? r : e * r;
+}
+
+// x as rounded to FP32: a product fused with its conversion to FP16 in one tile
+// size and not in the other would make an atom's result depend on the tile it
+// sits in
+__device__ __forceinline__ float fp32(float x) {
+  asm("" : "+v"(x));
+  return x;
 }
 
 // Activation derivatives of a wave's features, kept from the forward to the
@@ -197,6 +228,7 @@ struct Smem {
     // layer 1: the whole descriptor tile, row stride D + 8 <= 2 SH
     unsigned short Gt[2 * PL * MT * SH];
   };
+  float bias[4][HMAX];   // b1, b2, b3, w_o
   float epart[NW][MT];
   int atoms[MT];
 };
@@ -205,177 +237,172 @@ struct Smem<MODE, MT, true> {
   static constexpr int PL = act_split_fwd(MODE) ? 2 : 1;
   static constexpr int SH = HMAX + 8;
   unsigned short X[PL][MT][SH];
+  float bias[4][HMAX];
   float epart[NW][MT];
   int atoms[MT];
 };
 
-// write 4 consecutive features (values v) of one atom into an activation
-// buffer; LO: also the lo plane (the residual v - hi, rounded)
-template <int MODE, int MT, bool LO>
-__device__ __forceinline__ void put4(unsigned short (*buf)[MT][HMAX + 8], int atom, int f,
-                                     const float v[4]) {
-  unsigned short h[4];
+// ---- the GEMMs ---------------------------------------------------------------
+// A weight stream: the fragments of one wave's row tiles of one GEMM, taken in
+// substeps.  A k-step (32 k) is one substep, or two with split weights: its hi
+// fragments, then its lo fragments.  Every field is wave-uniform, a byte
+// offset into the blob, so a fragment load is one buffer instruction with a
+// scalar offset.
+struct WStream {
+  int row[FT];   // offset of each row tile's first fragment, hi plane
+  int plane;     // bytes from the hi to the lo plane
+  int nsub;      // substeps
+};
+
+// Row tiles rt0 .. (the last one there is, rtmax, stands in for those past it)
+// of the fragment array at element off, kstride k-steps each.
+__device__ __forceinline__ WStream wstream(long off, long plane_elems, int kstride, int rt0,
+                                           int rtmax, int wp) {
+  WStream s;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) h[i] = Ty<MODE>::cvt(v[i]);
-  uint2 w;
-  w.x = (unsigned)h[0] | ((unsigned)h[1] << 16);
-  w.y = (unsigned)h[2] | ((unsigned)h[3] << 16);
-  *reinterpret_cast<uint2*>(&buf[0][atom][f]) = w;
-  if constexpr (LO) {
-    unsigned short l[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) l[i] = Ty<MODE>::cvt(v[i] - Ty<MODE>::back(h[i]));
-    uint2 u;
-    u.x = (unsigned)l[0] | ((unsigned)l[1] << 16);
-    u.y = (unsigned)l[2] | ((unsigned)l[3] << 16);
-    *reinterpret_cast<uint2*>(&buf[1][atom][f]) = u;
-  }
+  for (int ft = 0; ft < FT; ++ft) s.row[ft] = (int)off * 2 + min(rt0 + ft, rtmax) * kstride * 1024;
+  s.plane = (int)plane_elems * 2;
+  s.nsub = kstride * wp;
+  return s;
 }
 
-// acc[ft][at] += sum over K of W-fragments (rows tiles rt0 + ft) x B from LDS buffer.
-// The weight fragments of k-step ks+1 are in flight while the MFMAs of ks run:
-// two register sets alternate (the loop is unrolled by two; nks is even), and
-// scheduling barriers keep the loads ahead of the MFMAs that do not need them.
-// First weight fragments of a GEMM (k-step 0).  Weights do not depend on LDS,
-// so a wave loads them before the epilogue and barrier that precede the GEMM.
-template <int NFT>
-__device__ __forceinline__ void gemm_first(uint4 (&a)[NFT], const unsigned short* __restrict__ wf,
-                                           int nks, const int* rtile, int lane) {
+// Substep sub of stream s (WP planes per k-step), or, past its end, the
+// substeps of the stream t that follows it (WPN planes).
+template <int WP, int WPN>
+__device__ __forceinline__ void load_sub(uint4v (&set)[FT], __amdgpu_buffer_rsrc_t blob,
+                                         const WStream& s, const WStream& t, int sub, int lane) {
+  const bool over = sub >= s.nsub;
+  const int v = over ? sub - s.nsub : sub;
+  const int off_s = (WP == 2 ? v >> 1 : v) * 1024 + (WP == 2 && (v & 1) ? s.plane : 0);
+  const int off_t = (WPN == 2 ? v >> 1 : v) * 1024 + (WPN == 2 && (v & 1) ? t.plane : 0);
+  const int off = over ? off_t : off_s;
 #pragma unroll
-  for (int ft = 0; ft < NFT; ++ft)
-    a[ft] = *reinterpret_cast<const uint4*>(wf + ((long)(rtile[ft] * nks) * 64 + lane) * 8);
+  for (int ft = 0; ft < FT; ++ft)
+    set[ft] = __builtin_amdgcn_raw_buffer_load_b128(blob, lane * 16,
+                                                    (over ? t.row[ft] : s.row[ft]) + off, 0);
 }
 
-template <int MODE, int MT, int NFT, bool SPLIT>
-__device__ __forceinline__ void gemm_tiles(floatx4 (&acc)[NFT][MT / 16],
-                                           const unsigned short* __restrict__ wf, long plane_elems,
-                                           int nks, int kstride, const int* rtile,
-                                           const unsigned short* bbase, long bplane, int lane,
-                                           int STRIDE, const uint4 (&a_first)[NFT]) {
+// Substeps [s0, s1) of a GEMM: acc[ft][at] += W x B, B read from LDS rows
+// [atom][k] (two planes with XP 2).  Per k-step and accumulator the products
+// are added in the order Whi xhi, Wlo xhi, Whi xlo.
+//
+// What bounds it is the latency of the weight fragments (every fragment is
+// read once per workgroup, from L2 or beyond it), so NS sets of them form a
+// ring: the sets of a k-step are refilled for the k-step NS / WP later as soon
+// as its MFMAs are issued, and past the end of this GEMM with the first
+// fragments of the next one, so that the fragments a layer starts with are on
+// their way during the epilogue before it.  On entry the ring holds substeps
+// s0 .. s0 + NS - 1, on exit those that follow.  The B fragments of the next
+// k-step are read behind the MFMAs of the current one.  s0, s1 and the
+// stream's length are multiples of NS.
+template <int MODE, int MT, int NFT, int WP, int XP, int NS, int WPN>
+__device__ __forceinline__ void gemm_ring(floatx4 (&acc)[NFT][MT / 16], uint4v (&ring)[NS][FT],
+                                          __amdgpu_buffer_rsrc_t blob, const WStream& cur,
+                                          const WStream& nxt, int s0, int s1,
+                                          const unsigned short* bbase, int bplane, int lane,
+                                          int stride) {
   constexpr int AT = MT / 16;
-  const int brow = lane & 15;
-  const int bk = (lane >> 4) * 8;
-  auto afrag = [&](int ft, int ks, long plane) {
-    return *reinterpret_cast<const uint4*>(wf + plane + ((long)(rtile[ft] * kstride + ks) * 64 + lane) * 8);
+  static_assert(NS % WP == 0, "a ring holds whole k-steps");
+  const unsigned short* bp = bbase + (lane & 15) * stride + (lane >> 4) * 8;
+  uint4v bh[AT], bl[XP == 2 ? AT : 1];
+  const int klast = (s1 - s0) / WP - 1;   // last k-step in the buffer
+  auto ldb = [&](int at, int k) {
+    bh[at] = *reinterpret_cast<const uint4v*>(bp + at * 16 * stride + k * 32);
+    if constexpr (XP == 2)
+      bl[at] = *reinterpret_cast<const uint4v*>(bp + bplane + at * 16 * stride + k * 32);
   };
-  auto step = [&](const uint4 (&a)[NFT], int ks) {
-    uint4 b[AT];
 #pragma unroll
-    for (int at = 0; at < AT; ++at)
-      b[at] = *reinterpret_cast<const uint4*>(bbase + (long)(at * 16 + brow) * STRIDE + ks * 32 + bk);
+  for (int at = 0; at < AT; ++at) ldb(at, 0);
+  int sub = s0;
+  do {   // s0 < s1
+    unroll<NS / WP>([&](auto kc) {
+      constexpr int u = decltype(kc)::value * WP;   // the k-step's first set
+      const int kn = min((sub - s0 + u) / WP + 1, klast);
+      if constexpr (WP == 2) {
 #pragma unroll
-    for (int ft = 0; ft < NFT; ++ft)
+        for (int at = 0; at < AT; ++at)
 #pragma unroll
-      for (int at = 0; at < AT; ++at) acc[ft][at] = Ty<MODE>::mma(a[ft], b[at], acc[ft][at]);
-    if constexpr (SPLIT) {
-      uint4 al[NFT], bl[AT];
+          for (int ft = 0; ft < NFT; ++ft)
+            acc[ft][at] = Ty<MODE>::mma(ring[u][ft], bh[at], acc[ft][at]);
+      }
 #pragma unroll
-      for (int ft = 0; ft < NFT; ++ft) al[ft] = afrag(ft, ks, plane_elems);
+      for (int at = 0; at < AT; ++at) {
 #pragma unroll
-      for (int at = 0; at < AT; ++at)
-        bl[at] = *reinterpret_cast<const uint4*>(bbase + bplane + (long)(at * 16 + brow) * STRIDE +
-                                                 ks * 32 + bk);
-#pragma unroll
-      for (int ft = 0; ft < NFT; ++ft)
-#pragma unroll
-        for (int at = 0; at < AT; ++at) {
-          acc[ft][at] = Ty<MODE>::mma(al[ft], b[at], acc[ft][at]);
-          acc[ft][at] = Ty<MODE>::mma(a[ft], bl[at], acc[ft][at]);
+        for (int ft = 0; ft < NFT; ++ft) {
+          acc[ft][at] = Ty<MODE>::mma(ring[u + WP - 1][ft], bh[at], acc[ft][at]);
+          if constexpr (XP == 2) acc[ft][at] = Ty<MODE>::mma(ring[u][ft], bl[at], acc[ft][at]);
         }
-    }
-  };
-  uint4 a0[NFT], a1[NFT];
+        ldb(at, kn);
+      }
 #pragma unroll
-  for (int ft = 0; ft < NFT; ++ft) a0[ft] = a_first[ft];
-  for (int ks = 0; ks < nks; ks += 2) {
-#pragma unroll
-    for (int ft = 0; ft < NFT; ++ft) a1[ft] = afrag(ft, ks + 1, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    step(a0, ks);
-    __builtin_amdgcn_sched_barrier(0);
-    if (ks + 2 < nks) {
-#pragma unroll
-      for (int ft = 0; ft < NFT; ++ft) a0[ft] = afrag(ft, ks + 2, 0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    step(a1, ks + 1);
-    __builtin_amdgcn_sched_barrier(0);
-  }
+      for (int p = 0; p < WP; ++p)
+        load_sub<WP, WPN>(ring[u + p], blob, cur, nxt, sub + u + p + NS, lane);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    sub += NS;
+  } while (sub < s1);
 }
 
-// Split-weight GEMM (mode 3 forward): acc += (Whi + Wlo) x B with one B plane.
-// Each k-step is two MFMA passes over the same B fragments, the hi fragments
-// (a0) then the lo fragments (a1); the lo fragments load while the hi MFMAs
-// run and the next hi fragments while the lo MFMAs run, so the register
-// footprint and the load-ahead distance are those of gemm_tiles.
-template <int MODE, int MT, int NFT>
-__device__ __forceinline__ void gemm_tiles_ws(floatx4 (&acc)[NFT][MT / 16],
-                                              const unsigned short* __restrict__ wf,
-                                              long plane_elems, int nks, int kstride,
-                                              const int* rtile, const unsigned short* bbase,
-                                              int lane, int STRIDE, const uint4 (&a_first)[NFT]) {
-  constexpr int AT = MT / 16;
-  const int brow = lane & 15;
-  const int bk = (lane >> 4) * 8;
-  auto afrag = [&](int ft, int ks, long plane) {
-    return *reinterpret_cast<const uint4*>(wf + plane + ((long)(rtile[ft] * kstride + ks) * 64 + lane) * 8);
-  };
-  uint4 a0[NFT], a1[NFT];
-#pragma unroll
-  for (int ft = 0; ft < NFT; ++ft) a0[ft] = a_first[ft];
-  for (int ks = 0; ks < nks; ++ks) {
-#pragma unroll
-    for (int ft = 0; ft < NFT; ++ft) a1[ft] = afrag(ft, ks, plane_elems);
-    __builtin_amdgcn_sched_barrier(0);
-    uint4 b[AT];
-#pragma unroll
-    for (int at = 0; at < AT; ++at)
-      b[at] = *reinterpret_cast<const uint4*>(bbase + (long)(at * 16 + brow) * STRIDE + ks * 32 + bk);
-#pragma unroll
-    for (int ft = 0; ft < NFT; ++ft)
-#pragma unroll
-      for (int at = 0; at < AT; ++at) acc[ft][at] = Ty<MODE>::mma(a0[ft], b[at], acc[ft][at]);
-    __builtin_amdgcn_sched_barrier(0);
-    if (ks + 1 < nks) {
-#pragma unroll
-      for (int ft = 0; ft < NFT; ++ft) a0[ft] = afrag(ft, ks + 1, 0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int ft = 0; ft < NFT; ++ft)
-#pragma unroll
-      for (int at = 0; at < AT; ++at) acc[ft][at] = Ty<MODE>::mma(a1[ft], b[at], acc[ft][at]);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-}
+template <int MODE, int MT>
+constexpr bool shares_cu() { return MT == 32 && !act_split_fwd(MODE); }
+// Weight fragment sets in flight: four (64 of the 256 registers a lane has; the
+// split mode's 32-row tiles have room for eight and gain nothing by them: 62.9
+// against 65.1 us on 2,139 C/H/N/O atoms), two in the 32-row tiles that share a
+// CU (128 registers).  Four need widths that make every stream a multiple of
+// the ring, which 128-wide ones do; any other width takes the kernel with two.
+template <int MODE, int MT>
+constexpr int ring_sets() { return shares_cu<MODE, MT>() ? 2 : 4; }
+inline bool ring_fits(int D, int H) { return D % 128 == 0 && H % 128 == 0; }
 
-// Forward GEMM of a layer: split weights only (modes 3, 4), split weights and
-// activations (modes 2, 5), or one rounding of each (modes 0, 1).
-template <int MODE, int MT, int NFT>
-__device__ __forceinline__ void gemm_fwd(floatx4 (&acc)[NFT][MT / 16],
-                                         const unsigned short* __restrict__ wf, long plane_elems,
-                                         int nks, int kstride, const int* rtile,
-                                         const unsigned short* bbase, long bplane, int lane,
-                                         int STRIDE, const uint4 (&a_first)[NFT]) {
-  if constexpr (MODE == 3 || MODE == 4)
-    gemm_tiles_ws<MODE, MT, NFT>(acc, wf, plane_elems, nks, kstride, rtile, bbase, lane, STRIDE,
-                                 a_first);
-  else
-    gemm_tiles<MODE, MT, NFT, act_split_fwd(MODE)>(acc, wf, plane_elems, nks, kstride, rtile,
-                                                   bbase, bplane, lane, STRIDE, a_first);
-}
+// One layer's values of a wave, rounded for the activation buffer: hi plane,
+// and the lo plane where the forward operands are split.
+template <int MODE, int MT, bool LO>
+struct Packed {
+  uint2 h[FT][MT / 16], l[LO ? FT : 1][LO ? MT / 16 : 1];
+  __device__ __forceinline__ void set(int ft, int at, const float v[4]) {
+    unsigned short x[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = Ty<MODE>::cvt(v[i]);
+    h[ft][at] = make_uint2((unsigned)x[0] | ((unsigned)x[1] << 16),
+                           (unsigned)x[2] | ((unsigned)x[3] << 16));
+    // packed here, not where it is stored: the FP32 values would stay live
+    asm volatile("" : "+v"(h[ft][at].x), "+v"(h[ft][at].y));
+    if constexpr (LO) {
+      unsigned short y[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y[i] = Ty<MODE>::cvt(v[i] - Ty<MODE>::back(x[i]));
+      l[ft][at] = make_uint2((unsigned)y[0] | ((unsigned)y[1] << 16),
+                             (unsigned)y[2] | ((unsigned)y[3] << 16));
+      asm volatile("" : "+v"(l[ft][at].x), "+v"(l[ft][at].y));
+    }
+  }
+  // features 64 w + 16 ft + fq .. + 3 of atom 16 at + ca
+  __device__ __forceinline__ void store(unsigned short (*buf)[MT][HMAX + 8], int w, int fq,
+                                        int ca) const {
+#pragma unroll
+    for (int ft = 0; ft < FT; ++ft)
+#pragma unroll
+      for (int at = 0; at < MT / 16; ++at) {
+        const int f = 64 * w + 16 * ft + fq;
+        *reinterpret_cast<uint2*>(&buf[0][at * 16 + ca][f]) = h[ft][at];
+        if constexpr (LO) *reinterpret_cast<uint2*>(&buf[1][at * 16 + ca][f]) = l[ft][at];
+      }
+  }
+};
 
 // 64-row tiles: one workgroup per CU (LDS); 32-row tiles in the BF16 / FP16
 // modes fit two workgroups per CU when the waves stay within 128 VGPRs.
-template <int MODE, int MT>
+template <int MODE, int MT, int NS>
 __global__ void __launch_bounds__(NW * 64)
-__attribute__((amdgpu_waves_per_eu(MT == 32 && !act_split_fwd(MODE) ? 4 : 2)))
+__attribute__((amdgpu_waves_per_eu(shares_cu<MODE, MT>() ? 4 : 2)))
 mlp_mfma_kernel(MlpArgs a) {
   constexpr int AT = MT / 16;
   constexpr bool LOF = act_split_fwd(MODE);   // forward operands carry lo planes
   constexpr bool LOB = act_split_bwd(MODE);   // backward operands carry lo planes
   constexpr bool INPLACE = in_place<MODE, MT>();
   constexpr int SH = HMAX + 8;
+  constexpr int WPF = fwd_planes(MODE), WPB = bwd_planes(MODE);
+  constexpr int XPF = LOF ? 2 : 1, XPB = LOB ? 2 : 1;
   typedef Smem<MODE, MT> S;
   __shared__ S sm;
   // output buffer of layers 2, bwd 3 (read by layer 3, bwd 2): Y, or X in place
@@ -383,7 +410,7 @@ mlp_mfma_kernel(MlpArgs a) {
     if constexpr (INPLACE) return sm.X; else return sm.Y;
   }();
   const int tid = threadIdx.x;
-  const int w = tid >> 6, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int tile = blockIdx.x;
   const int s = a.tiles[2 * tile], row0 = a.tiles[2 * tile + 1];
   if (s < 0) return;   // padding of the XCD-ordered tile table (whole workgroup)
@@ -393,267 +420,281 @@ mlp_mfma_kernel(MlpArgs a) {
   const BlobLayout BL = blob_layout(D, H, fwd_planes(MODE), bwd_planes(MODE));
   const unsigned short* wb = a.blobs[blob];
   const float* fsec = reinterpret_cast<const float*>(reinterpret_cast<const char*>(wb) + BL.bias_bytes);
-  const float* b1 = fsec;
-  const float* b2 = fsec + H;
-  const float* b3 = fsec + 2 * H;
-  const float* wo = fsec + 3 * H;
-  const float bo = fsec[4 * H];
-  if (tid < MT) {
-    int r = row0 + tid;
-    sm.atoms[tid] = r < rows ? a.perm[first + r] : -1;
-  }
+  // The two waves of a SIMD run the same layer between two barriers.  With
+  // different priorities the first finishes its MFMAs early and does its
+  // epilogue under the MFMAs of the second, instead of both at the same time
+  // (45.4 -> 43.3 us on 192 atoms, 223 -> 220 us on the 24,000-atom sphere).
+  if (w < NW / 2) __builtin_amdgcn_s_setprio(2);
   const bool wact = (w * 64) < H;   // this wave owns hidden features
-  int rt[FT];
-#pragma unroll
-  for (int ft = 0; ft < FT; ++ft) rt[ft] = 4 * w + ft;
   const int fq = (lane >> 4) * 4;   // first of the 4 features this lane holds in a C tile
   const int ca = lane & 15;         // atom column of this lane in a C tile
   // activation derivatives of layers 1 and 2 for this wave's features
   DerivRegs<MODE, FT, AT> s1, s2;
   const ActConst ac = act_const(a.alpha);
-  floatx4 acc[FT][AT];
-  const long phh = frag_elems(H / 16, H / 32);
-  uint4 pf[FT];   // first weight fragments of the next GEMM, loaded early
-  if (wact) gemm_first<FT>(pf, wb + BL.f1, D / 32, rt, lane);
+  const long phh = frag_elems(H / 16, H / 32), p1 = frag_elems(H / 16, D / 32);
+  const int hk = H / 32, hmax = H / 16 - 1, ntile = D / 16;
+  __amdgpu_buffer_rsrc_t blob_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<unsigned short*>(wb), 0, (int)BL.bias_bytes, 0x00020000);
+  const WStream W1 = wstream(BL.f1, p1, D / 32, FT * w, hmax, WPF);
+  const WStream W2 = wstream(BL.f2, phh, hk, FT * w, hmax, WPF);
+  const WStream W3 = wstream(BL.f3, phh, hk, FT * w, hmax, WPF);
+  const WStream V3 = wstream(BL.b3, phh, hk, FT * w, hmax, WPB);
+  const WStream V2 = wstream(BL.b2, phh, hk, FT * w, hmax, WPB);
+  // backward 1: dG tiles [nf1 w, nf1 w + nf1), then + nf1 NW, ...; three tiles
+  // per pass where that divides the tiles of a wave, else two
+  const int nf1 = (ntile + NW - 1) / NW % 3 == 0 ? 3 : 2;
+  auto w1stream = [&](int t0) {
+    return wstream(BL.b1, frag_elems(ntile, hk), hk, t0, ntile - 1, WPB);
+  };
+  uint4v ring[NS][FT];
+  if (wact) {
+#pragma unroll
+    for (int u = 0; u < NS; ++u) load_sub<WPF, WPF>(ring[u], blob_rsrc, W1, W2, u, lane);
+  }
+  // the four values of row `layer` of sm.bias this lane's features take
+  auto bias4 = [&](int layer, int ft) {
+    return *reinterpret_cast<const floatx4*>(&sm.bias[layer][64 * w + 16 * ft + fq]);
+  };
+  auto clear = [&](floatx4 (&acc)[FT][AT]) {
+#pragma unroll
+    for (int ft = 0; ft < FT; ++ft)
+#pragma unroll
+      for (int at = 0; at < AT; ++at) acc[ft][at] = floatx4{0.f, 0.f, 0.f, 0.f};
+  };
+  const int bpl = MT * SH;   // element offset of the lo plane
 
   // ------------------------------------------------------------ layer 1
+  // The descriptor tile G[atom][0 .. D) streams through LDS in chunks of CW
+  // columns: a chunk is loaded while the one before it is multiplied.  In
+  // place, the chunks take the buffer's columns in turn (chunk c + HMAX / CW
+  // overwrites chunk c, which every wave finished two barriers earlier);
+  // otherwise the whole tile is laid out across both buffers, row stride D + 8.
+  floatx4 acc1[FT][AT];
+  clear(acc1);
+  {
+    constexpr int CW = 128;
+    constexpr int GL = MT * CW / 4 / (NW * 64);   // float4 loads per thread and chunk
+    const int SG = INPLACE ? SH : D + 8;
+    const int gpl = MT * SG;
+    unsigned short* Gt = reinterpret_cast<unsigned short*>(&sm);
+    int atoms[GL];
 #pragma unroll
-  for (int ft = 0; ft < FT; ++ft)
+    for (int i = 0; i < GL; ++i) {
+      const int r = row0 + (tid >> 5) + 16 * i;
+      atoms[i] = r < rows ? a.perm[first + r] : -1;
+      if ((tid & 31) == 0) sm.atoms[(tid >> 5) + 16 * i] = atoms[i];
+    }
+    for (int t = tid; t < 4 * H; t += NW * 64) sm.bias[t / H][t % H] = fsec[t];
+    const int c4 = (tid & 31) * 4;
+    float4 g[GL];
+    auto fetch = [&](int c0) {
 #pragma unroll
-    for (int at = 0; at < AT; ++at) acc[ft][at] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const long p1 = frag_elems(H / 16, D / 32);
-  const long bpl = (long)MT * SH;   // element offset of the lo plane
-  if constexpr (INPLACE) {
-    // the descriptor tile G[atom][0 .. D) streams through the buffer in
-    // column blocks of up to HMAX features (one block when D <= HMAX)
-    for (int c0 = 0; c0 < D; c0 += HMAX) {
-      const int cw = min(HMAX, D - c0);
-      __syncthreads();   // atoms known; every wave done with the previous block
-      for (int e = tid; e < MT * cw / 4; e += NW * 64) {
-        int r = e / (cw / 4), c4 = (e % (cw / 4)) * 4;
-        int atom = sm.atoms[r];
-        float4 g = atom >= 0 ? *reinterpret_cast<const float4*>(a.G + (long)atom * a.ldg + c0 + c4)
-                             : make_float4(0.f, 0.f, 0.f, 0.f);
-        float v[4] = {g.x, g.y, g.z, g.w};
-        put4<MODE, MT, LOF>(sm.X, r, c4, v);
+      for (int i = 0; i < GL; ++i)
+        g[i] = (atoms[i] >= 0 && c0 + c4 < D)
+                   ? *reinterpret_cast<const float4*>(a.G + (long)atoms[i] * a.ldg + c0 + c4)
+                   : make_float4(0.f, 0.f, 0.f, 0.f);
+    };
+    fetch(0);
+    for (int c0 = 0; c0 < D; c0 += CW) {
+      const int lc = INPLACE ? c0 & (HMAX - 1) : c0;
+      if (c0 + c4 < D) {
+#pragma unroll
+        for (int i = 0; i < GL; ++i) {
+          const float v[4] = {g[i].x, g[i].y, g[i].z, g[i].w};
+          unsigned short* dst = Gt + (long)((tid >> 5) + 16 * i) * SG + lc + c4;
+          unsigned short h[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) h[q] = Ty<MODE>::cvt(v[q]);
+          *reinterpret_cast<uint2*>(dst) = make_uint2((unsigned)h[0] | ((unsigned)h[1] << 16),
+                                                      (unsigned)h[2] | ((unsigned)h[3] << 16));
+          if constexpr (LOF) {
+            unsigned short l[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) l[q] = Ty<MODE>::cvt(v[q] - Ty<MODE>::back(h[q]));
+            *reinterpret_cast<uint2*>(dst + gpl) =
+                make_uint2((unsigned)l[0] | ((unsigned)l[1] << 16),
+                           (unsigned)l[2] | ((unsigned)l[3] << 16));
+          }
+        }
       }
+      if (c0 + CW < D) fetch(c0 + CW);
       __syncthreads();
       if (wact) {
-        if (c0 > 0) gemm_first<FT>(pf, wb + BL.f1 + (long)(c0 / 32) * 512, D / 32, rt, lane);
-        gemm_fwd<MODE, MT, FT>(acc, wb + BL.f1 + (long)(c0 / 32) * 512, p1, cw / 32, D / 32, rt,
-                               &sm.X[0][0][0], bpl, lane, SH, pf);
+        gemm_ring<MODE, MT, FT, WPF, XPF, NS, WPF>(
+            acc1, ring, blob_rsrc, W1, W2, c0 / 32 * WPF, min(c0 + CW, D) / 32 * WPF, Gt + lc, gpl, lane, SG);
       }
     }
-  } else {
-    // the whole descriptor tile G[atom][0 .. D) (hi / lo), row stride D + 8,
-    // across both buffers
-    const int SG = D + 8;
-    __syncthreads();
-    for (int e = tid; e < MT * D / 4; e += NW * 64) {
-      int r = e / (D / 4), c4 = (e % (D / 4)) * 4;
-      int atom = sm.atoms[r];
-      float4 g = atom >= 0 ? *reinterpret_cast<const float4*>(a.G + (long)atom * a.ldg + c4)
-                           : make_float4(0.f, 0.f, 0.f, 0.f);
-      float v[4] = {g.x, g.y, g.z, g.w};
-      unsigned short* dst = sm.Gt + (long)r * SG + c4;
-      unsigned short h[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) h[i] = Ty<MODE>::cvt(v[i]);
-      uint2 ww;
-      ww.x = (unsigned)h[0] | ((unsigned)h[1] << 16);
-      ww.y = (unsigned)h[2] | ((unsigned)h[3] << 16);
-      *reinterpret_cast<uint2*>(dst) = ww;
-      if constexpr (LOF) {
-        unsigned short l[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) l[i] = Ty<MODE>::cvt(v[i] - Ty<MODE>::back(h[i]));
-        uint2 u;
-        u.x = (unsigned)l[0] | ((unsigned)l[1] << 16);
-        u.y = (unsigned)l[2] | ((unsigned)l[3] << 16);
-        *reinterpret_cast<uint2*>(dst + (long)MT * SG) = u;
-      }
-    }
-    __syncthreads();
-    if (wact)
-      gemm_fwd<MODE, MT, FT>(acc, wb + BL.f1, p1, D / 32, D / 32, rt, sm.Gt, (long)MT * SG, lane,
-                             SG, pf);
   }
-  if (wact) gemm_first<FT>(pf, wb + BL.f2, H / 32, rt, lane);
-  __syncthreads();   // every wave has read the tile before it is overwritten
-  // epilogue 1 -> X, s1
-  if (wact) {
+  // act(z) of a hidden layer, and its derivative for the backward pass
+  auto epilogue = [&](int layer, const floatx4 (&acc)[FT][AT], auto& P, auto& ds) {
+#pragma unroll
+    for (int ft = 0; ft < FT; ++ft) {
+      const floatx4 b = bias4(layer, ft);
+#pragma unroll
+      for (int at = 0; at < AT; ++at) {
+        float v[4], d[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) act_pair(acc[ft][at][i] + b[i], ac, v[i], d[i]);
+        ds.set4(ft, at, d);
+        P.set(ft, at, v);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+  // dZ = dH * act'
+  auto scale = [&](const floatx4 (&acc)[FT][AT], auto& P, const auto& ds) {
 #pragma unroll
     for (int ft = 0; ft < FT; ++ft)
 #pragma unroll
       for (int at = 0; at < AT; ++at) {
-        int f = 64 * w + 16 * ft + fq;
-        float v[4], d[4];
+        float v[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) act_pair(acc[ft][at][i] + b1[f + i], ac, v[i], d[i]);
-        s1.set4(ft, at, d);
-        put4<MODE, MT, LOF>(sm.X, at * 16 + ca, f, v);
+        for (int i = 0; i < 4; ++i) v[i] = fp32(acc[ft][at][i] * ds.get(ft, at, i));
+        P.set(ft, at, v);
+        __builtin_amdgcn_sched_barrier(0);
       }
+  };
+  {
+    Packed<MODE, MT, LOF> P;
+    if (wact) epilogue(0, acc1, P, s1);
+    __syncthreads();   // every wave has read the tile before it is overwritten
+    if (wact) P.store(sm.X, w, fq, ca);
   }
   __syncthreads();
   // ------------------------------------------------------------ layer 2
-  if (wact) {
-#pragma unroll
-    for (int ft = 0; ft < FT; ++ft)
-#pragma unroll
-      for (int at = 0; at < AT; ++at) acc[ft][at] = floatx4{0.f, 0.f, 0.f, 0.f};
-    gemm_fwd<MODE, MT, FT>(acc, wb + BL.f2, phh, H / 32, H / 32, rt, &sm.X[0][0][0], bpl, lane, SH, pf);
-    gemm_first<FT>(pf, wb + BL.f3, H / 32, rt, lane);
-  }
-  if constexpr (INPLACE) __syncthreads();
-  if (wact) {
-#pragma unroll
-    for (int ft = 0; ft < FT; ++ft)
-#pragma unroll
-      for (int at = 0; at < AT; ++at) {
-        int f = 64 * w + 16 * ft + fq;
-        float v[4], d[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) act_pair(acc[ft][at][i] + b2[f + i], ac, v[i], d[i]);
-        s2.set4(ft, at, d);
-        put4<MODE, MT, LOF>(Yb, at * 16 + ca, f, v);
-      }
+  {
+    Packed<MODE, MT, LOF> P;
+    if (wact) {
+      floatx4 acc[FT][AT];
+      clear(acc);
+      gemm_ring<MODE, MT, FT, WPF, XPF, NS, WPF>(acc, ring, blob_rsrc, W2, W3, 0, W2.nsub,
+                                                 &sm.X[0][0][0], bpl, lane, SH);
+      epilogue(1, acc, P, s2);
+    }
+    if constexpr (INPLACE) __syncthreads();
+    if (wact) P.store(Yb, w, fq, ca);
   }
   __syncthreads();
   // ------------------------------------------------------------ layer 3 + head
-  if (wact) {
+  {
+    Packed<MODE, MT, LOB> P;
+    if (wact) {
+      floatx4 acc[FT][AT];
+      clear(acc);
+      gemm_ring<MODE, MT, FT, WPF, XPF, NS, WPB>(acc, ring, blob_rsrc, W3, V3, 0, W3.nsub,
+                                                 &Yb[0][0][0], bpl, lane, SH);
+      float ep[AT];
 #pragma unroll
-    for (int ft = 0; ft < FT; ++ft)
+      for (int at = 0; at < AT; ++at) ep[at] = 0.f;
 #pragma unroll
-      for (int at = 0; at < AT; ++at) acc[ft][at] = floatx4{0.f, 0.f, 0.f, 0.f};
-    gemm_fwd<MODE, MT, FT>(acc, wb + BL.f3, phh, H / 32, H / 32, rt, &Yb[0][0][0], bpl, lane, SH, pf);
-    gemm_first<FT>(pf, wb + BL.b3, H / 32, rt, lane);
-  }
-  if constexpr (INPLACE) __syncthreads();
-  if (wact) {
-    float ep[AT];
+      for (int ft = 0; ft < FT; ++ft) {
+        const floatx4 b = bias4(2, ft), wv = bias4(3, ft);
 #pragma unroll
-    for (int at = 0; at < AT; ++at) ep[at] = 0.f;
+        for (int at = 0; at < AT; ++at) {
+          float v[4];
 #pragma unroll
-    for (int ft = 0; ft < FT; ++ft)
-#pragma unroll
-      for (int at = 0; at < AT; ++at) {
-        int f = 64 * w + 16 * ft + fq;
-        float v[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float wv = wo[f + i];
-          float act, d;
-          act_pair(acc[ft][at][i] + b3[f + i], ac, act, d);
-          ep[at] += act * wv;
-          v[i] = wv * d;   // dZ3 with upstream 1
+          for (int i = 0; i < 4; ++i) {
+            float act, d;
+            act_pair(acc[ft][at][i] + b[i], ac, act, d);
+            ep[at] += act * wv[i];
+            v[i] = fp32(wv[i] * d);   // dZ3 with upstream 1
+          }
+          P.set(ft, at, v);
+          asm volatile("" : "+v"(ep[at]));   // summed here, not sunk to its use
+          __builtin_amdgcn_sched_barrier(0);
         }
-        put4<MODE, MT, LOB>(sm.X, at * 16 + ca, f, v);
       }
 #pragma unroll
-    for (int at = 0; at < AT; ++at) {
-      float p = ep[at];
-      p += __shfl_xor(p, 16, 64);
-      p += __shfl_xor(p, 32, 64);
-      if (lane < 16) sm.epart[w][at * 16 + lane] = p;
+      for (int at = 0; at < AT; ++at) {
+        float p = ep[at];
+        p += __shfl_xor(p, 16, 64);
+        p += __shfl_xor(p, 32, 64);
+        if (lane < 16) sm.epart[w][at * 16 + lane] = p;
+      }
+    } else {
+      for (int t = lane; t < MT; t += 64) sm.epart[w][t] = 0.f;
     }
-  } else {
-    for (int t = lane; t < MT; t += 64) sm.epart[w][t] = 0.f;
+    if constexpr (INPLACE) __syncthreads();
+    if (wact) P.store(sm.X, w, fq, ca);
   }
   __syncthreads();
   if (tid < MT) {
     int atom = sm.atoms[tid];
     if (atom >= 0) {
-      float yv = bo;
+      float yv = fsec[4 * H];
 #pragma unroll
       for (int q = 0; q < NW; ++q) yv += sm.epart[q][tid];
       a.y[(long)net * a.N + atom] = yv;
     }
   }
   // ------------------------------------------------------------ backward 3: dZ3 -> dZ2
-  if (wact) {
-#pragma unroll
-    for (int ft = 0; ft < FT; ++ft)
-#pragma unroll
-      for (int at = 0; at < AT; ++at) acc[ft][at] = floatx4{0.f, 0.f, 0.f, 0.f};
-    gemm_tiles<MODE, MT, FT, LOB>(acc, wb + BL.b3, phh, H / 32, H / 32, rt, &sm.X[0][0][0], bpl, lane,
-                                  SH, pf);
-    gemm_first<FT>(pf, wb + BL.b2, H / 32, rt, lane);
-  }
-  if constexpr (INPLACE) __syncthreads();
-  if (wact) {
-#pragma unroll
-    for (int ft = 0; ft < FT; ++ft)
-#pragma unroll
-      for (int at = 0; at < AT; ++at) {
-        int f = 64 * w + 16 * ft + fq;
-        float v[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = acc[ft][at][i] * s2.get(ft, at, i);
-        put4<MODE, MT, LOB>(Yb, at * 16 + ca, f, v);
-      }
+  {
+    Packed<MODE, MT, LOB> P;
+    if (wact) {
+      floatx4 acc[FT][AT];
+      clear(acc);
+      gemm_ring<MODE, MT, FT, WPB, XPB, NS, WPB>(acc, ring, blob_rsrc, V3, V2, 0, V3.nsub,
+                                                 &sm.X[0][0][0], bpl, lane, SH);
+      scale(acc, P, s2);
+    }
+    if constexpr (INPLACE) __syncthreads();
+    if (wact) P.store(Yb, w, fq, ca);
   }
   __syncthreads();
   // ------------------------------------------------------------ backward 2: dZ2 -> dZ1
-  if (wact) {
+  const WStream V1 = w1stream(nf1 * w);
+  {
+    Packed<MODE, MT, LOB> P;
+    if (wact) {
+      floatx4 acc[FT][AT];
+      clear(acc);
+      gemm_ring<MODE, MT, FT, WPB, XPB, NS, WPB>(acc, ring, blob_rsrc, V2, V1, 0, V2.nsub,
+                                                 &Yb[0][0][0], bpl, lane, SH);
+      scale(acc, P, s1);
+    } else {
 #pragma unroll
-    for (int ft = 0; ft < FT; ++ft)
-#pragma unroll
-      for (int at = 0; at < AT; ++at) acc[ft][at] = floatx4{0.f, 0.f, 0.f, 0.f};
-    gemm_tiles<MODE, MT, FT, LOB>(acc, wb + BL.b2, phh, H / 32, H / 32, rt, &Yb[0][0][0], bpl, lane,
-                                  SH, pf);
-  }
-  if constexpr (INPLACE) __syncthreads();
-  if (wact) {
-#pragma unroll
-    for (int ft = 0; ft < FT; ++ft)
-#pragma unroll
-      for (int at = 0; at < AT; ++at) {
-        int f = 64 * w + 16 * ft + fq;
-        float v[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = acc[ft][at][i] * s1.get(ft, at, i);
-        put4<MODE, MT, LOB>(sm.X, at * 16 + ca, f, v);
-      }
-  }
-  uint4 pf2[2];   // first fragments of backward 1 (rows of dG tiles w, w + NW)
-  if (w < D / 16) {
-    int r0[2] = {w, w + NW < D / 16 ? w + NW : w};
-    gemm_first<2>(pf2, wb + BL.b1, H / 32, r0, lane);
+      for (int u = 0; u < NS; ++u) load_sub<WPB, WPB>(ring[u], blob_rsrc, V1, V1, u, lane);
+    }
+    if constexpr (INPLACE) __syncthreads();
+    if (wact) P.store(sm.X, w, fq, ca);
   }
   __syncthreads();
   // ------------------------------------------------------------ backward 1: dZ1 -> dG
-  {
-    const long pd = frag_elems(D / 16, H / 32);
-    float* dGn = a.dG + (long)net * a.N * a.ldg;
-    const int ntile = D / 16;
-    for (int t0 = w; t0 < ntile; t0 += 2 * NW) {
-      int rt2[2] = {t0, t0 + NW < ntile ? t0 + NW : t0};
-      floatx4 acc2[2][AT];
+  float* dGn = a.dG + (long)net * a.N * a.ldg;
+  auto backward1 = [&](auto nf) {
+    constexpr int NF1 = decltype(nf)::value;
+    for (int t0 = NF1 * w; t0 < ntile; t0 += NF1 * NW) {
+      const WStream c = w1stream(t0), n = w1stream(min(t0 + NF1 * NW, ntile - 1));
+      floatx4 acc2[NF1][AT];
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
+      for (int u = 0; u < NF1; ++u)
 #pragma unroll
         for (int at = 0; at < AT; ++at) acc2[u][at] = floatx4{0.f, 0.f, 0.f, 0.f};
-      gemm_tiles<MODE, MT, 2, LOB>(acc2, wb + BL.b1, pd, H / 32, H / 32, rt2, &sm.X[0][0][0], bpl, lane,
-                                   SH, pf2);
-      const int tn = t0 + 2 * NW;   // the next iteration's first fragments
-      if (tn < ntile) {
-        int rn[2] = {tn, tn + NW < ntile ? tn + NW : tn};
-        gemm_first<2>(pf2, wb + BL.b1, H / 32, rn, lane);
-      }
+      gemm_ring<MODE, MT, NF1, WPB, XPB, NS, WPB>(acc2, ring, blob_rsrc, c, n, 0, c.nsub,
+                                                  &sm.X[0][0][0], bpl, lane, SH);
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        if (u == 1 && rt2[1] == rt2[0]) continue;
+      for (int at = 0; at < AT; ++at) {
+        const int atom = sm.atoms[at * 16 + ca];
+        if (atom < 0) continue;
 #pragma unroll
-        for (int at = 0; at < AT; ++at) {
-          int atom = sm.atoms[at * 16 + ca];
-          if (atom < 0) continue;
-          int f = 16 * rt2[u] + fq;
-          *reinterpret_cast<float4*>(dGn + (long)atom * a.ldg + f) =
-              make_float4(acc2[u][at][0], acc2[u][at][1], acc2[u][at][2], acc2[u][at][3]);
-        }
+        for (int u = 0; u < NF1; ++u)
+          if (t0 + u < ntile)
+            *reinterpret_cast<float4*>(dGn + (long)atom * a.ldg + 16 * (t0 + u) + fq) =
+                make_float4(acc2[u][at][0], acc2[u][at][1], acc2[u][at][2], acc2[u][at][3]);
       }
     }
-  }
+  };
+  if (nf1 == 3) backward1(std::integral_constant<int, 3>());
+  else backward1(std::integral_constant<int, 2>());
+}
+
+template <int MODE, int MT>
+void launch(const MlpArgs& a, size_t pad, hipStream_t s) {
+  constexpr int NS = ring_sets<MODE, MT>();
+  if (NS == 2 || ring_fits(a.D, a.H))
+    mlp_mfma_kernel<MODE, MT, NS><<<a.ntiles, NW * 64, pad, s>>>(a);
+  else
+    mlp_mfma_kernel<MODE, MT, 2><<<a.ntiles, NW * 64, pad, s>>>(a);
 }
 
 }  // namespace
@@ -720,17 +761,15 @@ int tm_mlp_mfma(int N, int D, int H, int ntiles, const int* tiles, const int* se
     const size_t lds = mode == 5 ? sizeof(Smem<5, 32>) : sizeof(Smem<0, 32>);
     if (ntiles <= ncu && lds < 81920) pad = 81920 - lds + 256;
   }
-  if (mode == 0 && tile_rows == 64) mlp_mfma_kernel<0, 64><<<ntiles, NW * 64, 0, s>>>(a);
-  else if (mode == 0) mlp_mfma_kernel<0, 32><<<ntiles, NW * 64, pad, s>>>(a);
-  else if (mode == 1 && tile_rows == 64) mlp_mfma_kernel<1, 64><<<ntiles, NW * 64, 0, s>>>(a);
-  else if (mode == 1) mlp_mfma_kernel<1, 32><<<ntiles, NW * 64, pad, s>>>(a);
-  else if (mode == 3 && tile_rows == 64) mlp_mfma_kernel<3, 64><<<ntiles, NW * 64, 0, s>>>(a);
-  else if (mode == 3) mlp_mfma_kernel<3, 32><<<ntiles, NW * 64, pad, s>>>(a);
-  else if (mode == 4 && tile_rows == 64) mlp_mfma_kernel<4, 64><<<ntiles, NW * 64, 0, s>>>(a);
-  else if (mode == 4) mlp_mfma_kernel<4, 32><<<ntiles, NW * 64, pad, s>>>(a);
-  else if (mode == 5 && tile_rows == 64) mlp_mfma_kernel<5, 64><<<ntiles, NW * 64, 0, s>>>(a);
-  else if (mode == 5) mlp_mfma_kernel<5, 32><<<ntiles, NW * 64, pad, s>>>(a);
-  else mlp_mfma_kernel<2, 32><<<ntiles, NW * 64, 0, s>>>(a);
+  const bool big = tile_rows == 64;
+  switch (mode) {
+    case 0: big ? launch<0, 64>(a, 0, s) : launch<0, 32>(a, pad, s); break;
+    case 1: big ? launch<1, 64>(a, 0, s) : launch<1, 32>(a, pad, s); break;
+    case 2: launch<2, 32>(a, 0, s); break;
+    case 3: big ? launch<3, 64>(a, 0, s) : launch<3, 32>(a, pad, s); break;
+    case 4: big ? launch<4, 64>(a, 0, s) : launch<4, 32>(a, pad, s); break;
+    default: big ? launch<5, 64>(a, 0, s) : launch<5, 32>(a, pad, s); break;
+  }
   TM_LAUNCH_CHECK();
   return TM_OK;
 }
