@@ -359,9 +359,9 @@ int tm_coulomb_table(const double* consts, double rc_ee, double width, int add_e
  * cell-ordered xqc / elc that tm_charges writes, with the pair functions
  * from tm_coulomb_table's tables (device copy; at most 3072 float4 entries,
  * nint >= 16; inv_h, u0 = its scale) and float32 lane sums added in float64.
- * Same outputs as tm_coulomb (phi, grad, eatom by atom index; flags as its
- * range overflow); every centre's sums are formed in an order fixed by the
- * inputs. */
+ * Same outputs as tm_coulomb (phi, grad, eatom by atom index); flags is not
+ * written (the sweep's candidate list cannot overflow); every centre's sums
+ * are formed in an order fixed by the inputs. */
 int tm_coulomb_tab(int N, const double* box, const int* cell_start, const int* cell_atoms,
                        const int* cell_of, int nx, int ny, int nz, double csx, double csy,
                        double csz, double ox, double oy, double oz, int periodic, double rc_ee,

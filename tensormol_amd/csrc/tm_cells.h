@@ -14,6 +14,8 @@
 // outside it are clamped to edge cells, which only lowers index differences,
 // so the bound stays a lower bound of the true distance.
 #pragma once
+#include <math.h>
+
 #include "tm_common.h"
 
 struct CellGrid {
@@ -27,6 +29,13 @@ struct CellGrid {
   float cs[3];             // cell edges (A)
   float org[3];            // grid origin (A): cell k of an axis spans [org + k cs, org + (k+1) cs)
   int periodic;            // 1: wrap, 0: clamp
+  // stencil of one cutoff (tm_set_stencil, on the host)
+  int k[3];                // cells to either side of a centre's that can hold a neighbour
+  int full[3];             // 1: they wrap the whole periodic axis
+  int ny, nrow;            // stencil rows per z layer, and in all
+  unsigned magic;          // ceil(2^32 / ny): t / ny = (t magic) >> 32 for the row numbers here (ny > 1)
+  double len[3], inv_len[3];   // axis lengths nc cs and their reciprocals
+  float rc2, inv_cs0;      // squared trimmed cutoff, 1 / cs[0]
 };
 
 // Margin (A) added to the cutoff when rows are trimmed with the centre's own
@@ -34,11 +43,31 @@ struct CellGrid {
 // candidates stay a superset of the atoms inside the cutoff.
 constexpr float TM_TRIM_MARGIN = 2e-3f;
 
+// Stencil of cutoff rc over the grid.  Computed once per launch: with the
+// integer divisions and the ceilings of a cutoff in cells it cost each wave
+// about half of its instructions per 64 rows.
+inline void tm_set_stencil(CellGrid& g, float rc) {
+  for (int d = 0; d < 3; ++d) {
+    // a band further out is at least ceil(rc / cs) cells away.  An axis counts
+    // as wrapped two bands before it is, which decides the order of its rows
+    // and is kept, since sums are formed in that order.
+    g.k[d] = (int)ceilf((rc + TM_TRIM_MARGIN) / g.cs[d]);
+    g.full[d] = g.periodic && (2 * ((int)ceilf(rc / g.cs[d]) + 1) + 1 >= g.nc[d]);
+    g.len[d] = (double)g.nc[d] * (double)g.cs[d];
+    g.inv_len[d] = 1.0 / g.len[d];
+  }
+  g.ny = g.full[1] ? g.nc[1] : 2 * g.k[1] + 1;
+  g.nrow = g.ny * (g.full[2] ? g.nc[2] : 2 * g.k[2] + 1);
+  g.magic = (unsigned)((0x100000000ull + (unsigned)g.ny - 1) / (unsigned)g.ny);
+  const float rcm = rc + TM_TRIM_MARGIN;
+  g.rc2 = rcm * rcm;
+  g.inv_cs0 = 1.0f / g.cs[0];
+}
+
 // Distance along one axis from a centre at offset f inside its cell to the band
 // of cells d cells away (0 for its own band).
 __device__ __forceinline__ float tm_band_dist(int d, float f, float cs) {
-  const float v = d > 0 ? (float)d * cs - f : (d < 0 ? f - (float)(d + 1) * cs : 0.f);
-  return fmaxf(v, 0.f);
+  return fmaxf(fmaxf((float)d * cs - f, f - (float)(d + 1) * cs), 0.f);
 }
 
 // Lanes below this one whose bit is set in a wave-wide ballot.
@@ -57,96 +86,114 @@ struct RangeLds {
   int mark[64];   // range starts inside the current chunk, tagged with the chunk's base
 };
 
-// Builds the candidate ranges of atom i for cutoff rc into R (one wavefront,
-// all lanes participate).  Returns the number of candidates; *nrange gets the
-// number of ranges (capped at CAP, overflow flagged).  Every range is
-// non-empty, so the range starts pre[] increase strictly.
-// Rows are trimmed with the centre's position (px, py, pz): along y and z the
-// distance from the centre to a row's band of cells, along x the cells that
-// [x - s, x + s] covers with s^2 = (rc + margin)^2 - dy^2 - dz^2.  On an axis
-// whose stencil wraps the whole periodic box the cell-gap bound (|d| - 1) cs is
-// used instead (two images of a band can be equally near there).
-template <int CAP>
-__device__ inline int tm_build_ranges(int i, const CellGrid& g, float rc, RangeLds<CAP>& R, int lane,
-                                      int* flags, int* nrange, double px, double py, double pz) {
-  const int c = g.cell_of[i];
-  const int cx = c % g.nc[0], cy = (c / g.nc[0]) % g.nc[1], cz = c / (g.nc[0] * g.nc[1]);
-  int k[3];
-  bool full[3];
+// A centre's cell and its offset inside the cell.
+struct CellCentre {
+  int c[3];
   float f[3];
-  {
-    const int ci[3] = {cx, cy, cz};
-    const double p[3] = {px, py, pz};
-    for (int d = 0; d < 3; ++d) {
-      k[d] = (int)ceilf(rc / g.cs[d]) + 1;
-      full[d] = g.periodic && (2 * k[d] + 1 >= g.nc[d]);
-      double u = p[d] - (double)g.org[d];
-      if (g.periodic) {   // wrapped in FP64, so unwrapped coordinates keep their precision
-        const double Ld = (double)g.nc[d] * (double)g.cs[d];
-        u -= Ld * floor(u / Ld);
-      }
-      f[d] = (float)(u - (double)ci[d] * (double)g.cs[d]);   // offset inside the centre's cell
-    }
+};
+__device__ __forceinline__ CellCentre tm_centre(const CellGrid& g, int cell, double px, double py,
+                                                double pz) {
+  CellCentre o;
+  o.c[0] = cell % g.nc[0];
+  o.c[1] = (cell / g.nc[0]) % g.nc[1];
+  o.c[2] = cell / (g.nc[0] * g.nc[1]);
+  const double p[3] = {px, py, pz};
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    double u = p[d] - (double)g.org[d];
+    if (g.periodic && g.nc[d] < 3) u -= g.len[d] * floor(u / g.len[d]);
+    u -= (double)o.c[d] * (double)g.cs[d];
+    // wrapped in FP64, so unwrapped coordinates keep their precision; the
+    // offset lies within a cell of a multiple of the length, so the nearest one is it
+    if (g.periodic && g.nc[d] >= 3) u -= g.len[d] * rint(u * g.inv_len[d]);
+    o.f[d] = (float)u;   // offset inside the centre's cell
   }
-  R.mark[lane] = -1;   // no chunk base is negative; ordered by the wave barriers below
-  const int ny = full[1] ? g.nc[1] : 2 * k[1] + 1;
-  const int nz = full[2] ? g.nc[2] : 2 * k[2] + 1;
-  const float rcm = rc + TM_TRIM_MARGIN;
-  const float rc2 = rcm * rcm;
-  const float inv_cs0 = 1.0f / g.cs[0];
-  int nr = 0;   // wave-uniform
-  for (int base = 0; base < ny * nz; base += 64) {
-    int t = base + lane;
-    int lo0 = 0, hi0 = 0, lo1 = 0, hi1 = 0, cnt = 0;
-    if (t < ny * nz) {
-      int oy = t % ny, oz = t / ny;
-      int dy, dz, y, z;
-      bool ok = true;
-      if (full[1]) { y = oy; dy = y - cy; if (g.periodic) { if (dy > g.nc[1] / 2) dy -= g.nc[1]; if (dy < -g.nc[1] / 2) dy += g.nc[1]; } }
-      else { dy = oy - k[1]; y = cy + dy; if (g.periodic) y = ((y % g.nc[1]) + g.nc[1]) % g.nc[1]; else ok = ok && y >= 0 && y < g.nc[1]; }
-      if (full[2]) { z = oz; dz = z - cz; if (g.periodic) { if (dz > g.nc[2] / 2) dz -= g.nc[2]; if (dz < -g.nc[2] / 2) dz += g.nc[2]; } }
-      else { dz = oz - k[2]; z = cz + dz; if (g.periodic) z = ((z % g.nc[2]) + g.nc[2]) % g.nc[2]; else ok = ok && z >= 0 && z < g.nc[2]; }
-      if (ok) {
-        float my = full[1] ? fmaxf(0.f, (float)(abs(dy) - 1)) * g.cs[1] : tm_band_dist(dy, f[1], g.cs[1]);
-        float mz = full[2] ? fmaxf(0.f, (float)(abs(dz) - 1)) * g.cs[2] : tm_band_dist(dz, f[2], g.cs[2]);
-        float rem = rc2 - my * my - mz * mz;
-        if (rem > 0.f) {
-          const float sx = sqrtf(rem);
-          int xlo = cx + (int)floorf((f[0] - sx) * inv_cs0);
-          int xhi = cx + (int)floorf((f[0] + sx) * inv_cs0);
-          int row = g.nc[0] * (y + g.nc[1] * z);
-          if (g.periodic && xhi - xlo + 1 >= g.nc[0]) {
-            lo0 = g.cell_start[row]; hi0 = g.cell_start[row + g.nc[0]]; cnt = 1;
-          } else if (!g.periodic) {
-            xlo = max(xlo, 0);
-            xhi = min(xhi, g.nc[0] - 1);
-            if (xlo <= xhi) {
-              lo0 = g.cell_start[row + xlo]; hi0 = g.cell_start[row + xhi + 1]; cnt = 1;
-            }
-          } else {
-            if (xlo < 0) {
-              lo0 = g.cell_start[row + xlo + g.nc[0]]; hi0 = g.cell_start[row + g.nc[0]];
-              lo1 = g.cell_start[row]; hi1 = g.cell_start[row + xhi + 1]; cnt = 2;
-            } else if (xhi >= g.nc[0]) {
-              lo0 = g.cell_start[row + xlo]; hi0 = g.cell_start[row + g.nc[0]];
-              lo1 = g.cell_start[row]; hi1 = g.cell_start[row + xhi - g.nc[0] + 1]; cnt = 2;
-            } else {
-              lo0 = g.cell_start[row + xlo]; hi0 = g.cell_start[row + xhi + 1]; cnt = 1;
-            }
-          }
-          // keep only non-empty ranges (both halves of a wrapped row can be empty)
-          if (cnt == 2 && hi1 <= lo1) cnt = 1;
-          if (cnt >= 1 && hi0 <= lo0) { lo0 = lo1; hi0 = hi1; cnt -= 1; }
-        }
-      }
+  return o;
+}
+
+// The candidates of stencil row t of a centre: [lo0, lo0 + n0) and, where the
+// row wraps a periodic edge, [lo1, lo1 + n1) of the cell-ordered arrays.
+// Rows are trimmed with the centre's position: along y and z the distance from
+// the centre to a row's band of cells, along x the cells that [x - s, x + s]
+// covers with s^2 = (rc + margin)^2 - dy^2 - dz^2.  On an axis whose stencil
+// wraps the whole periodic box the cell-gap bound (|d| - 1) cs is used instead
+// (two images of a band can be equally near there).
+__device__ __forceinline__ void tm_row(const CellGrid& g, const CellCentre& o, int t, int& lo0,
+                                       int& n0, int& lo1, int& n1) {
+  lo0 = lo1 = n0 = n1 = 0;
+  if (t >= g.nrow) return;
+  const int tz = g.ny > 1 ? (int)__umulhi((unsigned)t, g.magic) : t, ty = t - tz * g.ny;
+  // band index along one axis, its cell and its distance; false outside an open grid
+  auto band = [&](int d, int off, int& cell, float& dist) {
+    if (g.full[d]) {
+      int dd = off - o.c[d];
+      if (dd > g.nc[d] / 2) dd -= g.nc[d];
+      if (dd < -g.nc[d] / 2) dd += g.nc[d];
+      cell = off;
+      dist = fmaxf(0.f, (float)(abs(dd) - 1)) * g.cs[d];
+      return true;
     }
+    const int dd = off - g.k[d];
+    cell = o.c[d] + dd;
+    dist = tm_band_dist(dd, o.f[d], g.cs[d]);
+    if (!g.periodic) return cell >= 0 && cell < g.nc[d];
+    if (cell < 0) cell += g.nc[d];           // 2 k + 1 < nc here, so one wrap is enough
+    else if (cell >= g.nc[d]) cell -= g.nc[d];
+    return true;
+  };
+  int y, z;
+  float my, mz;
+  const bool oky = band(1, ty, y, my), okz = band(2, tz, z, mz);
+  const float rem = g.rc2 - my * my - mz * mz;
+  if (!oky || !okz || !(rem > 0.f)) return;
+  const float sx = __builtin_amdgcn_sqrtf(rem);   // its last digit is far inside the margin
+  int xlo = o.c[0] + (int)floorf((o.f[0] - sx) * g.inv_cs0);
+  int xhi = o.c[0] + (int)floorf((o.f[0] + sx) * g.inv_cs0);
+  const int* start = g.cell_start + g.nc[0] * (y + g.nc[1] * z);
+  if (g.periodic && xhi - xlo + 1 >= g.nc[0]) {
+    xlo = 0;
+    xhi = g.nc[0] - 1;
+  }
+  if (!g.periodic) {
+    xlo = max(xlo, 0);
+    xhi = min(xhi, g.nc[0] - 1);
+    if (xlo > xhi) return;
+  }
+  // a wrapped row is its upper part, then its lower part
+  const bool wl = xlo < 0, wr = xhi >= g.nc[0];
+  if (wl) xlo += g.nc[0];
+  if (wr) xhi -= g.nc[0];
+  lo0 = start[xlo];
+  n0 = start[wl || wr ? g.nc[0] : xhi + 1] - lo0;
+  if (wl || wr) {
+    lo1 = start[0];
+    n1 = start[xhi + 1] - lo1;
+  }
+}
+
+// Builds the candidate ranges of atom i for the grid's cutoff into R (one
+// wavefront, all lanes participate).  Returns the number of candidates; *nrange
+// gets the number of ranges (capped at CAP, overflow flagged).  Every range is
+// non-empty, so the range starts pre[] increase strictly.
+template <int CAP>
+__device__ inline int tm_build_ranges(int i, const CellGrid& g, RangeLds<CAP>& R, int lane,
+                                      int* flags, int* nrange, double px, double py, double pz) {
+  const CellCentre o = tm_centre(g, g.cell_of[i], px, py, pz);
+  R.mark[lane] = -1;   // no chunk base is negative; ordered by the wave barriers below
+  int nr = 0;   // wave-uniform
+  for (int base = 0; base < g.nrow; base += 64) {
+    int lo0, n0, lo1, n1;
+    tm_row(g, o, base + lane, lo0, n0, lo1, n1);
+    // keep only non-empty ranges (both halves of a wrapped row can be empty)
+    int cnt = (n0 > 0) + (n1 > 0);
+    if (n0 <= 0) { lo0 = lo1; n0 = n1; }
     // compact the non-empty ranges of this round into R (lane order = row order)
     unsigned long long b1 = __ballot(cnt >= 1);
     unsigned long long b2 = __ballot(cnt >= 2);
     int before = tm_lanes_below(b1) + tm_lanes_below(b2);
     int slot = nr + before;
-    if (cnt >= 1 && slot < CAP) { R.lo[slot] = lo0; R.pre[slot + 1] = hi0 - lo0; }
-    if (cnt >= 2 && slot + 1 < CAP) { R.lo[slot + 1] = lo1; R.pre[slot + 2] = hi1 - lo1; }
+    if (cnt >= 1 && slot < CAP) { R.lo[slot] = lo0; R.pre[slot + 1] = n0; }
+    if (cnt >= 2 && slot + 1 < CAP) { R.lo[slot + 1] = lo1; R.pre[slot + 2] = n1; }
     nr += __popcll(b1) + __popcll(b2);
   }
   if (nr > CAP) {
@@ -224,8 +271,8 @@ __device__ __forceinline__ int tm_locate(RangeLds<CAP>& R, int nr, int total, in
 template <int CAP, class F>
 __device__ __forceinline__ void tm_sweep(int i, const int* __restrict__ mol,
                                          const int* __restrict__ mol_start, const CellGrid& g,
-                                         float rc, RangeLds<CAP>& R, int lane, int* flags,
-                                         double px, double py, double pz, F&& f) {
+                                         RangeLds<CAP>& R, int lane, int* flags, double px,
+                                         double py, double pz, F&& f) {
   if (g.cell_atoms == nullptr) {
     const int m = mol[i];
     const int lo = mol_start[m], hi = mol_start[m + 1];
@@ -236,7 +283,7 @@ __device__ __forceinline__ void tm_sweep(int i, const int* __restrict__ mol,
     return;
   }
   int nr = 0;
-  const int total = tm_build_ranges(i, g, rc, R, lane, flags, &nr, px, py, pz);
+  const int total = tm_build_ranges(i, g, R, lane, flags, &nr, px, py, pz);
   // Walk the concatenated ranges 64 candidates at a time.
   int r0 = 0;
   for (int base = 0; base < total; base += 64) {
@@ -252,8 +299,8 @@ __device__ __forceinline__ void tm_sweep(int i, const int* __restrict__ mol,
 template <int CAP, class LD, class F>
 __device__ __forceinline__ void tm_sweep_pf(int i, const int* __restrict__ mol,
                                             const int* __restrict__ mol_start, const CellGrid& g,
-                                            float rc, RangeLds<CAP>& R, int lane, int* flags,
-                                            double px, double py, double pz, LD&& load, F&& f) {
+                                            RangeLds<CAP>& R, int lane, int* flags, double px,
+                                            double py, double pz, LD&& load, F&& f) {
   if (g.cell_atoms == nullptr) {
     const int m = mol[i];
     const int lo = mol_start[m], hi = mol_start[m + 1];
@@ -267,7 +314,7 @@ __device__ __forceinline__ void tm_sweep_pf(int i, const int* __restrict__ mol,
     return;
   }
   int nr = 0;
-  const int total = tm_build_ranges(i, g, rc, R, lane, flags, &nr, px, py, pz);
+  const int total = tm_build_ranges(i, g, R, lane, flags, &nr, px, py, pz);
   int r0 = 0;
   auto locate = [&](int base) { return tm_locate(R, nr, total, lane, base, r0); };
   if (total <= 0) return;
@@ -283,6 +330,87 @@ __device__ __forceinline__ void tm_sweep_pf(int i, const int* __restrict__ mol,
     auto nxt = load(p, base + 64 + lane < total, 1);
     f(pc, vc, 1, cur);
     cur = nxt;
+  }
+}
+
+// Inclusive sum over the lanes of a wave (DPP row shifts and broadcasts).
+__device__ __forceinline__ int tm_wave_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);   // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);   // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);   // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);   // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);   // row_bcast:15
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);   // row_bcast:31
+  return x;
+}
+
+// The candidates of one centre as a list in LDS.  Each round takes 64 stencil
+// rows, one per lane, and writes their candidates behind those left over from
+// the round before (fewer than 64), in row order and at most CAP at a time;
+// whole chunks of 64 are then consumed.  load(p) fetches what f needs for
+// candidate p, one chunk ahead of its use; f(p, valid, payload) runs with all
+// lanes in lockstep.  Same candidates in the same order as tm_sweep: a lane
+// reads its candidate from the list where tm_sweep finds it by a search over
+// the ranges (35 vector instructions and a chain of three LDS round trips per
+// chunk).
+template <int CAP>
+struct ListLds {
+  int p[CAP];
+};
+
+template <int CAP, class LD, class F>
+__device__ __forceinline__ void tm_sweep_list(const CellGrid& g, const CellCentre& o,
+                                              ListLds<CAP>& L, int lane, LD&& load, F&& f) {
+  static_assert(CAP >= 192, "room for a chunk and what is left of the one before");
+  int have = 0;   // candidates in the list, from its start (wave-uniform)
+  for (int base = 0; base < g.nrow; base += 64) {
+    int lo0, n0, lo1, n1;
+    tm_row(g, o, base + lane, lo0, n0, lo1, n1);
+    const int n = n0 + n1, incl = tm_wave_scan(n), pre = incl - n;
+    const int total = __builtin_amdgcn_readlane(incl, 63);
+    for (int w0 = 0; w0 < total;) {   // the round's candidates [w0, w1)
+      const int w1 = min(total, w0 + CAP - have);
+      {
+        int q = max(pre, w0);
+        const int e0 = min(pre + n0, w1), e1 = min(incl, w1), to = have - w0;
+        for (; q < e0; ++q) L.p[to + q] = lo0 + (q - pre);
+        for (q = max(q, pre + n0); q < e1; ++q) L.p[to + q] = lo1 + (q - pre - n0);
+      }
+      have += w1 - w0;
+      w0 = w1;
+      __syncwarp();
+      if (have < 64) continue;
+      // two payloads in turn: one chunk is used while the next one's loads are
+      // in flight
+      int h = 64, p0 = L.p[lane], p1;
+      auto c0 = load(p0), c1 = c0;
+      for (;;) {
+        const bool m1 = h + 64 <= have;   // another whole chunk: its loads go first
+        p1 = m1 ? L.p[h + lane] : p0;
+        c1 = load(p1);
+        f(p0, true, c0);
+        if (!m1) break;
+        h += 64;
+        const bool m0 = h + 64 <= have;
+        p0 = m0 ? L.p[h + lane] : p1;
+        c0 = load(p0);
+        f(p1, true, c1);
+        if (!m0) break;
+        h += 64;
+      }
+      // what is left moves to the front
+      const int left = have - h;
+      const int v = lane < left ? L.p[h + lane] : 0;
+      __syncwarp();
+      if (lane < left) L.p[lane] = v;
+      have = left;
+      __syncwarp();
+    }
+  }
+  if (have > 0) {
+    const bool valid = lane < have;
+    const int p = L.p[valid ? lane : 0];
+    f(p, valid, load(p));
   }
 }
 

@@ -31,7 +31,7 @@ constexpr int C_RANGES = 480;    // 15 A stencil over ~2.3 A cells: <= ~230 rows
 struct CoulArgs {
   float alpha, r_sr, r_lr, zz, yy, shift, ea;     // bohr units
   float lin;                                     // ZZ / R_lr + YY (slope of the shift)
-  float rc, rc2;                                 // EE cutoff (A) and its square
+  float rc2;                                     // EE cutoff (A), squared
   float inv_width;                               // 1 / vdW poly width (bohr after scaling)
   int add_ecc, has_vdw;
   float c6[TM_MAX_ELE], r0[TM_MAX_ELE];
@@ -222,7 +222,7 @@ coulomb_kernel(int N, const float4* __restrict__ xq, const int* __restrict__ ele
       __syncwarp();
     }
   };
-  tm_sweep_pf(i, mol, mol_start, grid, a.rc, rng[w], lane, flags, (double)pi.x, (double)pi.y,
+  tm_sweep_pf(i, mol, mol_start, grid, rng[w], lane, flags, (double)pi.x, (double)pi.y,
               (double)pi.z, load, visit);
   drain(qn);
   double sphi = tm_wave_sum_d(acc.phi);
@@ -742,7 +742,6 @@ int tm_coulomb(int N, const float* xq, const int* elem, const int* mol, const in
   a.zz = (float)consts[3]; a.yy = (float)consts[4]; a.shift = (float)consts[5];
   a.ea = (float)consts[6];
   a.lin = (float)(consts[3] / consts[2] + consts[4]);
-  a.rc = (float)rc_ee;
   a.rc2 = (float)(rc_ee * rc_ee);
   a.inv_width = (float)(1.0 / width);
   a.add_ecc = add_ecc;
@@ -758,6 +757,7 @@ int tm_coulomb(int N, const float* xq, const int* elem, const int* mol, const in
   g.cs[0] = (float)csx; g.cs[1] = (float)csy; g.cs[2] = (float)csz;
   g.org[0] = (float)ox; g.org[1] = (float)oy; g.org[2] = (float)oz;
   g.periodic = periodic;
+  tm_set_stencil(g, (float)rc_ee);
   hipStream_t s = (hipStream_t)stream;
   if (cell_atoms != nullptr && xq != nullptr) {
     cell_gather_kernel<<<tm_div_up(N, 256), 256, 0, s>>>(N, cell_atoms, (const float4*)xq, elem,

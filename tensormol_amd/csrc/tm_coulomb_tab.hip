@@ -17,12 +17,21 @@
 //    where K's second derivative jumps.  A pair costs two table reads and ten
 //    FMAs for both energies and both derivatives instead of the erfc / exp /
 //    reciprocal chains.  The tables are read through the L1 cache (16 KiB for
-//    two elements), so the sweep keeps tm_coulomb's LDS footprint and
-//    occupancy.
+//    two elements); copies in LDS cost more waves than they save (86-91
+//    against 84-86 us on the 12,288-atom box).
+//  - Candidates as a list (tm_sweep_list) instead of a search over ranges.
 //  - Sums.  Each lane sums its pairs in float32 (a few tens per centre) and
 //    the lane sums are added in float64 in a fixed butterfly, instead of a
 //    float64 add per pair.  Queue order is candidate order, so the result
 //    depends only on the inputs.
+//
+// What bounds it: vector instructions, about 3,000 per centre on the box
+// (1,970 candidates, 1,420 pairs), a third of them pair arithmetic, at seven
+// waves per SIMD.  The list in place of the ranges, the stencil's constants
+// from the host, a queue that wraps instead of moving its rest to the front
+// and table reads that return under the next chunk's tests took the box from
+// 94 to 84 us, the open 24,000-atom sphere from 133 to 119 us (charges and the
+// mean potential included).
 #include <math.h>
 
 #include "tm_cells.h"
@@ -31,16 +40,13 @@ namespace {
 
 constexpr double CL_BOHRPERA = 1.889725989;
 constexpr int CT_WAVES = 4;
-// Candidate ranges per wave: CT_RANGES covers every grid of cells >= 2.3 A at
-// a 15 A cutoff (at most 386 ranges); CT_RANGES_WIDE (tm_coulomb's bound) wider
-// stencils.  The smaller LDS footprint fits one more workgroup per CU.
-constexpr int CT_RANGES = 392;
-constexpr int CT_RANGES_WIDE = 480;
-constexpr int CT_QCAP = 128;     // compacted pair queue per wave
+constexpr int CT_RANGES = 480;   // stencils of more ranges are refused (tm_coulomb's bound)
+constexpr int CT_LIST = 448;     // candidate list per wave
+constexpr int CT_QCAP = 128;     // compacted pair queue per wave (a ring)
 constexpr int CL_TABLE_MAX = 3072;   // float4 table entries (48 KiB)
 
 struct ClArgs {
-  float rc, rc2;   // cutoff (A) and its square
+  float rc2;       // cutoff (A), squared
   float inv_h;     // intervals per A
   float u0;        // table coordinate of r = 0 (in [0, 1))
   int nint, nele;
@@ -54,108 +60,126 @@ struct ClAcc {
   float phi, gx, gy, gz, ev;
 };
 
-// Energies and gradient of one pair from the tables; d = (x_j - x_i, q_j),
-// vo = the offset of the (e_i, e_j) vdW table.
-__device__ __forceinline__ void ct_pair(const ClArgs& a, const float4* __restrict__ tab, int vo,
-                                        float qi, float4 d, ClAcc& acc) {
-  // r_A = sqrt(s + 1e-27), the reference's regulariser (RawSymFunc.py:1330)
-  const float s = fmaf(d.x, d.x, fmaf(d.y, d.y, d.z * d.z)) + 1e-27f;
-  const float ir = __builtin_amdgcn_rsqf(s);
-  const float u = fmaf(s * ir, a.inv_h, a.u0);
-  const int k = max(0, min((int)u, a.nint - 1));
-  const float t = u - (float)k;
-  const float4 C = tab[k];
-  const float4 V = tab[vo + k];
-  // value and t-derivative of c0 + c1 t + c2 t^2 + c3 t^3 (Horner)
-  const float pc = fmaf(t, C.w, C.z), qc = fmaf(t, pc, C.y);
-  const float K = fmaf(t, qc, C.x), dK = fmaf(t, fmaf(t, C.w, pc), qc);
-  const float pv = fmaf(t, V.w, V.z), qv = fmaf(t, pv, V.y);
-  const float E = fmaf(t, qv, V.x), dV = fmaf(t, fmaf(t, V.w, pv), qv);
-  acc.phi = fmaf(K, d.w, acc.phi);
-  acc.ev += E;
-  // dE_pair/dr_A = (q_i q_j dK/dt + dV/dt) / h; dE/dx_i = -dE/dr_A (x_j - x_i) / r_A
-  const float sc = -fmaf(qi * d.w, dK, dV) * (a.inv_h * ir);
-  acc.gx = fmaf(sc, d.x, acc.gx);
-  acc.gy = fmaf(sc, d.y, acc.gy);
-  acc.gz = fmaf(sc, d.z, acc.gz);
+// Entry `byte` / 16 of a float4 array, by a byte offset the compiler keeps in
+// 32 bits.
+__device__ __forceinline__ float4 ld16(const float4* __restrict__ p, unsigned byte) {
+  return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(p) + byte);
 }
 
-template <int RCAP>
+// One pair in two halves: begin() forms its table coordinate and issues the
+// table reads, finish() adds its energies and gradient.  d = (x_j - x_i, q_j),
+// vo = the byte offset of the (e_i, e_j) vdW table.
+struct PairTab {
+  float4 d, C, V;
+  float t, ir;
+
+  __device__ __forceinline__ void begin(const ClArgs& a, const float4* __restrict__ tab,
+                                        unsigned vo, float4 dq) {
+    d = dq;
+    // r_A = sqrt(s + 1e-27), the reference's regulariser (RawSymFunc.py:1330)
+    const float s = fmaf(d.x, d.x, fmaf(d.y, d.y, d.z * d.z)) + 1e-27f;
+    ir = __builtin_amdgcn_rsqf(s);
+    const float u = fmaf(s * ir, a.inv_h, a.u0);
+    const int k = max(0, min((int)u, a.nint - 1));
+    t = u - (float)k;
+    C = ld16(tab, 16u * (unsigned)k);
+    V = ld16(tab, vo + 16u * (unsigned)k);
+  }
+
+  __device__ __forceinline__ void finish(const ClArgs& a, float qi, ClAcc& acc) const {
+    // value and t-derivative of c0 + c1 t + c2 t^2 + c3 t^3 (Horner)
+    const float pc = fmaf(t, C.w, C.z), qc = fmaf(t, pc, C.y);
+    const float K = fmaf(t, qc, C.x), dK = fmaf(t, fmaf(t, C.w, pc), qc);
+    const float pv = fmaf(t, V.w, V.z), qv = fmaf(t, pv, V.y);
+    const float E = fmaf(t, qv, V.x), dV = fmaf(t, fmaf(t, V.w, pv), qv);
+    acc.phi = fmaf(K, d.w, acc.phi);
+    acc.ev += E;
+    // dE_pair/dr_A = (q_i q_j dK/dt + dV/dt) / h; dE/dx_i = -dE/dr_A (x_j - x_i) / r_A
+    const float sc = -fmaf(qi * d.w, dK, dV) * (a.inv_h * ir);
+    acc.gx = fmaf(sc, d.x, acc.gx);
+    acc.gy = fmaf(sc, d.y, acc.gy);
+    acc.gz = fmaf(sc, d.z, acc.gz);
+  }
+};
+
+template <bool PERIODIC>
 __global__ void __launch_bounds__(CT_WAVES * 64)
 coulomb_tab_kernel(int N, const float4* __restrict__ xqc, const int* __restrict__ elc,
                    const double* __restrict__ box, CellGrid grid, ClArgs a,
                    const float4* __restrict__ tab, double* __restrict__ phi,
-                   double* __restrict__ grad, double* __restrict__ eatom,
-                   int* __restrict__ flags) {
+                   double* __restrict__ grad, double* __restrict__ eatom) {
   __shared__ float4 qx[CT_WAVES][CT_QCAP];
   __shared__ int qe[CT_WAVES][CT_QCAP];
-  __shared__ RangeLds<RCAP> rng[CT_WAVES];
-  __shared__ int voff[TM_MAX_ELE * TM_MAX_ELE];
-  if (threadIdx.x < TM_MAX_ELE * TM_MAX_ELE) {
-    const int ea = threadIdx.x / TM_MAX_ELE, eb = threadIdx.x % TM_MAX_ELE;
-    const int lo = min(ea, eb), hi = max(ea, eb);
-    voff[threadIdx.x] = (ea < a.nele && eb < a.nele)
-                            ? (1 + lo * a.nele - lo * (lo - 1) / 2 + (hi - lo)) * a.nint
-                            : 0;
-  }
-  __syncthreads();
+  __shared__ ListLds<CT_LIST> list[CT_WAVES];
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int cpi = blockIdx.x * CT_WAVES + w;   // centre, in cell order
   if (cpi >= N) return;   // wave-level synchronisation only below
   const int i = grid.cell_atoms[cpi];
   float Lx = 0.f, Ly = 0.f, Lz = 0.f, iLx = 0.f, iLy = 0.f, iLz = 0.f;
-  if (grid.periodic) {
+  if (PERIODIC) {
     Lx = (float)box[0]; Ly = (float)box[1]; Lz = (float)box[2];
     iLx = 1.0f / Lx; iLy = 1.0f / Ly; iLz = 1.0f / Lz;
   }
   const float4 pi = xqc[cpi];
-  const int* vrow = voff + (elc[cpi] & (TM_MAX_ELE - 1)) * TM_MAX_ELE;
+  // vdW table of the centre with element e: field e of 6 bits (at most 37 tables)
+  const int ei = elc[cpi] & (TM_MAX_ELE - 1);
+  unsigned long long vtab = 0;
+  for (int e = 0; e < a.nele; ++e) {
+    const int lo = min(ei, e), hi = max(ei, e);
+    vtab |= (unsigned long long)(1 + lo * a.nele - lo * (lo - 1) / 2 + (hi - lo)) << (6 * e);
+  }
   ClAcc acc = {0.f, 0.f, 0.f, 0.f, 0.f};
-  int qn = 0;   // wave-uniform queue length
-  auto drain = [&](int n) {   // evaluate the first n (<= 64) queued pairs
-    if (lane < n) ct_pair(a, tab, vrow[qe[w][lane] & (TM_MAX_ELE - 1)], pi.w, qx[w][lane], acc);
+  int qn = 0, qh = 0;   // queue length and head (0 or 64), wave-uniform
+  PairTab pair;         // this lane's pair of the batch whose table reads are in flight
+  bool pending = false;
+  auto begin = [&]() {
+    const float4 d = qx[w][qh + lane];
+    const int e = qe[w][qh + lane];
+    pair.begin(a, tab, ((unsigned)(vtab >> (6 * e)) & 63u) * (16u * (unsigned)a.nint), d);
   };
   struct Cand {
     float4 x;
     int e;
   };
-  // branch-free loads (invalid lanes read entry 0), masked by `valid` below
-  auto load = [&](int p, bool valid, int) {
-    const int q = valid ? p : 0;
-    return Cand{xqc[q], elc[q]};
-  };
-  auto visit = [&](int p, bool valid, int, const Cand& c) {
+  auto load = [&](int p) { return Cand{ld16(xqc, 16u * (unsigned)p), elc[(unsigned)p]}; };
+  auto visit = [&](int p, bool valid, const Cand& c) {
     float4 d;
-    d.x = cl_min_image(c.x.x - pi.x, Lx, iLx);
-    d.y = cl_min_image(c.x.y - pi.y, Ly, iLy);
-    d.z = cl_min_image(c.x.z - pi.z, Lz, iLz);
+    d.x = c.x.x - pi.x;
+    d.y = c.x.y - pi.y;
+    d.z = c.x.z - pi.z;
+    if (PERIODIC) {
+      d.x = cl_min_image(d.x, Lx, iLx);
+      d.y = cl_min_image(d.y, Ly, iLy);
+      d.z = cl_min_image(d.z, Lz, iLz);
+    }
     d.w = c.x.w;
-    const bool ok = valid && p != cpi && d.x * d.x + d.y * d.y + d.z * d.z < a.rc2;
+    // bitwise and: every test is evaluated, no branches
+    const bool ok = valid & (p != cpi) & (d.x * d.x + d.y * d.y + d.z * d.z < a.rc2);
     const unsigned long long bal = __ballot(ok);
-    const int before = tm_lanes_below(bal);
     if (ok) {
-      qx[w][qn + before] = d;
-      qe[w][qn + before] = c.e;
+      const int q = (qh + qn + tm_lanes_below(bal)) & (CT_QCAP - 1);
+      qx[w][q] = d;
+      qe[w][q] = c.e & (TM_MAX_ELE - 1);
     }
     qn += __popcll(bal);
     __syncwarp();
     if (qn >= 64) {
-      drain(64);
-      __syncwarp();
-      // move the remainder (< 64 entries) to the front
-      float4 t4;
-      int te = 0;
-      const bool mv = lane < qn - 64;
-      if (mv) { t4 = qx[w][64 + lane]; te = qe[w][64 + lane]; }
-      __syncwarp();
-      if (mv) { qx[w][lane] = t4; qe[w][lane] = te; }
+      // a batch's table reads return during the next chunk's tests
+      if (pending) pair.finish(a, pi.w, acc);
+      begin();
+      pending = true;
       qn -= 64;
+      qh ^= 64;
       __syncwarp();
     }
   };
-  tm_sweep_pf(i, nullptr, nullptr, grid, a.rc, rng[w], lane, flags, (double)pi.x, (double)pi.y,
-              (double)pi.z, load, visit);
-  drain(qn);
+  tm_sweep_list(grid, tm_centre(grid, grid.cell_of[i], (double)pi.x, (double)pi.y, (double)pi.z),
+                list[w], lane, load, visit);
+  if (pending) pair.finish(a, pi.w, acc);
+  if (lane < qn) {
+    begin();
+    pair.finish(a, pi.w, acc);
+  }
   const double sphi = tm_wave_sum_d((double)acc.phi);
   const double gx = tm_wave_sum_d((double)acc.gx);
   const double gy = tm_wave_sum_d((double)acc.gy);
@@ -293,13 +317,12 @@ int tm_coulomb_tab(int N, const double* box, const int* cell_start, const int* c
   const double cs[3] = {csx, csy, csz};
   const int nc[3] = {nx, ny, nz};
   const int need = tm_range_bound(rc_ee, cs, nc, periodic);
-  TM_REQUIRE(need <= CT_RANGES_WIDE,
+  TM_REQUIRE(need <= CT_RANGES,
              "tm_coulomb_tab: cells of %.2f A are too small for a %.1f A cutoff (a sweep "
              "could need %d candidate ranges, room for %d)", fmin(csx, fmin(csy, csz)), rc_ee,
-             need, CT_RANGES_WIDE);
+             need, CT_RANGES);
   if (N == 0) return TM_OK;
   ClArgs a;
-  a.rc = (float)rc_ee;
   a.rc2 = (float)(rc_ee * rc_ee);
   a.inv_h = (float)inv_h;
   a.u0 = (float)u0;
@@ -312,13 +335,10 @@ int tm_coulomb_tab(int N, const double* box, const int* cell_start, const int* c
   g.cs[0] = (float)csx; g.cs[1] = (float)csy; g.cs[2] = (float)csz;
   g.org[0] = (float)ox; g.org[1] = (float)oy; g.org[2] = (float)oz;
   g.periodic = periodic;
-  const dim3 grid(tm_div_up(N, CT_WAVES)), block(CT_WAVES * 64);
-  if (need <= CT_RANGES)
-    coulomb_tab_kernel<CT_RANGES><<<grid, block, 0, (hipStream_t)stream>>>(
-        N, (const float4*)xqc, elc, box, g, a, (const float4*)table, phi, grad, eatom, flags);
-  else
-    coulomb_tab_kernel<CT_RANGES_WIDE><<<grid, block, 0, (hipStream_t)stream>>>(
-        N, (const float4*)xqc, elc, box, g, a, (const float4*)table, phi, grad, eatom, flags);
+  tm_set_stencil(g, (float)rc_ee);
+  const auto k = periodic ? coulomb_tab_kernel<true> : coulomb_tab_kernel<false>;
+  k<<<tm_div_up(N, CT_WAVES), CT_WAVES * 64, 0, (hipStream_t)stream>>>(
+      N, (const float4*)xqc, elc, box, g, a, (const float4*)table, phi, grad, eatom);
   TM_LAUNCH_CHECK();
   return TM_OK;
 }

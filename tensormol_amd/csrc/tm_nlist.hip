@@ -47,7 +47,7 @@ __global__ void __launch_bounds__(NL_WAVES * 64)
 nl_rows_kernel(int N, const double* __restrict__ pos, const int* __restrict__ elem,
                const int* __restrict__ mol, const int* __restrict__ mol_start,
                const double* __restrict__ box, CellGrid grid, int nele,
-               double s_r, double s_a, float rc, int ldr, int lda,
+               double s_r, double s_a, int ldr, int lda,
                int* __restrict__ nbr, int* __restrict__ ncnt, int* __restrict__ rseg,
                int* __restrict__ ang, int* __restrict__ acnt, int* __restrict__ aseg,
                int* __restrict__ flags) {
@@ -88,7 +88,7 @@ nl_rows_kernel(int N, const double* __restrict__ pos, const int* __restrict__ el
       }
       count += __popcll(bal);
     };
-    tm_sweep(i, mol, mol_start, grid, rc, rng[w], lane, flags, xi, yi, zi, visit);
+    tm_sweep(i, mol, mol_start, grid, rng[w], lane, flags, xi, yi, zi, visit);
     if (count > NL_LDS_CAP || count > ldr) {
       if (lane == 0) atomicOr(&flags[TM_FLAG_NB_OVERFLOW], 1);
       count = min(count, min(NL_LDS_CAP, ldr));
@@ -404,7 +404,7 @@ template <bool FILL>
 __global__ void __launch_bounds__(NL_WAVES * 64)
 pairs_kernel(int N, const double* __restrict__ pos, const int* __restrict__ mol,
              const int* __restrict__ mol_start, const int* __restrict__ nreal,
-             const double* __restrict__ box, CellGrid grid, float rc, double s_c, int half,
+             const double* __restrict__ box, CellGrid grid, double s_c, int half,
              int* __restrict__ count, const long* __restrict__ start, int* __restrict__ out,
              int* __restrict__ flags) {
   __shared__ RangeLds<1024> rng[NL_WAVES];
@@ -438,7 +438,7 @@ pairs_kernel(int N, const double* __restrict__ pos, const int* __restrict__ mol,
     if (FILL && ok) out[o + cnt + tm_lanes_below(bal)] = j;
     cnt += __popcll(bal);
   };
-  tm_sweep(i, mol, mol_start, grid, rc, rng[w], lane, flags, xi, yi, zi, visit);
+  tm_sweep(i, mol, mol_start, grid, rng[w], lane, flags, xi, yi, zi, visit);
   if (!FILL && lane == 0) count[i] = cnt;
 }
 
@@ -449,7 +449,7 @@ extern "C" {
 static CellGrid make_grid(const int* cell_start, const int* cell_atoms, const int* cell_of,
                           const int* cell_pos, const double* posc, const int* molc, int nx, int ny,
                           int nz, double csx, double csy, double csz, double ox, double oy,
-                          double oz, int periodic) {
+                          double oz, int periodic, double rc) {
   CellGrid g;
   g.cell_start = cell_start; g.cell_atoms = cell_atoms; g.cell_of = cell_of;
   g.cell_pos = cell_pos; g.posc = posc; g.molc = molc;
@@ -457,6 +457,7 @@ static CellGrid make_grid(const int* cell_start, const int* cell_atoms, const in
   g.cs[0] = (float)csx; g.cs[1] = (float)csy; g.cs[2] = (float)csz;
   g.org[0] = (float)ox; g.org[1] = (float)oy; g.org[2] = (float)oz;
   g.periodic = periodic;
+  tm_set_stencil(g, (float)rc);
   return g;
 }
 
@@ -520,9 +521,9 @@ int tm_nl_build(int N, const double* pos, const int* elem, const int* mol, const
   if (N == 0) return TM_OK;
   hipStream_t s = (hipStream_t)stream;
   CellGrid g = make_grid(cell_start, cell_atoms, cell_of, cell_pos, posc, molc, nx, ny, nz, csx, csy,
-                         csz, ox, oy, oz, periodic);
+                         csz, ox, oy, oz, periodic, rc);
   nl_rows_kernel<<<tm_div_up(N, NL_WAVES), NL_WAVES * 64, 0, s>>>(
-      N, pos, elem, mol, mol_start, box, g, nele, s_r, s_a, (float)rc, ldr, lda, nbr, ncnt, rseg,
+      N, pos, elem, mol, mol_start, box, g, nele, s_r, s_a, ldr, lda, nbr, ncnt, rseg,
       ang, acnt, aseg, flags);
   TM_LAUNCH_CHECK();
   if (rev != nullptr) {   // else tm_sym_forward fills rev
@@ -561,13 +562,13 @@ int tm_pairs(int N, const double* pos, const int* mol, const int* mol_start, con
   if (N == 0) return TM_OK;
   hipStream_t s = (hipStream_t)stream;
   CellGrid g = make_grid(cell_start, cell_atoms, cell_of, cell_pos, posc, molc, nx, ny, nz, csx, csy,
-                         csz, ox, oy, oz, periodic);
+                         csz, ox, oy, oz, periodic, rc);
   if (start == nullptr)
     pairs_kernel<false><<<tm_div_up(N, NL_WAVES), NL_WAVES * 64, 0, s>>>(
-        N, pos, mol, mol_start, nreal, box, g, (float)rc, s_c, half, count, nullptr, nullptr, flags);
+        N, pos, mol, mol_start, nreal, box, g, s_c, half, count, nullptr, nullptr, flags);
   else
     pairs_kernel<true><<<tm_div_up(N, NL_WAVES), NL_WAVES * 64, 0, s>>>(
-        N, pos, mol, mol_start, nreal, box, g, (float)rc, s_c, half, count, start, out, flags);
+        N, pos, mol, mol_start, nreal, box, g, s_c, half, count, start, out, flags);
   TM_LAUNCH_CHECK();
   return TM_OK;
 }
