@@ -84,29 +84,20 @@ __device__ __forceinline__ void powz_pair(float b, const SymArgs& a, float& Az, 
   dAz = b > 0.f ? a.zeta * Az * __builtin_amdgcn_rcpf(b) : 0.f;
 }
 
-template <int RC>
-struct RowLds {
-  static constexpr bool has_fc = true, has_fa = true, has_el = true;
-  float4 d[SYM_WAVES][RC];      // (x_j - x_i, r)
-  float fc[SYM_WAVES][RC];      // radial cutoff function
-  float fa[SYM_WAVES][RC];      // angular cutoff function
-  int el[SYM_WAVES][RC];
-};
-// The forward's row: the angular cutoff is formed once per triple instead,
-// which keeps its LDS small enough for 7 waves per SIMD.
+// A centre's row in LDS: x_j - x_i and r, and the radial cutoff where many
+// lanes read it.  What one lane needs once (elements, the angular cutoff) is
+// formed where it is used, which keeps the kernels at six to seven waves per
+// SIMD.
 template <int RC>
 struct RowLdsFwd {
-  static constexpr bool has_fc = true, has_fa = false, has_el = false;
+  static constexpr bool has_fc = true;
   float4 d[SYM_WAVES][RC];
   float fc[SYM_WAVES][RC];
 };
-// The adjoint's row: its radial pass forms fc and reads the element itself
-// (lane = neighbour), which keeps its LDS small enough for 6 waves per SIMD.
 template <int RC>
 struct RowLdsAdj {
-  static constexpr bool has_fc = false, has_fa = true, has_el = false;
+  static constexpr bool has_fc = false;
   float4 d[SYM_WAVES][RC];
-  float fa[SYM_WAVES][RC];
 };
 
 __device__ __forceinline__ float cutoff_fc(float k, float r) { return 0.5f * (__cosf(k * r) + 1.0f); }
@@ -125,8 +116,8 @@ __device__ __forceinline__ float cutoff_dfc(float k, float r) { return -0.5f * k
 template <class LDS>
 __device__ __forceinline__ void load_row(int i, int w, int lane, const double* __restrict__ pos,
                                          const double* __restrict__ box, const int* __restrict__ mol,
-                                         const int* __restrict__ elem, const int* __restrict__ nbr,
-                                         int n, int ldr, const SymArgs& a, LDS& L) {
+                                         const int* __restrict__ nbr, int n, int ldr,
+                                         const SymArgs& a, LDS& L) {
   // minimum image with the reciprocal edge (iL = 0 for open boundaries): it
   // differs from d - L rint(d / L) only at |d| = L/2, far beyond the cutoff
   double Lx = 0, Ly = 0, Lz = 0, iLx = 0, iLy = 0, iLz = 0;
@@ -144,9 +135,7 @@ __device__ __forceinline__ void load_row(int i, int w, int lane, const double* _
     float dz = (float)(ez - Lz * rint(ez * iLz));
     float r = sqrtf(dx * dx + dy * dy + dz * dz + 1e-27f);
     L.d[w][q] = make_float4(dx, dy, dz, r);
-    if constexpr (LDS::has_fa) L.fa[w][q] = cutoff_fc(a.ka, r);
     if constexpr (LDS::has_fc) L.fc[w][q] = cutoff_fc(a.kr, r);
-    if constexpr (LDS::has_el) L.el[w][q] = elem[j];
   }
 }
 
@@ -203,7 +192,7 @@ sym_fwd_kernel(int N, const double* __restrict__ pos, const double* __restrict__
     segs[w][0][lane] = min(rseg[(long)i * (a.nele + 1) + lane], n);
     segs[w][1][lane] = aseg[(long)i * (a.nele + 1) + lane];
   }
-  load_row(i, w, lane, pos, box, mol, elem, nbr, n, ldr, a, L);
+  load_row(i, w, lane, pos, box, mol, nbr, n, ldr, a, L);
   __syncwarp();
   float* Gi = G + (long)i * ldg;
   // ---------------- radial: lane = (half h, shell s)
@@ -331,79 +320,140 @@ sym_fwd_kernel(int N, const double* __restrict__ pos, const double* __restrict__
   }
 }
 
-// dE/dG (two contributions combined: gE + u_i * gQ) -> w slots
+// dE/dG (two contributions combined: gE + u_i * gQ) -> w slots.
+//
+// Angular part: triples (a, b) of sub-list members a < b, numbered t =
+// b (b - 1) / 2 + a.  A window of ADJ_TC triples is evaluated, lane = triple,
+// its contributions to a and to b left in LDS; then lane = member adds its own.
+// Numbered like this, a member's triples come in ascending order of the
+// partner, so "add over partners" is a plain loop whose LDS reads do not
+// depend on each other.  (Numbered by element pair, as in the forward, a
+// member had to search its triples block by block: 7,000 of a wave's 26,000
+// cycles on the water box, 15,000 of 43,000 on the C/H/N/O sphere.)
+//
+// What bounds it now: the instructions of the triples (some 450 per 64) and of
+// the 32 radial shells per neighbour, and the dE/dG rows (1 to 6 KB per
+// centre), which are on their way while the neighbour row is staged.
+// Adjoint and force gather: 12,288-atom box 54 -> 38 us, 24,000-atom sphere
+// 175 -> 81 us, 2,139 chain atoms 41 -> 21 us.
+constexpr int ADJ_TC = 128;   // triples per window, two per lane
+
 template <int ZI, int RC>
-__global__ void __launch_bounds__(SYM_WAVES * 64) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ void __launch_bounds__(SYM_WAVES * 64) __attribute__((amdgpu_waves_per_eu(RC == 128 ? 6 : 4)))
 sym_adj_kernel(int N, const double* __restrict__ pos, const double* __restrict__ box,
                const int* __restrict__ mol, const int* __restrict__ elem,
                const int* __restrict__ nbr, const int* __restrict__ ncnt,
-               const int* __restrict__ rseg, const int* __restrict__ ang,
-               const int* __restrict__ acnt, const int* __restrict__ aseg, int ldr, int lda,
+               const int* __restrict__ ang, const int* __restrict__ acnt, int ldr, int lda,
                SymArgs a, const float* __restrict__ gE, const float* __restrict__ gQ,
                const float* __restrict__ u, const double* __restrict__ phi,
-               const double* __restrict__ phimean, int ldg, float4* __restrict__ wslot) {
+               const double* __restrict__ phimean, int ldg, int vec4,
+               float4* __restrict__ wslot) {
+  constexpr int NQ = RC / 64;   // neighbours (and members) per lane
+  constexpr int TU = ZI > 0 ? NT : 1;
   __shared__ RowLdsAdj<RC> L;
-  extern __shared__ float gdyn[];   // SYM_WAVES * D floats: dE/dG of each wave's centre
-  float* gw = gdyn + (threadIdx.x >> 6) * a.D;
-  __shared__ float wacc[3][SYM_WAVES][RC];    // w per neighbour slot (x, y, z planes)
-  __shared__ float cab[2][3][SYM_WAVES][64];       // per triple: contributions to j (0) and k (1)
-  __shared__ int segs[SYM_WAVES][2][TM_MAX_ELE + 1];
+  // window: contributions of each triple to b (planes 0-2) and to a (3-5), x y z;
+  // afterwards the members' sums by neighbour slot
+  __shared__ float cw[SYM_WAVES][6 * ADJ_TC];
+  static_assert(3 * RC <= 6 * ADJ_TC, "the members' sums reuse the window");
+  __shared__ int mem[SYM_WAVES][RC];   // member: position in the row | element << 16
+  extern __shared__ float4 gdyn[];     // dE/dG of each wave's centre, D rounded up to 4 floats
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int i = blockIdx.x * SYM_WAVES + w;
-  if (i >= N) return;
-  const int n = min(ncnt[i], RC);
-  if (lane <= a.nele) {
-    segs[w][0][lane] = min(rseg[(long)i * (a.nele + 1) + lane], n);
-    segs[w][1][lane] = aseg[(long)i * (a.nele + 1) + lane];
-  }
+  if (i >= N) return;   // only wave-level synchronisation below
+  // the radial part as it is, the angular part from a 16-byte boundary
+  const int off = a.nele * a.nr, offa = (off + 3) & ~3, D4 = (a.D + offa - off + 3) >> 2;
+  float* gw = reinterpret_cast<float*>(gdyn + w * D4);
+  const int n = min(ncnt[i], RC), m = min(min(acnt[i], lda), RC);
   // charge upstream u_i = phi_i - mean_m(phi) (as tm_charge_upstream) unless given
   const float ui = gQ == nullptr ? 0.f
                    : (u != nullptr ? u[i] : (float)(phi[i] - phimean[mol[i]]));
-  for (int f = lane; f < a.D; f += 64) {
-    float v = gE[(long)i * ldg + f];
-    if (gQ != nullptr) v += ui * gQ[(long)i * ldg + f];
-    gw[f] = v;
+  const float* gEi = gE + (long)i * ldg;
+  const float* gQi = gQ + (long)i * ldg;
+  if (vec4) {   // D <= 1024: at most four float4 per lane, all on their way before the row
+    float4 v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int f = 4 * (lane + 64 * k);
+      if (f < a.D) {
+        v[k] = *reinterpret_cast<const float4*>(gEi + f);
+        if (gQ != nullptr) {
+          const float4 z = *reinterpret_cast<const float4*>(gQi + f);
+          v[k].x += ui * z.x; v[k].y += ui * z.y; v[k].z += ui * z.z; v[k].w += ui * z.w;
+        }
+      }
+    }
+    load_row(i, w, lane, pos, box, mol, nbr, n, ldr, a, L);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int f = 4 * (lane + 64 * k);
+      if (f < a.D) *reinterpret_cast<float4*>(gw + f) = v[k];   // off % 4 == 0 here
+    }
+  } else {
+    for (int f = lane; f < a.D; f += 64) {
+      float v = gEi[f];
+      if (gQ != nullptr) v += ui * gQi[f];
+      gw[f < off ? f : f + offa - off] = v;
+    }
+    load_row(i, w, lane, pos, box, mol, nbr, n, ldr, a, L);
   }
-  load_row(i, w, lane, pos, box, mol, elem, nbr, n, ldr, a, L);
+  for (int x = lane; x < m; x += 64) {
+    const int q = ang[(long)i * lda + x];
+    mem[w][x] = q | (elem[nbr[(long)i * ldr + q]] << 16);
+  }
   __syncwarp();
   // ---------------- radial: lane = neighbour
   const float kr = a.kr;
-  for (int q = lane; q < n; q += 64) {
-    float4 d = L.d[w][q];
-    float r = d.w;
-    int e = elem[nbr[(long)i * ldr + q]];
-    float fc = cutoff_fc(kr, r);
-    float dfc = cutoff_dfc(kr, r);
-    float dEdr = 0.f;
-    for (int s = 0; s < a.nr; ++s) {
-      float x = r - a.rs_r[s];
-      float ex = __expf(-a.eta * x * x);
-      dEdr += gw[e * a.nr + s] * ex * (dfc - 2.0f * a.eta * x * fc);
+  float wx[NQ], wy[NQ], wz[NQ];
+#pragma unroll
+  for (int k = 0; k < NQ; ++k) {
+    const int q = lane + 64 * k;
+    wx[k] = wy[k] = wz[k] = 0.f;
+    if (q < n) {
+      float4 d = L.d[w][q];
+      float r = d.w;
+      int e = elem[nbr[(long)i * ldr + q]];
+      float fc = cutoff_fc(kr, r);
+      float dfc = cutoff_dfc(kr, r);
+      float dEdr = 0.f;
+      const float* gr = gw + e * a.nr;
+      auto shell = [&](float gs, int s) {
+        float x = r - a.rs_r[s];
+        float ex = __expf(-a.eta * x * x);
+        dEdr += gs * ex * (dfc - 2.0f * a.eta * x * fc);
+      };
+      if ((a.nr & 3) == 0) {
+        for (int s = 0; s < a.nr; s += 4) {
+          const float4 g4 = *reinterpret_cast<const float4*>(gr + s);
+          shell(g4.x, s); shell(g4.y, s + 1); shell(g4.z, s + 2); shell(g4.w, s + 3);
+        }
+      } else {
+        for (int s = 0; s < a.nr; ++s) shell(gr[s], s);
+      }
+      float sc = dEdr * __builtin_amdgcn_rcpf(r);
+      wx[k] = sc * d.x;
+      wy[k] = sc * d.y;
+      wz[k] = sc * d.z;
     }
-    float sc = dEdr * __builtin_amdgcn_rcpf(r);
-    wacc[0][w][q] = sc * d.x;
-    wacc[1][w][q] = sc * d.y;
-    wacc[2][w][q] = sc * d.z;
   }
-  __syncwarp();
-  // ---------------- angular: lane = triple, contributions staged per chunk
-  const int m = min(acnt[i], lda);
-  const int* arow = ang + (long)i * lda;
+  // ---------------- angular
   const int ntrip = m * (m - 1) / 2;
-  const int off = a.nele * a.nr;
-  float4 wang = make_float4(0.f, 0.f, 0.f, 0.f);   // lane = sub-list member
-  const int* sg = segs[w][1];
-  int eq = -1, lq = 0;   // element and in-element index of member `lane`
-  if (lane < m)
-    for (int e = 0; e < a.nele; ++e)
-      if (lane >= sg[e] && lane < sg[e + 1]) { eq = e; lq = lane - sg[e]; }
-  for (int base = 0; base < ntrip; base += 64) {
-    int t = base + lane;
-    if (t < ntrip) {
-      int ja, kb, p;
-      decode_triple(t, segs[w][1], a.nele, ja, kb, p);
-      int qj = arow[ja], qk = arow[kb];
-      float4 dj = L.d[w][qj], dk = L.d[w][qk];
+  float ax[NQ], ay[NQ], az[NQ];   // sums of members lane, lane + 64, ...
+#pragma unroll
+  for (int k = 0; k < NQ; ++k) ax[k] = ay[k] = az[k] = 0.f;
+  float* cwv = cw[w];
+  for (int T0 = 0; T0 < ntrip; T0 += ADJ_TC) {
+    const int len = min(ADJ_TC, ntrip - T0);
+    for (int uu = lane; uu < len; uu += 64) {
+      const int t = T0 + uu;
+      // b: the largest with b (b - 1) / 2 <= t
+      int kb = (int)((1.0f + __builtin_amdgcn_sqrtf(1.0f + 8.0f * (float)t)) * 0.5f);
+      if (kb * (kb - 1) / 2 > t) --kb;
+      if ((kb + 1) * kb / 2 <= t) ++kb;
+      const int ja = t - kb * (kb - 1) / 2;
+      const int mj = mem[w][ja], mk = mem[w][kb];
+      const int ej = mj >> 16, ek = mk >> 16;   // ej <= ek: the sub-list is sorted
+      const int p = ej * a.nele - ej * (ej - 1) / 2 + (ek - ej);
+      float4 dj = L.d[w][mj & 0xffff], dk = L.d[w][mk & 0xffff];
       float rj = dj.w, rk = dk.w;
       const float irj = __builtin_amdgcn_rcpf(rj), irk = __builtin_amdgcn_rcpf(rk);
       float inv = irj * irk;
@@ -412,7 +462,7 @@ sym_adj_kernel(int N, const double* __restrict__ pos, const double* __restrict__
       float sn = sin_between(dj, dk, inv);
       float cos_over_sin = sn > 1e-6f ? c * __builtin_amdgcn_rcpf(sn) : 0.f;
       float ravg = 0.5f * (rj + rk);
-      float fj = L.fa[w][qj], fk = L.fa[w][qk];
+      float fj = cutoff_fc(a.ka, rj), fk = cutoff_fc(a.ka, rk);
       float dfj = cutoff_dfc(a.ka, rj), dfk = cutoff_dfc(a.ka, rk);
       float F = fj * fk;
       float R[NA], Rp[NA];
@@ -422,16 +472,17 @@ sym_adj_kernel(int N, const double* __restrict__ pos, const double* __restrict__
         R[s] = __expf(-a.eta * x * x);
         Rp[s] = -2.0f * a.eta * x * R[s];
       }
-      const float* gp = gw + off + p * 64;
+      const float4* gp = reinterpret_cast<const float4*>(gw + offa + p * 64);
       float dEdc = 0.f, dEdrav = 0.f, dEdF = 0.f;
-#pragma unroll
+#pragma unroll TU
       for (int tt = 0; tt < NT; ++tt) {
+        const float4 g0 = gp[2 * tt], g1 = gp[2 * tt + 1];
+        const float gv[NA] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
         float S = 0.f, Sp = 0.f;
 #pragma unroll
         for (int s = 0; s < NA; ++s) {
-          float gv = gp[tt * NA + s];
-          S += gv * R[s];
-          Sp += gv * Rp[s];
+          S += gv[s] * R[s];
+          Sp += gv[s] * Rp[s];
         }
         float v = c * a.cos_t[tt] + sn * a.sin_t[tt];
         float b = 1.0f + v;
@@ -441,6 +492,7 @@ sym_adj_kernel(int N, const double* __restrict__ pos, const double* __restrict__
         dEdc += dAz * dv * S;
         dEdrav += Az * Sp;
         dEdF += Az * S;
+        __builtin_amdgcn_sched_barrier(0);   // one theta point's row in registers at a time
       }
       // the common factor 2^(1 - zeta) of every term, applied once
       dEdc *= a.two_1mz * F;
@@ -450,68 +502,70 @@ sym_adj_kernel(int N, const double* __restrict__ pos, const double* __restrict__
       float cj = (dEdrav * 0.5f + dEdF * dfj * fk - dEdc * c * irj) * irj;
       float ck = (dEdrav * 0.5f + dEdF * fj * dfk - dEdc * c * irk) * irk;
       float x = dEdc * inv;
-      cab[0][0][w][lane] = cj * dj.x + x * dk.x;
-      cab[0][1][w][lane] = cj * dj.y + x * dk.y;
-      cab[0][2][w][lane] = cj * dj.z + x * dk.z;
-      cab[1][0][w][lane] = ck * dk.x + x * dj.x;
-      cab[1][1][w][lane] = ck * dk.y + x * dj.y;
-      cab[1][2][w][lane] = ck * dk.z + x * dj.z;
+      cwv[uu] = ck * dk.x + x * dj.x;
+      cwv[ADJ_TC + uu] = ck * dk.y + x * dj.y;
+      cwv[2 * ADJ_TC + uu] = ck * dk.z + x * dj.z;
+      cwv[3 * ADJ_TC + uu] = cj * dj.x + x * dk.x;
+      cwv[4 * ADJ_TC + uu] = cj * dj.y + x * dk.y;
+      cwv[5 * ADJ_TC + uu] = cj * dj.z + x * dk.z;
     }
     __syncwarp();
-    // Member `lane` gathers its contributions from the triples [base, base + cnt)
-    // in ascending triple order, walking only its own partners: in a same-element
-    // block it is k of (j < k) at t = k(k-1)/2 + j, then j at t = k'(k'-1)/2 + j
-    // for k' > j; in a cross block (ea < eb) t = kb_local * la + ja_local.
-    if (eq >= 0) {
-      const int cnt = min(64, ntrip - base);
-      // contribution of triple slot u to its j (h = 0) or k (h = 1) member
-      auto add = [&](int h, int u) {
-        wang.x += cab[h][0][w][u]; wang.y += cab[h][1][w][u]; wang.z += cab[h][2][w][u];
-      };
-      int bo = 0;   // first triple of the block
-      for (int ea = 0; ea < a.nele; ++ea) {
-        const int la = sg[ea + 1] - sg[ea];
-        for (int eb = ea; eb < a.nele; ++eb) {
-          const int lb = sg[eb + 1] - sg[eb];
-          const int nb = ea == eb ? la * (la - 1) / 2 : la * lb;
-          const int lo = base - bo, hi = lo + cnt;   // chunk window, block-local
-          if (hi > 0 && lo < nb) {
-            if (ea == eb) {
-              if (eq == ea) {
-                const int t0 = lq * (lq - 1) / 2;
-                for (int r = max(0, lo - t0); r < min(lq, hi - t0); ++r) add(1, t0 + r - lo);
-                for (int r = lq + 1; r < la; ++r) {
-                  const int t = r * (r - 1) / 2 + lq;
-                  if (t >= hi) break;
-                  if (t >= lo) add(0, t - lo);
-                }
-              }
-            } else if (eq == ea) {
-              for (int kl = 0; kl < lb; ++kl) {
-                const int t = kl * la + lq;
-                if (t >= hi) break;
-                if (t >= lo) add(0, t - lo);
-              }
-            } else if (eq == eb) {
-              const int t0 = lq * la;
-              for (int r = max(0, lo - t0); r < min(la, hi - t0); ++r) add(1, t0 + r - lo);
-            }
-          }
-          bo += nb;
-        }
+    // members add their triples of the window in ascending order of the partner
+    // y: below the member its number is x (x - 1) / 2 + y, above it y (y - 1) / 2 + x
+    const int last = T0 + len - 1;
+    int bh = (int)((1.0f + __builtin_amdgcn_sqrtf(1.0f + 8.0f * (float)last)) * 0.5f);
+    if (bh * (bh - 1) / 2 > last) --bh;
+    if ((bh + 1) * bh / 2 <= last) ++bh;   // the window's last b
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) {
+      const int x = lane + 64 * k;
+      if (64 * k > bh) break;
+      const int tx = x * (x - 1) / 2 - T0;
+      int ty = -T0;   // y (y - 1) / 2 - T0
+#pragma unroll 4
+      for (int y = 0; y <= bh; ++y) {
+        const bool below = y < x;
+        const int t = below ? tx + y : ty + x;
+        const bool ok = (unsigned)t < (unsigned)len && y != x && x <= bh;
+        const float* c = cwv + (ok ? t : 0) + (below ? 0 : 3 * ADJ_TC);
+        const float cx = c[0], cy = c[ADJ_TC], cz = c[2 * ADJ_TC];
+        ax[k] += ok ? cx : 0.f;
+        ay[k] += ok ? cy : 0.f;
+        az[k] += ok ? cz : 0.f;
+        ty += y;
       }
     }
     __syncwarp();
   }
-  if (lane < m) {
-    int q = arow[lane];
-    wacc[0][w][q] += wang.x;
-    wacc[1][w][q] += wang.y;
-    wacc[2][w][q] += wang.z;
+  if (m > 1) {   // the members' sums, by neighbour slot
+    for (int q = lane; q < n; q += 64) cwv[q] = cwv[RC + q] = cwv[2 * RC + q] = 0.f;
+    __syncwarp();
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) {
+      const int x = lane + 64 * k;
+      if (x < m) {
+        const int q = mem[w][x] & 0xffff;
+        cwv[q] = ax[k];
+        cwv[RC + q] = ay[k];
+        cwv[2 * RC + q] = az[k];
+      }
+    }
+    __syncwarp();
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) {
+      const int q = lane + 64 * k;
+      if (q < n) {
+        wx[k] += cwv[q];
+        wy[k] += cwv[RC + q];
+        wz[k] += cwv[2 * RC + q];
+      }
+    }
   }
-  __syncwarp();
-  for (int q = lane; q < n; q += 64)
-    wslot[(long)i * ldr + q] = make_float4(wacc[0][w][q], wacc[1][w][q], wacc[2][w][q], 0.f);
+#pragma unroll
+  for (int k = 0; k < NQ; ++k) {
+    const int q = lane + 64 * k;
+    if (q < n) wslot[(long)i * ldr + q] = make_float4(wx[k], wy[k], wz[k], 0.f);
+  }
 }
 
 // Velocity Verlet state advanced by the force gather (VV = true): the kick of
@@ -617,7 +671,7 @@ sym_jvp_kernel(int N, const double* __restrict__ pos, const double* __restrict__
     segs[w][0][lane] = min(rseg[(long)i * (a.nele + 1) + lane], n);
     segs[w][1][lane] = aseg[(long)i * (a.nele + 1) + lane];
   }
-  load_row(i, w, lane, pos, box, mol, elem, nbr, n, ldr, a, L);
+  load_row(i, w, lane, pos, box, mol, nbr, n, ldr, a, L);
   const float kr = a.kr, ka = a.ka;
   {
     const double uxi = du[3 * i], uyi = du[3 * i + 1], uzi = du[3 * i + 2];
@@ -827,9 +881,13 @@ int tm_sym_adjoint(int N, const double* pos, const double* box, const int* mol, 
   hipStream_t s = (hipStream_t)stream;
   auto k = ldr <= 128 ? (a.zeta_int == 8 ? sym_adj_kernel<8, 128> : sym_adj_kernel<0, 128>)
                       : (a.zeta_int == 8 ? sym_adj_kernel<8, 256> : sym_adj_kernel<0, 256>);
-  k<<<tm_div_up(N, SYM_WAVES), SYM_WAVES * 64, sizeof(float) * SYM_WAVES * a.D, s>>>(
-      N, pos, box, mol, elem, nbr, ncnt, rseg, ang, acnt, aseg, ldr, lda, a, gE, gQ, u, phi,
-      phimean, ldg, (float4*)wslot);
+  auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
+  const int off = nele * nr;
+  const int vec4 = off % 4 == 0 && a.D % 4 == 0 && ldg % 4 == 0 && aligned(gE) && aligned(gQ);
+  const int D4 = (a.D + ((off + 3) & ~3) - off + 3) / 4;
+  k<<<tm_div_up(N, SYM_WAVES), SYM_WAVES * 64, sizeof(float4) * SYM_WAVES * D4, s>>>(
+      N, pos, box, mol, elem, nbr, ncnt, ang, acnt, ldr, lda, a, gE, gQ, u, phi, phimean, ldg,
+      vec4, (float4*)wslot);
   TM_LAUNCH_CHECK();
   return TM_OK;
 }
