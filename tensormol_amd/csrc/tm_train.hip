@@ -35,6 +35,11 @@ constexpr int GT = 128;       // C tile edge per workgroup (four waves of 64 x 6
 constexpr int GK = 64;        // K per staged step (two v_mfma_f32_16x16x32_bf16 deep)
 constexpr int LROW = GK + 8;  // LDS row of a staged operand, in bf16 (144 B, padded)
 constexpr int MAXG = 16;      // GEMMs per grouped launch
+constexpr int MINSTEPS = 16;  // K steps below which a split is not made shorter
+// 128 x 128 tiles below which 64 x 128 ones are used (four per CU).  Softplus
+// epilogue, N = K = 512: 2,560 rows (80 tiles) 18.9 -> 13.3 us, 10,240 (320)
+// 27.5 -> 23.6, 20,480 (640) 41.3 -> 37.2; 40,960 (1,280) 66.4 against 69.3.
+constexpr int HALF_UNITS = 1024;
 constexpr int NXCD = 8;       // XCDs; workgroups are dealt to them round-robin
 
 enum { EPI_STORE = 0, EPI_SOFTPLUS = 1, EPI_TANGENT = 2, EPI_REVERSE = 3 };
@@ -55,16 +60,37 @@ struct GemmDev {
   long cstride;        // floats between the splits' partial outputs
   int M, N, K, lda, ldb, ldc;
   int kchunk;          // K range of one split (a multiple of GK)
+  int nsplit;          // splits that hold a part of K (at least one)
   int vec_out;         // every row-indexed epilogue array takes 16-byte accesses
-  int tiles_n;         // column tiles
-  int tile0;           // first linear tile of this GEMM
+  int tiles, tiles_n;  // C tiles, column tiles
 };
 
 struct GemmBatch {
-  GemmDev g[MAXG];
-  int ngroups, ntiles, per_xcd, epi, io;
+  int unit0[MAXG];     // first unit (C tile of one K split) of each GEMM
+  int ngroups, nunits, per_xcd, epi, io;
   float alpha;
+  GemmDev g[MAXG];
 };
+
+// A workgroup's unit: GEMM, K split and C tile; gi < 0 past the last.
+// Workgroups are dealt to the XCDs round-robin, so workgroup w takes unit
+// (w % 8) * per_xcd + w / 8: each XCD runs a contiguous run of units, and the
+// column tiles of a row block (which share their A rows) meet in one L2.  The
+// units run split by split, tile by tile, GEMM by GEMM, so that GEMMs of
+// unequal K still load the XCDs evenly.
+struct Unit {
+  int gi, split, tm, tn;
+};
+__device__ __forceinline__ Unit unit_of(const GemmBatch& gb) {
+  const int u = (blockIdx.x % NXCD) * gb.per_xcd + blockIdx.x / NXCD;
+  if (u >= gb.nunits) return {-1, 0, 0, 0};
+  int gi = 0;
+#pragma unroll
+  for (int i = 1; i < MAXG; ++i) gi += u >= gb.unit0[i] ? 1 : 0;
+  const int tiles = gb.g[gi].tiles, tiles_n = gb.g[gi].tiles_n;
+  const int local = u - gb.unit0[gi], split = local / tiles, t = local - split * tiles;
+  return {gi, split, t / tiles_n, t % tiles_n};
+}
 
 __device__ __forceinline__ unsigned bf16_bits(float x) {
   return __builtin_bit_cast(unsigned short, (__bf16)x);
@@ -234,6 +260,27 @@ __device__ __forceinline__ void st4h(unsigned short* __restrict__ p, long o, int
   }
 }
 
+// log(1 + e^z) / a of z = a (x + b) and its derivative sigmoid(z), without
+// overflow; the derivative times w.
+__device__ __forceinline__ void softplus_epi(float x, float b, float w, float a, float ia, float& h,
+                                             float& s, float& sw) {
+  const float z = a * (x + b);
+  const float e = __expf(-fabsf(z));
+  h = (fmaxf(z, 0.f) + __logf(1.0f + e)) * ia;
+  s = z >= 0.f ? __fdividef(1.0f, 1.0f + e) : __fdividef(e, 1.0f + e);
+  sw = s * w;
+}
+// The fused multiply-adds are written out: both kernels must round alike.
+__device__ __forceinline__ void tangent_epi(float x, float sg, float ym, float w, float a, float& zt,
+                                            float& ht, float& zb) {
+  zt = x;
+  ht = x * sg;
+  zb = __builtin_fmaf(w, a * sg * (1.0f - sg) * x, sg * ym * w);
+}
+__device__ __forceinline__ float reverse_epi(float x, float sg, float u1, float u2, float a) {
+  return __builtin_fmaf(sg, x, a * sg * (1.0f - sg) * u1 * u2);
+}
+
 // Epilogue of one C tile staged in LDS (Cs[row * CLD + col]): thread t takes
 // columns 4 (t % 32) .. + 3 of rows t / 32 + 8 r.  The outputs (C, aux, out2)
 // never overlap the inputs (bias, s, x1, x2), which restrict states, so a
@@ -278,20 +325,11 @@ __device__ __forceinline__ void epilogue_tile(
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       if (epi == EPI_SOFTPLUS) {
-        const float z = a * (v[k] + bv[k]);
-        // log(1 + e^z) / a and its derivative sigmoid(z), without overflow
-        const float e = __expf(-fabsf(z));
-        r0[k] = (fmaxf(z, 0.f) + __logf(1.0f + e)) * ia;
-        r1[k] = z >= 0.f ? __fdividef(1.0f, 1.0f + e) : __fdividef(e, 1.0f + e);
-        r2[k] = r1[k] * wv[k];
+        softplus_epi(v[k], bv[k], wv[k], a, ia, r0[k], r1[k], r2[k]);
       } else if (epi == EPI_TANGENT) {
-        const float sg = sv[k];
-        r0[k] = v[k];
-        r1[k] = v[k] * sg;
-        r2[k] = sg * ym * wv[k] + a * sg * (1.0f - sg) * v[k] * wv[k];
+        tangent_epi(v[k], sv[k], ym, wv[k], a, r0[k], r1[k], r2[k]);
       } else if (epi == EPI_REVERSE) {
-        const float sg = sv[k];
-        r0[k] = sg * v[k] + a * sg * (1.0f - sg) * u1[k] * u2[k];
+        r0[k] = reverse_epi(v[k], sv[k], u1[k], u2[k], a);
       } else {
         r0[k] = v[k] + bv[k];
       }
@@ -313,29 +351,23 @@ __device__ __forceinline__ void epilogue_tile(
 }
 
 // C tile (GT x GT) of one GEMM of the batch per workgroup, four waves of
-// 64 x 64 (4 x 4 MFMA tiles); blockIdx.y is the K split.  Operands are staged
+// 64 x 64 (4 x 4 MFMA tiles).  Operands are staged
 // through two LDS buffers as BF16 [row][k]; MFMA fragment: lane l takes row
 // l % 16 and k elements 8 (l / 16) .. + 7; the accumulator holds rows
 // 4 (l / 16) .. + 3 of column l % 16.  The next K step's operands are loaded
 // into registers while the current one is multiplied.
-// Workgroups are dealt to the XCDs round-robin, so workgroup w takes tile
-// (w % 8) * per_xcd + w / 8: each XCD runs a contiguous run of tiles, and the
-// column tiles of a row block (which share their A rows) meet in one L2.
 template <bool TA, bool TB, bool VEC, bool BF>
 __global__ void __launch_bounds__(256) gemm_bf16_kernel(const GemmBatch gb) {
   // two staged K steps of A and B, and after the K loop the C tile
   __shared__ __align__(16) unsigned char lds[2 * 2 * GT * LROW * 2];
   auto As = reinterpret_cast<unsigned short (*)[GT][LROW]>(lds);
   auto Bs = reinterpret_cast<unsigned short (*)[GT][LROW]>(lds + 2 * GT * LROW * 2);
-  const int t = (blockIdx.x % NXCD) * gb.per_xcd + blockIdx.x / NXCD;
-  if (t >= gb.ntiles) return;
-  int gi = 0;
-  while (gi + 1 < gb.ngroups && t >= gb.g[gi + 1].tile0) ++gi;
-  const GemmDev& g = gb.g[gi];
+  const Unit un = unit_of(gb);
+  if (un.gi < 0) return;
+  const GemmDev& g = gb.g[un.gi];
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  const int local = t - g.tile0;
-  const int m0 = (local / g.tiles_n) * GT, n0 = (local % g.tiles_n) * GT;
-  const int k_begin = blockIdx.y * g.kchunk;
+  const int m0 = un.tm * GT, n0 = un.tn * GT;
+  const int k_begin = un.split * g.kchunk;
   const int k_end = min(g.K, k_begin + g.kchunk);
   const int nsteps = k_end > k_begin ? (k_end - k_begin + GK - 1) / GK : 0;
   const int wm = (w >> 1) * 64, wn = (w & 1) * 64;
@@ -403,20 +435,386 @@ __global__ void __launch_bounds__(256) gemm_bf16_kernel(const GemmBatch gb) {
         Cs[(wm + 16 * i + (lane >> 4) * 4 + q) * CLD + wn + 16 * j + (lane & 15)] = acc[i][j][q];
   __syncthreads();
   epilogue_tile(Cs, m0, n0, g.M, g.N, g.ldc, gb.epi, gb.alpha, g.vec_out != 0, gb.io, g.crow,
-                g.C != nullptr ? g.C + (long)blockIdx.y * g.cstride : nullptr, g.aux, g.out2,
+                g.C != nullptr ? g.C + (long)un.split * g.cstride : nullptr, g.aux, g.out2,
                 g.bias, g.s, g.x1, g.x2, tid);
+}
+
+// ---------------------------------------------------------------------------
+// The GEMM of BF16 operands in the layouts that the training step keeps them
+// in (gemm_wide() below says which); gemm_bf16_kernel takes everything else.
+// Its K order per output is that kernel's, so the results are equal bit for
+// bit.
+//
+// What bounded these GEMMs (8 to 12 K steps each) was not arithmetic: the
+// epilogue, one body for all four formulas with a branch per row, took 10 of
+// 27 us even for a plain store (20,000 cycles of instruction fetch and of one
+// load latency per row), 2-byte loads of the operand stored across k another
+// third, and the first instructions' chain of scalar loads 2 us.  Here each
+// epilogue is its own kernel with branch-free buffer accesses and the next
+// rows' inputs in flight, operands load in 16-byte chunks two K steps ahead,
+// and a launch of few tiles uses 64 x 128 ones (HALF_UNITS).  10,240 rows,
+// N = K = 512: plain 27.7 -> 17.2 us, softplus 33.8 -> 23, tangent 32.2 ->
+// 18.4, reverse 31.0 -> 21.7; the weight-gradient launch of 10,398 atoms
+// 259 -> 124 us, of which 40 came from units that run split by split, so that
+// every XCD gets the same share of GEMMs with unequal K.  What is left is the
+// issue of loads, LDS stores and LDS reads by one or two workgroups per CU
+// (a step's MFMAs are a quarter of its time) and launch latency.
+//
+// LDS image of a staged operand: S[row][k] in BF16, 128 bytes per row, so an
+// MFMA fragment (8 consecutive k of one row) is one 16-byte read.  Chunk c (16
+// bytes) of a row sits at c ^ swz(row): the 16 rows of a fragment read, the 8
+// chunks of a row store and eight lanes (rows 8 l + e) of a transposing store
+// fall on different banks.
+__device__ __forceinline__ int swz(int row) { return ((row >> 1) ^ (row >> 3)) & 7; }
+__device__ __forceinline__ int lds_at(int row, int chunk) {
+  return row * GK + ((chunk ^ swz(row)) << 3);
+}
+
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+constexpr unsigned OOB = 0x80000000u;   // a byte offset past every buffer: reads 0, writes nothing
+
+// Buffer over `bytes` from p; offsets of a tile stay far below the clamp.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_buffer(const void* p, long bytes) {
+  const long n = p == nullptr ? 0 : min(max(bytes, 0l), 0x7ffffff8l);
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)n, 0x00027000);
+}
+
+// One operand's share of a K step (ROWS rows x GK) in registers between its
+// global load and its LDS store.  Loads are branch-free buffer loads, so that
+// the waits the compiler sets count exactly the loads in flight (a branch
+// around them makes it wait for all).
+// KCONT, element (r, k) at X[r * ld + k]: thread t takes the 16 bytes at k =
+// 8 (t % 8) of rows t / 8 + 32 i; a row past the last is read as the last (it
+// only feeds outputs that are not stored), a chunk past K reads zero.
+// Otherwise element (r, k) at X[k * ld + r]: thread t takes the 16 bytes of
+// rows 8 (t % 16) .. + 7 at k = 4 (t / 16) .. + 3 (16 lanes read 256
+// contiguous bytes) and transposes its 4 x 8 block with 16 byte permutes on
+// the way to LDS.  The buffer ends with the operand (rounded up to the 16
+// bytes a load takes), so that k past K reads zero.  A single row (the output
+// layer's weights) is read by value.
+template <bool KCONT, int ROWS>
+struct WideStage {
+  static_assert(KCONT || ROWS == GT, "the transposing form stages GT rows");
+  static constexpr int NV = ROWS / 32;
+  u32x4 v[NV];
+  __amdgpu_buffer_rsrc_t buf;
+  unsigned voff[KCONT ? NV : 1];
+  unsigned kstep;     // bytes per k (not KCONT)
+  int kleft;          // K left behind this thread's chunk (KCONT)
+  bool narrow;
+
+  __device__ __forceinline__ void init(const unsigned short* X, int ld, int rows, int r0, int K,
+                                       int k_begin, int tid) {
+    if constexpr (KCONT) {
+      buf = tile_buffer(X + (long)r0 * ld + k_begin,
+                        2 * ((long)(rows - 1 - r0) * ld + K - k_begin));
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+        voff[i] = 2u * (unsigned)(min((tid >> 3) + 32 * i, rows - 1 - r0) * ld) + (tid & 7) * 16u;
+      kleft = K - k_begin - (tid & 7) * 8;
+      narrow = false;
+      kstep = 0;
+    } else {
+      narrow = rows == 1;
+      const long end = 2 * ((long)(K - 1 - k_begin) * ld + rows - r0);
+      buf = tile_buffer(X + (long)k_begin * ld + r0, narrow ? end : (end + 15) & ~15l);
+      kstep = 2u * ld;
+      voff[0] = 4u * (tid >> 4) * kstep + (tid & 15) * 16u;
+      if (narrow && (tid & 15) != 0) voff[0] = OOB;
+      kleft = 0;
+    }
+  }
+
+  // K step `step`; kill = OOB loads nothing.
+  __device__ __forceinline__ void load(int step, unsigned kill) {
+    if constexpr (KCONT) {
+      const unsigned dead = kleft > step * GK ? kill : OOB;
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+        v[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                             buf, voff[i] | dead, step * (2 * GK), 0));
+    } else {
+      const unsigned o = (voff[0] + (unsigned)step * (GK * kstep)) | kill;
+      if (narrow) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          v[q] = u32x4{(unsigned)(unsigned short)__builtin_amdgcn_raw_buffer_load_b16(
+                           buf, o + q * kstep, 0, 0), 0u, 0u, 0u};
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          v[q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                               buf, o + q * kstep, 0, 0));
+      }
+    }
+  }
+
+  __device__ __forceinline__ void store(unsigned short* S, int tid) const {
+    if constexpr (KCONT) {
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+        *reinterpret_cast<u32x4*>(&S[lds_at((tid >> 3) + 32 * i, tid & 7)]) = v[i];
+    } else {
+      const int row = 8 * (tid & 15), k = 4 * (tid >> 4);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {   // row 8 l + e at k .. k + 3
+        const unsigned sel = e & 1 ? 0x07060302u : 0x05040100u;
+        *reinterpret_cast<u32x2*>(&S[lds_at(row + e, k >> 3) + (k & 4)]) =
+            u32x2{__builtin_amdgcn_perm(v[1][e >> 1], v[0][e >> 1], sel),
+                  __builtin_amdgcn_perm(v[3][e >> 1], v[2][e >> 1], sel)};
+      }
+    }
+  }
+};
+
+__device__ __forceinline__ float4 buf_ld4(__amdgpu_buffer_rsrc_t b, unsigned o) {
+  return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(b, o, 0, 0));
+}
+// Four values at element offset e, FP32 or rounded to BF16.
+__device__ __forceinline__ void buf_st4(__amdgpu_buffer_rsrc_t b, unsigned e, bool half,
+                                        const float (&v)[4]) {
+  if (half)
+    __builtin_amdgcn_raw_buffer_store_b64(
+        u32x2{bf16_bits(v[0]) | (bf16_bits(v[1]) << 16), bf16_bits(v[2]) | (bf16_bits(v[3]) << 16)},
+        b, e * 2u, 0, 0);
+  else
+    __builtin_amdgcn_raw_buffer_store_b128(
+        __builtin_bit_cast(u32x4, make_float4(v[0], v[1], v[2], v[3])), b, e * 4u, 0, 0);
+}
+
+template <bool TA, bool TB, int EPI, int GM>
+__global__ void __launch_bounds__(256, GM == GT ? 2 : 3) gemm_wide_kernel(const GemmBatch gb) {
+  // two staged K steps of A (GM rows) and B, and after the K loop the C tile
+  constexpr int AOP = GM * GK, BOP = GT * GK;   // elements of a staged operand
+  constexpr int MI = GM / 32;                   // 16-row blocks per wave
+  constexpr int CB = GM * CLD * 4, OB = 4 * (AOP + BOP);
+  __shared__ __align__(16) unsigned char lds[CB > OB ? CB : OB];
+  unsigned short* As = reinterpret_cast<unsigned short*>(lds);
+  unsigned short* Bs = As + 2 * AOP;
+  const Unit un = unit_of(gb);
+  if (un.gi < 0) return;
+  const GemmDev& g = gb.g[un.gi];
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int M = g.M, N = g.N, split = un.split;
+  const int m0 = un.tm * GM, n0 = un.tn * GT;
+  const int k_begin = split * g.kchunk;
+  const int nsteps = max(min(g.K - k_begin, g.kchunk) + GK - 1, 0) / GK;
+  const int wm = (w >> 1) * (GM / 2), wn = (w & 1) * 64;
+  WideStage<!TA, GM> sa[2];
+  WideStage<TB, GT> sb[2];
+  sa[0].init(reinterpret_cast<const unsigned short*>(g.A), g.lda, M, m0, g.K, k_begin, tid);
+  sb[0].init(reinterpret_cast<const unsigned short*>(g.B), g.ldb, N, n0, g.K, k_begin, tid);
+  sa[1] = sa[0];
+  sb[1] = sb[0];
+  auto load = [&](int step, auto& xa, auto& xb) {
+    const unsigned kill = step < nsteps ? 0u : OOB;
+    xa.load(step, kill);
+    xb.load(step, kill);
+  };
+  load(0, sa[0], sb[0]);
+  __builtin_amdgcn_sched_barrier(0);   // in this order: the waits count loads in flight
+  load(1, sa[1], sb[1]);
+  __builtin_amdgcn_sched_barrier(0);
+  floatx4 acc[MI][4];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  // 16-row blocks of this wave's quadrant that hold output; the others only
+  // feed rows and columns that are not stored
+  const int nj = (N - n0 - wn + 15) >> 4, mi = nj > 0 ? min((M - m0 - wm + 15) >> 4, MI) : 0;
+  const int fr = lane & 15, fc = lane >> 4;
+  // One K step from LDS buffer b.
+  auto multiply = [&](int b, auto full) {
+    const unsigned short* Ab = As + b * AOP;
+    const unsigned short* Bb = Bs + b * BOP;
+#pragma unroll
+    for (int kk = 0; kk < GK / 8; kk += 4) {
+      uint4 fa[MI], fb[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        fb[j] = *reinterpret_cast<const uint4*>(&Bb[lds_at(wn + 16 * j + fr, kk + fc)]);
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+        fa[i] = *reinterpret_cast<const uint4*>(&Ab[lds_at(wm + 16 * i + fr, kk + fc)]);
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        if (full || i < mi) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                __builtin_bit_cast(bf16x8, fb[j]), __builtin_bit_cast(bf16x8, fa[i]), acc[i][j], 0,
+                0, 0);
+        }
+      }
+    }
+  };
+  // The waves of a workgroup may take different branches here: they meet at
+  // the same number of barriers.
+  auto kloop = [&](auto full) {
+    for (int step = 0; step < nsteps; step += 2) {
+      sa[0].store(As, tid);
+      sb[0].store(Bs, tid);
+      __syncthreads();
+      load(step + 2, sa[0], sb[0]);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(0, full);
+      sa[1].store(As + AOP, tid);
+      sb[1].store(Bs + BOP, tid);
+      __syncthreads();
+      load(step + 3, sa[1], sb[1]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (step + 1 < nsteps) multiply(1, full);
+    }
+  };
+  if (mi == MI) kloop(std::true_type{});
+  else kloop(std::false_type{});
+  // Epilogue (the formulas: epilogue_tile).  The C tile goes through LDS;
+  // thread t takes columns 4 (t % 32) .. + 3 of rows t / 32 + 8 r, ER rows at
+  // a time.  The row-indexed inputs of the next ER rows are in flight while
+  // these are computed and stored; the first are requested before the tile is
+  // in LDS.  Rows past the last lie outside the buffers: they read zero and
+  // write nothing.
+  constexpr int ER = 4, NB = GM / 8 / ER;
+  constexpr bool HAS_S = EPI == EPI_TANGENT || EPI == EPI_REVERSE;
+  const int c = (tid & 31) * 4, n = n0 + c, row = tid >> 5, io = gb.io;
+  const long ldc = g.ldc, left = (long)(M - 1 - m0) * ldc + N;   // elements from row m0 on
+  const long at = (long)m0 * ldc;
+  const unsigned e0 = (unsigned)(row * (int)ldc + n);
+  const unsigned estep = 8u * (unsigned)ldc;                     // elements from r to r + 1
+  auto fbuf = [&](const float* p) { return tile_buffer(p == nullptr ? p : p + at, left * 4); };
+  auto obuf = [&](float* p, int bit) {
+    const int bytes = io & bit ? 2 : 4;
+    return tile_buffer(p == nullptr ? nullptr : reinterpret_cast<char*>(p) + at * bytes,
+                       left * bytes);
+  };
+  float bv[4] = {0.f, 0.f, 0.f, 0.f}, wv[4] = {0.f, 0.f, 0.f, 0.f};
+  __amdgpu_buffer_rsrc_t bs = fbuf(g.s), b1 = fbuf(g.x1), b2 = fbuf(g.x2);
+  struct In {
+    float4 s[ER], u1[ER], u2[ER];
+    float ym[ER];
+  } cur, nxt;
+  const bool has_out2 = EPI != EPI_STORE && EPI != EPI_REVERSE && g.out2 != nullptr;
+  auto fetch = [&](In& q, int b) {
+#pragma unroll
+    for (int j = 0; j < ER; ++j) {
+      const unsigned e = e0 + (unsigned)(ER * b + j) * estep;
+      if (HAS_S) q.s[j] = buf_ld4(bs, e * 4u);
+      if (EPI == EPI_REVERSE) {
+        q.u1[j] = buf_ld4(b1, e * 4u);
+        q.u2[j] = buf_ld4(b2, e * 4u);
+      }
+      if (EPI == EPI_TANGENT)
+        q.ym[j] = has_out2 ? g.x2[min(m0 + row + 8 * (ER * b + j), M - 1)] : 0.f;
+    }
+  };
+  int crow[EPI == EPI_STORE ? GM / 8 : 1];
+  if (n < N) {
+    fetch(cur, 0);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (g.bias != nullptr && n + k < N) bv[k] = g.bias[n + k];
+      if (has_out2) wv[k] = g.x1[n + k];
+    }
+    if (EPI == EPI_STORE && g.crow != nullptr) {
+#pragma unroll
+      for (int r = 0; r < GM / 8; ++r) crow[r] = g.crow[min(m0 + row + 8 * r, M - 1)];
+    }
+  }
+  __syncthreads();   // every wave is done with the staged operands
+  float* Cs = reinterpret_cast<float*>(lds);
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      *reinterpret_cast<floatx4*>(&Cs[(wm + 16 * i + fr) * CLD + wn + 16 * j + fc * 4]) = acc[i][j];
+  __syncthreads();
+  if (n >= N) return;
+  const float* Ct = Cs + row * CLD + c;
+  if constexpr (EPI == EPI_STORE) {
+    float* C = g.C + (long)split * g.cstride;
+    const bool half = (io & 2) != 0;
+    if (g.crow == nullptr && g.vec_out && n + 4 <= N) {
+      const __amdgpu_buffer_rsrc_t bc = obuf(C, 2);
+#pragma unroll 4
+      for (int r = 0; r < GM / 8; ++r) {
+        const float4 f = *reinterpret_cast<const float4*>(Ct + r * 8 * CLD);
+        const float o[4] = {f.x + bv[0], f.y + bv[1], f.z + bv[2], f.w + bv[3]};
+        buf_st4(bc, e0 + r * estep, half, o);
+      }
+    } else {   // a row map, or columns that do not take 16-byte stores
+      const int nv = min(4, N - n);
+#pragma unroll
+      for (int r = 0; r < GM / 8; ++r) {
+        const int m = m0 + row + 8 * r;
+        if (m >= M) break;
+        const long o = (long)(g.crow != nullptr ? crow[r] : m) * ldc + n;
+        const float4 f = *reinterpret_cast<const float4*>(Ct + r * 8 * CLD);
+        const float v[4] = {f.x + bv[0], f.y + bv[1], f.z + bv[2], f.w + bv[3]};
+        if (half) st4h(reinterpret_cast<unsigned short*>(C), o, nv, g.vec_out != 0, v);
+        else st4(C, o, nv, g.vec_out != 0, v);
+      }
+    }
+    return;
+  }
+  const float a = gb.alpha, ia = 1.0f / a;
+  const __amdgpu_buffer_rsrc_t bc = obuf(g.C, 2), ba = obuf(g.aux, 4), bo = obuf(g.out2, 8);
+  const bool hc = (io & 2) != 0, ha = (io & 4) != 0, ho = (io & 8) != 0;
+#pragma unroll 1
+  for (int b = 0; b < NB; ++b) {
+    if (HAS_S && b + 1 < NB) fetch(nxt, b + 1);
+#pragma unroll
+    for (int j = 0; j < ER; ++j) {
+      const unsigned e = e0 + (unsigned)(ER * b + j) * estep;
+      const float4 f = *reinterpret_cast<const float4*>(Ct + (ER * b + j) * 8 * CLD);
+      const float v[4] = {f.x, f.y, f.z, f.w};
+      float sv[4], u1[4], u2[4], r0[4], r1[4], r2[4];
+      if (HAS_S) { sv[0] = cur.s[j].x; sv[1] = cur.s[j].y; sv[2] = cur.s[j].z; sv[3] = cur.s[j].w; }
+      if (EPI == EPI_REVERSE) {
+        u1[0] = cur.u1[j].x; u1[1] = cur.u1[j].y; u1[2] = cur.u1[j].z; u1[3] = cur.u1[j].w;
+        u2[0] = cur.u2[j].x; u2[1] = cur.u2[j].y; u2[2] = cur.u2[j].z; u2[3] = cur.u2[j].w;
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if constexpr (EPI == EPI_SOFTPLUS) softplus_epi(v[k], bv[k], wv[k], a, ia, r0[k], r1[k], r2[k]);
+        else if constexpr (EPI == EPI_TANGENT)
+          tangent_epi(v[k], sv[k], cur.ym[j], wv[k], a, r0[k], r1[k], r2[k]);
+        else r0[k] = reverse_epi(v[k], sv[k], u1[k], u2[k], a);
+      }
+      if (EPI != EPI_TANGENT || g.C != nullptr) buf_st4(bc, e, hc, r0);
+      if (EPI != EPI_REVERSE) buf_st4(ba, e, ha, r1);
+      if (has_out2) buf_st4(bo, e, ho, r2);
+    }
+    if (HAS_S) cur = nxt;
+  }
 }
 
 // out = sum over the splits of their partial outputs, in split order; one
 // GEMM of the batch per blockIdx.y.
-__global__ void split_sum_kernel(const GemmBatch gb, int nsplit) {
+__global__ void split_sum_kernel(const GemmBatch gb) {
   const GemmDev& g = gb.g[blockIdx.y];
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long)g.M * g.N) return;
-  const long o = (t / g.N) * g.ldc + t % g.N;
-  float v = 0.f;
-  for (int z = 0; z < nsplit; ++z) v += g.C[z * g.cstride + o];
-  g.out[o] = v;
+  const long n4 = (g.N + 3) / 4;
+  if (t >= n4 * g.M) return;
+  const long m = t < 0x7fffffff ? (int)t / (int)n4 : t / n4;
+  const int n = (int)(t - m * n4) * 4;
+  const long o = m * g.ldc + n;
+  if (g.vec_out && n + 4 <= g.N) {
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+    for (int z = 0; z < g.nsplit; ++z) {
+      const float4 x = *reinterpret_cast<const float4*>(g.C + z * g.cstride + o);
+      v.x += x.x; v.y += x.y; v.z += x.z; v.w += x.w;
+    }
+    *reinterpret_cast<float4*>(g.out + o) = v;
+    return;
+  }
+  for (int k = 0; k < 4 && n + k < g.N; ++k) {
+    float v = 0.f;
+    for (int z = 0; z < g.nsplit; ++z) v += g.C[z * g.cstride + o + k];
+    g.out[o + k] = v;
+  }
 }
 
 // Elementwise steps between the GEMMs (row r < M, column n < H; ld = row stride
@@ -605,49 +1003,85 @@ int tm_gemm_bf16_grouped(int ngroups, const tm_gemm_group* groups, int ta, int t
                                {TM_GEMM_K(true, false), TM_GEMM_K(true, true)}};
 #undef TM_GEMM_K
   const Kern kern = kerns[ta ? 1 : 0][tb ? 1 : 0][(vec ? 2 : 0) + (bf ? 1 : 0)];
-  for (int g0 = 0; g0 < ngroups;) {
-    GemmBatch gb;
-    gb.ngroups = 0;
-    gb.ntiles = 0;
-    gb.epi = epi;
-    gb.io = io;
-    gb.alpha = alpha;
-    long max_mn = 0;
-    for (; g0 < ngroups && gb.ngroups < MAXG; ++g0) {
-      const tm_gemm_group& q = groups[g0];
-      if (q.M == 0 || q.N == 0) continue;
-      GemmDev& d = gb.g[gb.ngroups++];
-      d.A = static_cast<const float*>(q.A);
-      d.B = static_cast<const float*>(q.B);
-      d.out = static_cast<float*>(q.C);
-      d.C = nsplit > 1 ? q.work : static_cast<float*>(q.C);
-      d.bias = q.bias; d.s = q.s; d.aux = static_cast<float*>(q.aux);
-      d.x1 = q.x1; d.x2 = q.x2; d.out2 = static_cast<float*>(q.out2);
-      d.crow = q.crow;
-      {
-        // 16-byte epilogue accesses: FP32 arrays 16-byte aligned, BF16 outputs 8-byte
-        const bool rev = epi == EPI_REVERSE;
-        d.vec_out = q.ldc % 4 == 0 && aligned(d.C, (io & 2) && nsplit == 1 ? 8 : 16) &&
-                    aligned(q.aux, (io & 4) ? 8 : 16) && aligned(q.out2, (io & 8) ? 8 : 16) &&
-                    aligned(q.s, 16) && (!rev || (aligned(q.x1, 16) && aligned(q.x2, 16)));
+  // gemm_wide_kernel's layouts: BF16 operands in 16-byte chunks (or a single
+  // row with ld elements from k to k + 1); 32-bit offsets; 16-byte epilogue accesses (the plain epilogue stores any width).
+  auto gemm_wide = [&](const tm_gemm_group& q, bool vec_out) {
+    auto oper = [&](const void* p, long ld, int rows, bool kcont) {
+      if (kcont) return ld % 8 == 0 && q.K % 8 == 0 && aligned(p, 16) && (GT * ld + q.K) * 2 < (1l << 31);
+      return ld >= rows && (rows == 1 || (ld % 8 == 0 && aligned(p, 16))) &&
+             (q.K + 4l * GK) * ld * 2 < (1l << 31);
+    };
+    return bf && oper(q.A, q.lda, q.M, !ta) && oper(q.B, q.ldb, q.N, tb != 0) && q.ldc >= q.N &&
+           (long)GT * q.ldc * 4 < (1l << 31) &&
+           (epi == EPI_STORE || (vec_out && q.N % 4 == 0));
+  };
+#define TM_GEMM_W(a, b, m)                                                              \
+  {gemm_wide_kernel<a, b, EPI_STORE, m>, gemm_wide_kernel<a, b, EPI_SOFTPLUS, m>,       \
+   gemm_wide_kernel<a, b, EPI_TANGENT, m>, gemm_wide_kernel<a, b, EPI_REVERSE, m>}
+  const Kern wides[2][2][4] = {{TM_GEMM_W(false, false, GT), TM_GEMM_W(false, true, GT)},
+                               {TM_GEMM_W(true, false, GT), TM_GEMM_W(true, true, GT)}};
+  const Kern halves[2][4] = {TM_GEMM_W(false, false, GT / 2), TM_GEMM_W(false, true, GT / 2)};
+#undef TM_GEMM_W
+  for (int wide = 1; wide >= 0; --wide) {
+    for (int g0 = 0; g0 < ngroups;) {
+      GemmBatch gb;
+      gb.ngroups = 0;
+      gb.nunits = 0;
+      gb.epi = epi;
+      gb.io = io;
+      gb.alpha = alpha;
+      long most = 0;
+      for (; g0 < ngroups && gb.ngroups < MAXG; ++g0) {
+        const tm_gemm_group& q = groups[g0];
+        if (q.M == 0 || q.N == 0) continue;
+        GemmDev d;
+        d.A = static_cast<const float*>(q.A);
+        d.B = static_cast<const float*>(q.B);
+        d.out = static_cast<float*>(q.C);
+        d.C = nsplit > 1 ? q.work : static_cast<float*>(q.C);
+        d.bias = q.bias; d.s = q.s; d.aux = static_cast<float*>(q.aux);
+        d.x1 = q.x1; d.x2 = q.x2; d.out2 = static_cast<float*>(q.out2);
+        d.crow = q.crow;
+        {
+          // 16-byte epilogue accesses: FP32 arrays 16-byte aligned, BF16 outputs 8-byte
+          const bool rev = epi == EPI_REVERSE;
+          d.vec_out = q.ldc % 4 == 0 && aligned(d.C, (io & 2) && nsplit == 1 ? 8 : 16) &&
+                      aligned(q.aux, (io & 4) ? 8 : 16) && aligned(q.out2, (io & 8) ? 8 : 16) &&
+                      aligned(q.s, 16) && (!rev || (aligned(q.x1, 16) && aligned(q.x2, 16))) &&
+                      (nsplit == 1 || aligned(q.C, 16));
+        }
+        if (gemm_wide(q, d.vec_out != 0) != (wide != 0)) continue;
+        d.M = q.M; d.N = q.N; d.K = q.K;
+        d.lda = q.lda; d.ldb = q.ldb; d.ldc = q.ldc;
+        d.cstride = (long)q.M * q.ldc;
+        const int steps = (q.K + GK - 1) / GK;
+        const int per = std::max((steps + nsplit - 1) / nsplit, std::min(steps, MINSTEPS));
+        d.kchunk = std::max(per, 1) * GK;
+        d.nsplit = per == 0 ? 1 : (steps + per - 1) / per;
+        d.tiles_n = tm_div_up(q.N, GT);
+        d.tiles = d.tiles_n * tm_div_up(q.M, GT);
+        gb.nunits += d.tiles * d.nsplit;
+        most = std::max(most, (long)q.M * ((q.N + 3) / 4));
+        gb.g[gb.ngroups++] = d;
       }
-      d.M = q.M; d.N = q.N; d.K = q.K;
-      d.lda = q.lda; d.ldb = q.ldb; d.ldc = q.ldc;
-      d.cstride = (long)q.M * q.ldc;
-      const int steps = (q.K + GK - 1) / GK;
-      d.kchunk = steps == 0 ? GK : ((steps + nsplit - 1) / nsplit) * GK;
-      d.tiles_n = tm_div_up(q.N, GT);
-      d.tile0 = gb.ntiles;
-      gb.ntiles += d.tiles_n * tm_div_up(q.M, GT);
-      max_mn = std::max(max_mn, (long)q.M * q.N);
-    }
-    if (gb.ngroups == 0) continue;
-    gb.per_xcd = tm_div_up(gb.ntiles, NXCD);
-    kern<<<dim3(NXCD * gb.per_xcd, nsplit), 256, 0, st>>>(gb);
-    TM_LAUNCH_CHECK();
-    if (nsplit > 1) {
-      split_sum_kernel<<<dim3(tm_div_up(max_mn, 256), gb.ngroups), 256, 0, st>>>(gb, nsplit);
+      if (gb.ngroups == 0) continue;
+      const bool half = wide && !ta && gb.nunits < HALF_UNITS;
+      gb.nunits = 0;
+      for (int i = 0; i < MAXG; ++i) {
+        gb.unit0[i] = i < gb.ngroups ? gb.nunits : 0x7fffffff;
+        if (i >= gb.ngroups) continue;
+        GemmDev& d = gb.g[i];
+        d.tiles = d.tiles_n * tm_div_up(d.M, half ? GT / 2 : GT);
+        gb.nunits += d.tiles * d.nsplit;
+      }
+      gb.per_xcd = tm_div_up(gb.nunits, NXCD);
+      const Kern k = !wide ? kern : half ? halves[tb ? 1 : 0][epi] : wides[ta ? 1 : 0][tb ? 1 : 0][epi];
+      k<<<NXCD * gb.per_xcd, 256, 0, st>>>(gb);
       TM_LAUNCH_CHECK();
+      if (nsplit > 1) {
+        split_sum_kernel<<<dim3(tm_div_up(most, 256), gb.ngroups), 256, 0, st>>>(gb);
+        TM_LAUNCH_CHECK();
+      }
     }
   }
   return TM_OK;
