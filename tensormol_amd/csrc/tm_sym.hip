@@ -113,11 +113,24 @@ __device__ __forceinline__ float sin_between(const float4& dj, const float4& dk,
 }
 __device__ __forceinline__ float cutoff_dfc(float k, float r) { return -0.5f * k * __sinf(k * r); }
 
-template <class LDS>
+// A lane's slots of row i; slots past the row's end hold anything.  Read
+// before the row's length is known, so that the two loads overlap.
+template <int RC>
+__device__ __forceinline__ void row_slots(int (&jq)[RC / 64], const int* __restrict__ nbr, int i,
+                                          int lane, int ldr) {
+#pragma unroll
+  for (int k = 0; k < RC / 64; ++k) {
+    const int q = lane + 64 * k;
+    jq[k] = q < ldr ? nbr[(long)i * ldr + q] : 0;
+  }
+}
+
+// more(q, j, d): what else slot q needs
+template <int RC, class LDS, class More>
 __device__ __forceinline__ void load_row(int i, int w, int lane, const double* __restrict__ pos,
                                          const double* __restrict__ box, const int* __restrict__ mol,
-                                         const int* __restrict__ nbr, int n, int ldr,
-                                         const SymArgs& a, LDS& L) {
+                                         const int (&jq)[RC / 64], int n, const SymArgs& a, LDS& L,
+                                         More more) {
   // minimum image with the reciprocal edge (iL = 0 for open boundaries): it
   // differs from d - L rint(d / L) only at |d| = L/2, far beyond the cutoff
   double Lx = 0, Ly = 0, Lz = 0, iLx = 0, iLy = 0, iLz = 0;
@@ -127,8 +140,10 @@ __device__ __forceinline__ void load_row(int i, int w, int lane, const double* _
     iLx = 1.0 / Lx; iLy = 1.0 / Ly; iLz = 1.0 / Lz;
   }
   const double xi = pos[3 * i], yi = pos[3 * i + 1], zi = pos[3 * i + 2];
-  for (int q = lane; q < n; q += 64) {
-    int j = nbr[(long)i * ldr + q];
+#pragma unroll
+  for (int k = 0; k < RC / 64; ++k) {
+    const int q = lane + 64 * k, j = jq[k];
+    if (q >= n) break;
     double ex = pos[3 * j] - xi, ey = pos[3 * j + 1] - yi, ez = pos[3 * j + 2] - zi;
     float dx = (float)(ex - Lx * rint(ex * iLx));
     float dy = (float)(ey - Ly * rint(ey * iLy));
@@ -136,39 +151,124 @@ __device__ __forceinline__ void load_row(int i, int w, int lane, const double* _
     float r = sqrtf(dx * dx + dy * dy + dz * dz + 1e-27f);
     L.d[w][q] = make_float4(dx, dy, dz, r);
     if constexpr (LDS::has_fc) L.fc[w][q] = cutoff_fc(a.kr, r);
+    more(q, j, L.d[w][q]);
   }
 }
 
-// decode triple index t (in the centre's enumeration) into sub-list
-// positions (ja, kb) and the element pair p; blocks are ordered by
-// (ea <= eb) and inside a block by (k, j)
-__device__ __forceinline__ void decode_triple(int t, const int* seg, int nele, int& ja, int& kb,
-                                              int& p) {
-  p = 0;
-  for (int ea = 0; ea < nele; ++ea) {
-    int la = seg[ea + 1] - seg[ea];
-    for (int eb = ea; eb < nele; ++eb, ++p) {
-      int lb = seg[eb + 1] - seg[eb];
-      int nb = (ea == eb) ? la * (la - 1) / 2 : la * lb;
-      if (t < nb) {
-        if (ea != eb) {
-          kb = seg[eb] + t / la;
-          ja = seg[ea] + t % la;
-        } else {
-          // k-major triangle: k = 1.., j < k; t = k(k-1)/2 + j
-          int k = (int)((1.0f + sqrtf(1.0f + 8.0f * (float)t)) * 0.5f);
-          while (k * (k - 1) / 2 > t) --k;
-          while ((k + 1) * k / 2 <= t) ++k;
-          kb = seg[ea] + k;
-          ja = seg[ea] + (t - k * (k - 1) / 2);
-        }
-        return;
+// Segment boundary e of a lane register that holds boundary l in lane l.
+__device__ __forceinline__ int seg_at(int v, int e) { return __builtin_amdgcn_readlane(v, e); }
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_swap(float x) {   // another lane's x of the same quad
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL,
+                                                               0xf, 0xf, true));
+}
+// x of lane ^ 4: lanes 0-3 and 8-11 of a row read four lanes up, the others down
+__device__ __forceinline__ float dpp_swap4(float x) {
+  const int v = __builtin_bit_cast(int, x);
+  const int up = __builtin_amdgcn_update_dpp(0, v, 0x104, 0xf, 0x5, false);
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(up, v, 0x114, 0xf, 0xa, false));
+}
+
+// Sum of v[s] over the 8 lanes of a group, for s = the lane's own number g:
+// ((0 + 1) + (2 + 3)) + ((4 + 5) + (6 + 7)).  Each step hands half of the
+// shells that are left to the partner and keeps the other half.
+__device__ __forceinline__ float group_sum8(const float (&v)[8], int g) {
+  const bool b0 = g & 1, b1 = g & 2, b2 = g & 4;
+  float x[4], y[2];
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    x[k] = (b0 ? v[2 * k + 1] : v[2 * k]) + dpp_swap<0xB1>(b0 ? v[2 * k] : v[2 * k + 1]);
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+    y[k] = (b1 ? x[2 * k + 1] : x[2 * k]) + dpp_swap<0x4E>(b1 ? x[2 * k] : x[2 * k + 1]);
+  return (b2 ? y[1] : y[0]) + dpp_swap4(b2 ? y[0] : y[1]);
+}
+
+// The angular functions of one centre, 64 triples at a time.  Triples are
+// ordered by element pair (ea <= eb), inside a pair by (k, j), so each pair is
+// a contiguous range of the enumeration.
+// Phase A: lane = triple, stage(ja, kb) puts its geometry into LDS (ja, kb:
+// places in the angular sub-list).  Phase B: lane = (theta point t, triple
+// group g); it takes every 8th triple u of a pair's range, term(u, acc) adds it
+// to one accumulator per shell.  When a pair ends, the 8 groups are summed and
+// lane (t, g) writes shell s = g.
+// av: boundary e of the sub-list's element segments in lane e.
+//
+// An atom of an organic molecule has some 50 triples in ten pairs, so what a
+// pair costs besides its triples decides.  The walk over the pairs is
+// wave-uniform (scalar registers) and keeps its place from chunk to chunk, an
+// empty pair is one store, the 8 groups are summed with lane permutes of the
+// vector unit (24 LDS permutes before), and members' places come from LDS, not
+// from the list in memory.  Angular part of a wave, median cycles: 12,288-atom
+// water box 10,400 -> 7,100, 24,000-atom C/H/N/O sphere 33,200 -> 16,300.
+// Lists and descriptors of 37 chains (2,139 atoms) 38.5 -> 25.4 us, of the box
+// 76 -> 64; descriptors of 10,398 chain atoms 61 -> 36 and their tangent
+// 74 -> 47.  Reading the next pair's first triples ahead and keeping the pairs'
+// ranges per lane gained nothing.
+template <class Stage, class Term>
+__device__ __forceinline__ void angular_pass(int lane, int nele, int nelep, int av, int ntrip,
+                                             float scale, float* __restrict__ out, Stage stage,
+                                             Term term) {
+  const int g = lane & 7;
+  float acc[NA];
+#pragma unroll
+  for (int s = 0; s < NA; ++s) acc[s] = 0.f;
+  int p = 0, ea = 0, eb = 0, T = 0;   // pair in progress and its first triple
+  auto pairs = [&](int x, int y) {
+    const int la = seg_at(av, x + 1) - seg_at(av, x);
+    return x == y ? la * (la - 1) / 2 : la * (seg_at(av, y + 1) - seg_at(av, y));
+  };
+  for (int base = 0; base < ntrip; base += 64) {
+    const int cnt = min(64, ntrip - base), t = base + lane;
+    {
+      // place of triple t: walk over the pairs that this chunk touches
+      int sa = 0, sb = 0, la = 0, tl = 0;
+      int xa = ea, xb = eb, X = T;
+      while (X < base + cnt && xa < nele) {
+        const int s0 = seg_at(av, xa), l0 = seg_at(av, xa + 1) - s0, s1 = seg_at(av, xb);
+        const bool in = t >= X;
+        sa = in ? s0 : sa;
+        sb = in ? s1 : sb;
+        la = in ? (xa == xb ? 0 : l0) : la;
+        tl = in ? t - X : tl;
+        X += pairs(xa, xb);
+        if (++xb == nele) xb = ++xa;
       }
-      t -= nb;
+      int ja, kb;
+      if (la == 0) {   // k-major triangle: tl = k (k - 1) / 2 + j, j < k
+        int k = (int)((1.0f + sqrtf(1.0f + 8.0f * (float)tl)) * 0.5f);
+        k -= k * (k - 1) / 2 > tl ? 1 : 0;
+        k += (k + 1) * k / 2 <= tl ? 1 : 0;
+        kb = sb + k;
+        ja = sa + (tl - k * (k - 1) / 2);
+      } else {         // (tl + 1/2) / la is at least 1 / (2 la) away from an integer
+        const int k = (int)(((float)tl + 0.5f) * __builtin_amdgcn_rcpf((float)la));
+        kb = sb + k;
+        ja = sa + (tl - k * la);
+      }
+      if (t < ntrip) stage(ja, kb);
     }
+    __syncwarp();
+    while (p < nelep) {
+      const int n = pairs(ea, eb), Te = T + n;
+      const int lo = max(T - base, 0), hi = min(Te - base, cnt);   // chunk-local part
+      for (int u = lo + ((g - lo) & 7); u < hi; u += 8) term(u, acc);
+      if (Te > base + cnt) break;   // goes on in the next chunk
+      float x = 0.f;
+      if (n > 0) {
+        x = group_sum8(acc, g);
+#pragma unroll
+        for (int s = 0; s < NA; ++s) acc[s] = 0.f;
+      }
+      out[p * 64 + lane] = scale * x;
+      T = Te;
+      ++p;
+      if (++eb == nele) eb = ++ea;
+    }
+    __syncwarp();
   }
-  ja = kb = 0;
-  p = -1;
+  for (; p < nelep; ++p) out[p * 64 + lane] = 0.f;
 }
 
 template <int ZI, int RC>
@@ -183,27 +283,31 @@ sym_fwd_kernel(int N, const double* __restrict__ pos, const double* __restrict__
   __shared__ RowLdsFwd<RC> L;
   __shared__ float4 tq[SYM_WAVES][64];        // per triple: (cos theta, sin theta, fc_j fc_k, -)
   __shared__ float4 tR[SYM_WAVES][64][NA / 4];   // per triple: exp(-eta (ravg - Rs_s)^2), s = 0..7
-  __shared__ int segs[SYM_WAVES][2][TM_MAX_ELE + 1];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  __shared__ unsigned char apos[SYM_WAVES][RC];   // row position of each sub-list member
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int i = blockIdx.x * SYM_WAVES + w;
   if (i >= N) return;   // only wave-level synchronisation below
-  const int n = min(ncnt[i], RC);
-  if (lane <= a.nele) {
-    segs[w][0][lane] = min(rseg[(long)i * (a.nele + 1) + lane], n);
-    segs[w][1][lane] = aseg[(long)i * (a.nele + 1) + lane];
-  }
-  load_row(i, w, lane, pos, box, mol, nbr, n, ldr, a, L);
+  int jq[RC / 64];
+  row_slots<RC>(jq, nbr, i, lane, ldr);
+  const int n = min(ncnt[i], RC), m = min(acnt[i], lda);
+  // element segments of the row and of the sub-list, boundary e in lane e
+  const int le = min(lane, a.nele);
+  const int rv = min(rseg[(long)i * (a.nele + 1) + le], n);
+  const int av = min(aseg[(long)i * (a.nele + 1) + le], m);
+  for (int x = lane; x < m; x += 64) apos[w][x] = (unsigned char)ang[(long)i * lda + x];
+  load_row<RC>(i, w, lane, pos, box, mol, jq, n, a, L, [](int, int, const float4&) {});
   __syncwarp();
   float* Gi = G + (long)i * ldg;
   // ---------------- radial: lane = (half h, shell s)
   {
     const int h = lane >> 5, s = lane & 31;
     for (int e = 0; e < a.nele; ++e) {
-      int lo = segs[w][0][e], hi = segs[w][0][e + 1];
+      const int lo = seg_at(rv, e), hi = seg_at(rv, e + 1);
       for (int s0 = 0; s0 < a.nr; s0 += 32) {
         int ss = s0 + s;
         float rs = ss < a.nr ? a.rs_r[ss] : 0.f;
         float acc = 0.f;
+#pragma unroll 4
         for (int q = lo + h; q < hi; q += 2) {
           float r = L.d[w][q].w;
           float x = r - rs;
@@ -215,95 +319,45 @@ sym_fwd_kernel(int N, const double* __restrict__ pos, const double* __restrict__
     }
   }
   // ---------------- angular
-  // Phase A: lane = triple, stages its geometry in LDS.  Phase B: lane =
-  // (theta point t, triple group g); a lane takes every 8th triple of an
-  // element-pair segment, forms (1 + cos(theta - theta_t))^zeta fc_j fc_k once
-  // and adds it times R_s to one accumulator per shell s.  When a segment
-  // ends, a butterfly over g sums the 8 groups and lane (t, g) writes shell
-  // s = g.  Triples are ordered by element pair (blocks ea <= eb), so each
-  // segment is a contiguous range of the enumeration.
-  const int m = min(acnt[i], lda);
-  const int* arow = ang + (long)i * lda;
-  const int ntrip = m * (m - 1) / 2;
-  const int off = a.nele * a.nr;
-  const int ot = lane >> 3, g = lane & 7;
-  const float ct = a.cos_t[ot], st = a.sin_t[ot];
-  const int* sg = segs[w][1];
-  float acc[NA];
+  // Phase B forms (1 + cos(theta - theta_t))^zeta fc_j fc_k once per triple and
+  // theta point and adds it times R_s to the shells.
+  const float ct = a.cos_t[lane >> 3], st = a.sin_t[lane >> 3];
+  angular_pass(
+      lane, a.nele, a.nelep, av, m * (m - 1) / 2, a.two_1mz, Gi + a.nele * a.nr,
+      [&](int ja, int kb) {
+        const int qj = apos[w][ja], qk = apos[w][kb];
+        float4 dj = L.d[w][qj], dk = L.d[w][qk];
+        const float inv = __builtin_amdgcn_rcpf(dj.w * dk.w);
+        float c = (dj.x * dk.x + dj.y * dk.y + dj.z * dk.z) * inv;
+        c = fminf(fmaxf(c, -1.0f), 1.0f);
+        float sn = sin_between(dj, dk, inv);
+        float ravg = 0.5f * (dj.w + dk.w);
+        tq[w][lane] = make_float4(c, sn, cutoff_fc(a.ka, dj.w) * cutoff_fc(a.ka, dk.w), 0.f);
+        float R[NA];
 #pragma unroll
-  for (int s = 0; s < NA; ++s) acc[s] = 0.f;
-  int pdone = 0;   // segments [0, pdone) are written
-  auto flush = [&](int p) {
-    float v[NA];
-#pragma unroll
-    for (int s = 0; s < NA; ++s) {
-      float x = acc[s];
-      x += __shfl_xor(x, 1, 64);
-      x += __shfl_xor(x, 2, 64);
-      x += __shfl_xor(x, 4, 64);
-      v[s] = x;
-      acc[s] = 0.f;
-    }
-    float out = v[0];
-#pragma unroll
-    for (int s = 1; s < NA; ++s) out = g == s ? v[s] : out;
-    Gi[off + p * 64 + ot * NA + g] = a.two_1mz * out;
-  };
-  for (int base = 0; base < ntrip; base += 64) {
-    int t = base + lane;
-    if (t < ntrip) {
-      int ja, kb, p;
-      decode_triple(t, sg, a.nele, ja, kb, p);
-      int qj = arow[ja], qk = arow[kb];
-      float4 dj = L.d[w][qj], dk = L.d[w][qk];
-      const float inv = __builtin_amdgcn_rcpf(dj.w * dk.w);
-      float c = (dj.x * dk.x + dj.y * dk.y + dj.z * dk.z) * inv;
-      c = fminf(fmaxf(c, -1.0f), 1.0f);
-      float sn = sin_between(dj, dk, inv);
-      float ravg = 0.5f * (dj.w + dk.w);
-      tq[w][lane] = make_float4(c, sn, cutoff_fc(a.ka, dj.w) * cutoff_fc(a.ka, dk.w), 0.f);
-      float R[NA];
-#pragma unroll
-      for (int s = 0; s < NA; ++s) {
-        float x = ravg - a.rs_a[s];
-        R[s] = __expf(-a.eta * x * x);
-      }
-      tR[w][lane][0] = make_float4(R[0], R[1], R[2], R[3]);
-      tR[w][lane][1] = make_float4(R[4], R[5], R[6], R[7]);
-    }
-    __syncwarp();
-    const int cnt = min(64, ntrip - base);
-    int T = 0, p = 0;   // first triple of segment p
-    for (int ea = 0; ea < a.nele; ++ea) {
-      const int la = sg[ea + 1] - sg[ea];
-      for (int eb = ea; eb < a.nele; ++eb, ++p) {
-        const int lb = sg[eb + 1] - sg[eb];
-        const int Te = T + (ea == eb ? la * (la - 1) / 2 : la * lb);
-        const int lo = max(T - base, 0), hi = min(Te - base, cnt);   // chunk-local part
-        for (int u = lo + ((g - lo) & 7); u < hi; u += 8) {
-          const float4 q = tq[w][u];
-          const float4 r0 = tR[w][u][0], r1 = tR[w][u][1];
-          const float AF = powz<ZI>(1.0f + (q.x * ct + q.y * st), a) * q.z;
-          acc[0] += AF * r0.x; acc[1] += AF * r0.y; acc[2] += AF * r0.z; acc[3] += AF * r0.w;
-          acc[4] += AF * r1.x; acc[5] += AF * r1.y; acc[6] += AF * r1.z; acc[7] += AF * r1.w;
+        for (int s = 0; s < NA; ++s) {
+          float x = ravg - a.rs_a[s];
+          R[s] = __expf(-a.eta * x * x);
         }
-        if (p >= pdone && Te <= base + cnt) {   // segment complete (wave-uniform)
-          flush(p);
-          pdone = p + 1;
-        }
-        T = Te;
-      }
-    }
-    __syncwarp();
-  }
-  for (int p = pdone; p < a.nelep; ++p) Gi[off + p * 64 + lane] = 0.f;
+        tR[w][lane][0] = make_float4(R[0], R[1], R[2], R[3]);
+        tR[w][lane][1] = make_float4(R[4], R[5], R[6], R[7]);
+      },
+      [&](int u, float (&acc)[NA]) {
+        const float4 q = tq[w][u];
+        const float4 r0 = tR[w][u][0], r1 = tR[w][u][1];
+        const float AF = powz<ZI>(1.0f + (q.x * ct + q.y * st), a) * q.z;
+        acc[0] += AF * r0.x; acc[1] += AF * r0.y; acc[2] += AF * r0.z; acc[3] += AF * r0.w;
+        acc[4] += AF * r1.x; acc[5] += AF * r1.y; acc[6] += AF * r1.z; acc[7] += AF * r1.w;
+      });
   if (rev == nullptr) return;
   // Mirror slots (the rev output of the neighbour build): rev[i*ldr+q] =
   // j*ldr + position of i in row j, found by binary search in the element
   // segment of row j that holds i (rows are sorted by (element, index)).
   const int ei = elem[i];
-  for (int q = lane; q < n; q += 64) {
-    const int j = nbr[(long)i * ldr + q];
+#pragma unroll
+  for (int k = 0; k < RC / 64; ++k) {
+    const int q = lane + 64 * k, j = jq[k];
+    if (q >= n) break;
     int lo = rseg[(long)j * (a.nele + 1) + ei];
     int hi = rseg[(long)j * (a.nele + 1) + ei + 1];
     const int* row = nbr + (long)j * ldr;
@@ -357,12 +411,14 @@ sym_adj_kernel(int N, const double* __restrict__ pos, const double* __restrict__
   static_assert(3 * RC <= 6 * ADJ_TC, "the members' sums reuse the window");
   __shared__ int mem[SYM_WAVES][RC];   // member: position in the row | element << 16
   extern __shared__ float4 gdyn[];     // dE/dG of each wave's centre, D rounded up to 4 floats
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int i = blockIdx.x * SYM_WAVES + w;
   if (i >= N) return;   // only wave-level synchronisation below
   // the radial part as it is, the angular part from a 16-byte boundary
   const int off = a.nele * a.nr, offa = (off + 3) & ~3, D4 = (a.D + offa - off + 3) >> 2;
   float* gw = reinterpret_cast<float*>(gdyn + w * D4);
+  int jq[NQ];
+  row_slots<RC>(jq, nbr, i, lane, ldr);
   const int n = min(ncnt[i], RC), m = min(min(acnt[i], lda), RC);
   // charge upstream u_i = phi_i - mean_m(phi) (as tm_charge_upstream) unless given
   const float ui = gQ == nullptr ? 0.f
@@ -382,7 +438,7 @@ sym_adj_kernel(int N, const double* __restrict__ pos, const double* __restrict__
         }
       }
     }
-    load_row(i, w, lane, pos, box, mol, nbr, n, ldr, a, L);
+    load_row<RC>(i, w, lane, pos, box, mol, jq, n, a, L, [](int, int, const float4&) {});
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const int f = 4 * (lane + 64 * k);
@@ -394,7 +450,7 @@ sym_adj_kernel(int N, const double* __restrict__ pos, const double* __restrict__
       if (gQ != nullptr) v += ui * gQi[f];
       gw[f < off ? f : f + offa - off] = v;
     }
-    load_row(i, w, lane, pos, box, mol, nbr, n, ldr, a, L);
+    load_row<RC>(i, w, lane, pos, box, mol, jq, n, a, L, [](int, int, const float4&) {});
   }
   for (int x = lane; x < m; x += 64) {
     const int q = ang[(long)i * lda + x];
@@ -662,40 +718,37 @@ sym_jvp_kernel(int N, const double* __restrict__ pos, const double* __restrict__
   // d cos theta, d ravg, ravg), R_s for s = 0..7
   __shared__ float4 tqa[SYM_WAVES][64], tqb[SYM_WAVES][64];
   __shared__ float4 tR[SYM_WAVES][64][NA / 4];
-  __shared__ int segs[SYM_WAVES][2][TM_MAX_ELE + 1];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  __shared__ unsigned char apos[SYM_WAVES][RC];   // row position of each sub-list member
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int i = blockIdx.x * SYM_WAVES + w;
   if (i >= N) return;   // only wave-level synchronisation below
-  const int n = min(ncnt[i], RC);
-  if (lane <= a.nele) {
-    segs[w][0][lane] = min(rseg[(long)i * (a.nele + 1) + lane], n);
-    segs[w][1][lane] = aseg[(long)i * (a.nele + 1) + lane];
-  }
-  load_row(i, w, lane, pos, box, mol, nbr, n, ldr, a, L);
+  int jq[RC / 64];
+  row_slots<RC>(jq, nbr, i, lane, ldr);
+  const int n = min(ncnt[i], RC), m = min(acnt[i], lda);
+  const int le = min(lane, a.nele);
+  const int rv = min(rseg[(long)i * (a.nele + 1) + le], n);
+  const int av = min(aseg[(long)i * (a.nele + 1) + le], m);
+  for (int x = lane; x < m; x += 64) apos[w][x] = (unsigned char)ang[(long)i * lda + x];
   const float kr = a.kr, ka = a.ka;
-  {
-    const double uxi = du[3 * i], uyi = du[3 * i + 1], uzi = du[3 * i + 2];
-    __syncwarp();
-    for (int q = lane; q < n; q += 64) {
-      const int j = nbr[(long)i * ldr + q];
-      const float tx = (float)(du[3 * j] - uxi), ty = (float)(du[3 * j + 1] - uyi);
-      const float tz = (float)(du[3 * j + 2] - uzi);
-      const float4 d = L.d[w][q];
-      T.t[w][q] = make_float4(tx, ty, tz, (d.x * tx + d.y * ty + d.z * tz) * __builtin_amdgcn_rcpf(d.w));
-      T.dfc[w][q] = -0.5f * kr * __sinf(kr * d.w);
-    }
-  }
+  const double uxi = du[3 * i], uyi = du[3 * i + 1], uzi = du[3 * i + 2];
+  load_row<RC>(i, w, lane, pos, box, mol, jq, n, a, L, [&](int q, int j, const float4& d) {
+    const float tx = (float)(du[3 * j] - uxi), ty = (float)(du[3 * j + 1] - uyi);
+    const float tz = (float)(du[3 * j + 2] - uzi);
+    T.t[w][q] = make_float4(tx, ty, tz, (d.x * tx + d.y * ty + d.z * tz) * __builtin_amdgcn_rcpf(d.w));
+    T.dfc[w][q] = -0.5f * kr * __sinf(kr * d.w);
+  });
   __syncwarp();
   float* Vi = V + (long)i * ldg;
   // ---------------- radial: lane = (half h, shell s)
   {
     const int h = lane >> 5, s = lane & 31;
     for (int e = 0; e < a.nele; ++e) {
-      int lo = segs[w][0][e], hi = segs[w][0][e + 1];
+      const int lo = seg_at(rv, e), hi = seg_at(rv, e + 1);
       for (int s0 = 0; s0 < a.nr; s0 += 32) {
         int ss = s0 + s;
         float rs = ss < a.nr ? a.rs_r[ss] : 0.f;
         float acc = 0.f;
+#pragma unroll 4
         for (int q = lo + h; q < hi; q += 2) {
           float r = L.d[w][q].w;
           float x = r - rs;
@@ -708,104 +761,54 @@ sym_jvp_kernel(int N, const double* __restrict__ pos, const double* __restrict__
     }
   }
   // ---------------- angular
-  // The forward's layout (sym_fwd_kernel): phase A lane = triple stages the
-  // triple's geometry and its tangents in LDS; phase B lane = (theta point t,
-  // triple group g) takes every 8th triple of an element-pair segment, forms
-  // (1 + cos(theta - theta_t))^zeta and its derivative once, and adds
+  // Phase B forms (1 + cos(theta - theta_t))^zeta and its derivative once per
+  // triple and theta point, and adds
   //   X R_s + Y R'_s,  X = A' v' c' F + A F',  Y = A r' F
-  // to one accumulator per shell s (A = (1 + v)^zeta, v = cos(theta - theta_t),
-  // c', r', F' the tangents of cos theta, ravg and fc_j fc_k); a butterfly
-  // over g at each segment end, lane (t, g) writes shell s = g.
-  const int m = min(acnt[i], lda);
-  const int* arow = ang + (long)i * lda;
-  const int ntrip = m * (m - 1) / 2;
-  const int off = a.nele * a.nr;
-  const int ot = lane >> 3, g = lane & 7;
-  const float ct = a.cos_t[ot], st = a.sin_t[ot];
-  const int* sg = segs[w][1];
-  float acc[NA];
+  // to the shells (A = (1 + v)^zeta, v = cos(theta - theta_t), c', r', F' the
+  // tangents of cos theta, ravg and fc_j fc_k).
+  const float ct = a.cos_t[lane >> 3], st = a.sin_t[lane >> 3];
+  angular_pass(
+      lane, a.nele, a.nelep, av, m * (m - 1) / 2, a.two_1mz, Vi + a.nele * a.nr,
+      [&](int ja, int kb) {
+        const int qj = apos[w][ja], qk = apos[w][kb];
+        float4 dj = L.d[w][qj], dk = L.d[w][qk];
+        float4 uj = T.t[w][qj], uk = T.t[w][qk];
+        float rj = dj.w, rk = dk.w;
+        const float irj = __builtin_amdgcn_rcpf(rj), irk = __builtin_amdgcn_rcpf(rk);
+        float inv = irj * irk;
+        float c = (dj.x * dk.x + dj.y * dk.y + dj.z * dk.z) * inv;
+        c = fminf(fmaxf(c, -1.0f), 1.0f);
+        float sn = sin_between(dj, dk, inv);
+        float dc = (uj.x * dk.x + uj.y * dk.y + uj.z * dk.z + dj.x * uk.x + dj.y * uk.y +
+                    dj.z * uk.z) * inv - c * (uj.w * irj + uk.w * irk);
+        const float fj = cutoff_fc(ka, rj), fk = cutoff_fc(ka, rk);
+        const float dfj = cutoff_dfc(ka, rj), dfk = cutoff_dfc(ka, rk);
+        float ravg = 0.5f * (rj + rk);
+        tqa[w][lane] = make_float4(c, sn, sn > 1e-6f ? c * __builtin_amdgcn_rcpf(sn) : 0.f,
+                                   fj * fk);
+        tqb[w][lane] = make_float4(dfj * uj.w * fk + fj * dfk * uk.w, dc, 0.5f * (uj.w + uk.w),
+                                   ravg);
+        float R[NA];
 #pragma unroll
-  for (int s = 0; s < NA; ++s) acc[s] = 0.f;
-  int pdone = 0;   // segments [0, pdone) are written
-  auto flush = [&](int p) {
-    float v[NA];
-#pragma unroll
-    for (int s = 0; s < NA; ++s) {
-      float x = acc[s];
-      x += __shfl_xor(x, 1, 64);
-      x += __shfl_xor(x, 2, 64);
-      x += __shfl_xor(x, 4, 64);
-      v[s] = x;
-      acc[s] = 0.f;
-    }
-    float out = v[0];
-#pragma unroll
-    for (int s = 1; s < NA; ++s) out = g == s ? v[s] : out;
-    Vi[off + p * 64 + ot * NA + g] = a.two_1mz * out;
-  };
-  for (int base = 0; base < ntrip; base += 64) {
-    int t = base + lane;
-    if (t < ntrip) {
-      int ja, kb, p;
-      decode_triple(t, sg, a.nele, ja, kb, p);
-      int qj = arow[ja], qk = arow[kb];
-      float4 dj = L.d[w][qj], dk = L.d[w][qk];
-      float4 uj = T.t[w][qj], uk = T.t[w][qk];
-      float rj = dj.w, rk = dk.w;
-      const float irj = __builtin_amdgcn_rcpf(rj), irk = __builtin_amdgcn_rcpf(rk);
-      float inv = irj * irk;
-      float c = (dj.x * dk.x + dj.y * dk.y + dj.z * dk.z) * inv;
-      c = fminf(fmaxf(c, -1.0f), 1.0f);
-      float sn = sin_between(dj, dk, inv);
-      float dc = (uj.x * dk.x + uj.y * dk.y + uj.z * dk.z + dj.x * uk.x + dj.y * uk.y +
-                  dj.z * uk.z) * inv - c * (uj.w * irj + uk.w * irk);
-      const float fj = cutoff_fc(ka, rj), fk = cutoff_fc(ka, rk);
-      const float dfj = cutoff_dfc(ka, rj), dfk = cutoff_dfc(ka, rk);
-      float ravg = 0.5f * (rj + rk);
-      tqa[w][lane] = make_float4(c, sn, sn > 1e-6f ? c * __builtin_amdgcn_rcpf(sn) : 0.f,
-                                 fj * fk);
-      tqb[w][lane] = make_float4(dfj * uj.w * fk + fj * dfk * uk.w, dc, 0.5f * (uj.w + uk.w),
-                                 ravg);
-      float R[NA];
-#pragma unroll
-      for (int s = 0; s < NA; ++s) {
-        float x = ravg - a.rs_a[s];
-        R[s] = __expf(-a.eta * x * x);
-      }
-      tR[w][lane][0] = make_float4(R[0], R[1], R[2], R[3]);
-      tR[w][lane][1] = make_float4(R[4], R[5], R[6], R[7]);
-    }
-    __syncwarp();
-    const int cnt = min(64, ntrip - base);
-    int T0 = 0, p = 0;   // first triple of segment p
-    for (int ea = 0; ea < a.nele; ++ea) {
-      const int la = sg[ea + 1] - sg[ea];
-      for (int eb = ea; eb < a.nele; ++eb, ++p) {
-        const int lb = sg[eb + 1] - sg[eb];
-        const int Te = T0 + (ea == eb ? la * (la - 1) / 2 : la * lb);
-        const int lo = max(T0 - base, 0), hi = min(Te - base, cnt);   // chunk-local part
-        for (int u = lo + ((g - lo) & 7); u < hi; u += 8) {
-          const float4 qa = tqa[w][u], qb = tqb[w][u];
-          float Az, dAz;
-          powz_pair<ZI>(1.0f + (qa.x * ct + qa.y * st), a, Az, dAz);
-          const float dv = ct - qa.z * st;
-          const float X = dAz * dv * qb.y * qa.w + Az * qb.x;
-          const float Y2 = -2.0f * a.eta * Az * qb.z * qa.w;   // times (ravg - R_s) R_s
-          const float4 r0 = tR[w][u][0], r1 = tR[w][u][1];
-          const float R[NA] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
-#pragma unroll
-          for (int s = 0; s < NA; ++s) acc[s] += R[s] * (X + Y2 * (qb.w - a.rs_a[s]));
+        for (int s = 0; s < NA; ++s) {
+          float x = ravg - a.rs_a[s];
+          R[s] = __expf(-a.eta * x * x);
         }
-        if (p >= pdone && Te <= base + cnt) {   // segment complete (wave-uniform)
-          flush(p);
-          pdone = p + 1;
-        }
-        T0 = Te;
-      }
-    }
-    __syncwarp();
-  }
-  for (int p = pdone; p < a.nelep; ++p) Vi[off + p * 64 + lane] = 0.f;
+        tR[w][lane][0] = make_float4(R[0], R[1], R[2], R[3]);
+        tR[w][lane][1] = make_float4(R[4], R[5], R[6], R[7]);
+      },
+      [&](int u, float (&acc)[NA]) {
+        const float4 qa = tqa[w][u], qb = tqb[w][u];
+        float Az, dAz;
+        powz_pair<ZI>(1.0f + (qa.x * ct + qa.y * st), a, Az, dAz);
+        const float dv = ct - qa.z * st;
+        const float X = dAz * dv * qb.y * qa.w + Az * qb.x;
+        const float Y2 = -2.0f * a.eta * Az * qb.z * qa.w;   // times (ravg - R_s) R_s
+        const float4 r0 = tR[w][u][0], r1 = tR[w][u][1];
+        const float R[NA] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
+#pragma unroll
+        for (int s = 0; s < NA; ++s) acc[s] += R[s] * (X + Y2 * (qb.w - a.rs_a[s]));
+      });
 }
 
 int fill_args(SymArgs& a, int nele, int nr, float eta, float zeta, float rr, float ra,
