@@ -338,6 +338,16 @@ int tm_coulomb(int N, const float* xq, const int* elem, const int* mol, const in
                int add_ecc, int has_vdw, int nele, const double* c6, const double* r0, float* xqc,
                int* elc, double* phi, double* grad, double* eatom, int* flags, void* stream);
 
+/* tm_charges with means and tm_coulomb without a cell grid in one launch, from
+ * raw charges and positions.  Same outputs as the two calls, up to the order of
+ * the float64 sum of a molecule's raw charges; qmean of a molecule without
+ * atoms is 0. */
+int tm_coulomb_raw(int N, int B, const float* qraw, const double* pos, const int* elem,
+                   const int* mol, const int* mol_start, const double* box, int periodic,
+                   const double* consts, double rc_ee, double width, int add_ecc, int has_vdw,
+                   int nele, const double* c6, const double* r0, double* qmean, float* xq, double* q,
+                   double* qx, double* phi, double* grad, double* eatom, int* flags, void* stream);
+
 /* Tables of the pair functions tm_coulomb_tab reads (host only, no device
  * work): nint intervals of width h = rc_ee / (nint - 1) (A), interval k
  * spanning [k h - off, (k + 1) h - off] with off in [0, h) chosen so that a

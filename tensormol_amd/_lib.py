@@ -41,6 +41,7 @@ SIGNATURES = {
     "tm_charge_upstream": [I, P, P, P, P, P],
     "tm_coulomb": [I, P, P, P, P, P, P, P, P, P, P, I, I, I, D, D, D, D, D, D, I, P, D, D, I, I, I, P, P, P, P,
                    P, P, P, P, P],
+    "tm_coulomb_raw": [I, I, P, P, P, P, P, P, I, P, D, D, I, I, I, P, P, P, P, P, P, P, P, P, P, P],
     "tm_coulomb_table": [P, D, D, I, I, I, P, P, I, P, P],
     "tm_coulomb_tab": [I, P, P, P, P, I, I, I, D, D, D, D, D, D, I, D, I, P, I, D, D, P, P, P, P,
                            P, P, P],

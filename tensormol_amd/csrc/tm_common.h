@@ -73,8 +73,41 @@ __device__ __forceinline__ float tm_wave_sum(float v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
 }
+// Sum over the wave, in every lane, in the order of a butterfly over lane ^ 32,
+// ^ 16, ^ 8, ^ 4, ^ 2, ^ 1, without a trip through LDS.  The halves and the rows
+// of 16 lanes are exchanged by swaps; after that lanes that differ by 16 or 32
+// hold the same sum, after the step of 8 also lanes that differ by 8, and so on,
+// so a rotation of the row by 8, 4, 2, 1 reads what lane ^ 8, 4, 2, 1 holds.
+struct tm_d2 {
+  double a, b;
+};
+template <int ROWS>
+__device__ __forceinline__ tm_d2 tm_swap_d(double v) {
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  const u2 x = __builtin_bit_cast(u2, v);
+  auto swap = [](unsigned u) {
+    if constexpr (ROWS == 32) return __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    else return __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  };
+  const auto lo = swap(x.x), hi = swap(x.y);
+  return {__builtin_bit_cast(double, u2{(unsigned)lo[0], (unsigned)hi[0]}),
+          __builtin_bit_cast(double, u2{(unsigned)lo[1], (unsigned)hi[1]})};
+}
+template <int N>
+__device__ __forceinline__ double tm_row_ror_d(double v) {
+  typedef int i2 __attribute__((ext_vector_type(2)));
+  const i2 x = __builtin_bit_cast(i2, v);
+  return __builtin_bit_cast(double, i2{__builtin_amdgcn_update_dpp(0, x.x, 0x120 + N, 0xf, 0xf, true),
+                                       __builtin_amdgcn_update_dpp(0, x.y, 0x120 + N, 0xf, 0xf, true)});
+}
 __device__ __forceinline__ double tm_wave_sum_d(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  const tm_d2 h = tm_swap_d<32>(v);
+  v = h.a + h.b;
+  const tm_d2 r = tm_swap_d<16>(v);
+  v = r.a + r.b;
+  v += tm_row_ror_d<8>(v);
+  v += tm_row_ror_d<4>(v);
+  v += tm_row_ror_d<2>(v);
+  v += tm_row_ror_d<1>(v);
   return v;
 }

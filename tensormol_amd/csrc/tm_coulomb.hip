@@ -18,6 +18,7 @@
 // Neighbors.py:262-282), evaluated on the fly from the cell grid; no pair
 // list is stored.  One wavefront per centre gathers its own terms, so every
 // per-atom sum is formed in a fixed order (no atomics) and accumulated in FP64.
+#include <algorithm>
 #include <mutex>
 
 #include "tm_cells.h"
@@ -130,13 +131,28 @@ constexpr int QCAP = 128;   // compacted pair queue per wave
 // fixed order.
 // MOLC: the cell-ordered candidates carry molecule ids (several systems share
 // the grid); a template parameter so the candidate loads are branch-free.
-template <bool MOLC>
+// RAW: molecule sweeps straight from raw charges and positions.  Every wave
+// sums its molecule's raw charges itself, in one order, and forms the neutral
+// charges of its candidates as it loads them; the wave of an atom writes the
+// atom's charge and dipole terms.  That saves the launches that would form the
+// means and the charges first: 160 molecules of 8 to 256 atoms 23.4 -> TIME us.
+struct RawCharges {
+  const float* qraw;
+  const double* pos;
+  double* qmean;
+  double* q;
+  double* qx;
+  float4* xq;
+  int B;
+};
+template <bool MOLC, bool RAW>
 __global__ void __launch_bounds__(C_WAVES * 64)
 coulomb_kernel(int N, const float4* __restrict__ xq, const int* __restrict__ elem,
                const float4* __restrict__ xqc, const int* __restrict__ elc,
                const int* __restrict__ mol, const int* __restrict__ mol_start,
                const double* __restrict__ box, CellGrid grid, CoulArgs a, double* __restrict__ phi,
-               double* __restrict__ grad, double* __restrict__ eatom, int* __restrict__ flags) {
+               double* __restrict__ grad, double* __restrict__ eatom, int* __restrict__ flags,
+               RawCharges raw) {
   __shared__ float4 qx[C_WAVES][QCAP];
   __shared__ int qe[C_WAVES][QCAP];
   __shared__ RangeLds<C_RANGES> rng[C_WAVES];
@@ -149,8 +165,9 @@ coulomb_kernel(int N, const float4* __restrict__ xq, const int* __restrict__ ele
     vdw_q[threadIdx.x] = 6.0f * q6 * q6;
   }
   __syncthreads();
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int wi = blockIdx.x * C_WAVES + w;
+  if (RAW && lane == 0 && wi < raw.B && mol_start[wi] == mol_start[wi + 1]) raw.qmean[wi] = 0.0;
   if (wi >= N) return;   // wave-level synchronisation only below
   // centres are visited in cell order so neighbouring waves share candidates in L2
   const int i = grid.cell_atoms != nullptr ? grid.cell_atoms[wi] : wi;
@@ -161,7 +178,28 @@ coulomb_kernel(int N, const float4* __restrict__ xq, const int* __restrict__ ele
     Lx = (float)box[3 * mi]; Ly = (float)box[3 * mi + 1]; Lz = (float)box[3 * mi + 2];
     iLx = 1.0f / Lx; iLy = 1.0f / Ly; iLz = 1.0f / Lz;
   }
-  const float4 pi = cpi >= 0 ? xqc[cpi] : xq[i];
+  float4 pi;
+  double mean = 0.0;
+  if constexpr (RAW) {
+    const int lo = mol_start[mi], hi = mol_start[mi + 1];
+    const double x = raw.pos[3 * (long)i], y = raw.pos[3 * (long)i + 1], z = raw.pos[3 * (long)i + 2];
+    const double qr = (double)raw.qraw[i];
+    double v = 0.0;
+    for (int b = lo + lane; b < hi; b += 64) v += (double)raw.qraw[b];
+    mean = tm_wave_sum_d(v) / (double)(hi - lo);
+    const double qi = qr - mean;
+    pi = make_float4((float)x, (float)y, (float)z, (float)qi);
+    if (lane == 0) {
+      raw.q[i] = qi;
+      raw.xq[i] = pi;
+      raw.qx[3 * (long)i] = qi * x * BOHRPERA_D;
+      raw.qx[3 * (long)i + 1] = qi * y * BOHRPERA_D;
+      raw.qx[3 * (long)i + 2] = qi * z * BOHRPERA_D;
+      if (i == lo) raw.qmean[mi] = mean;
+    }
+  } else {
+    pi = cpi >= 0 ? xqc[cpi] : xq[i];
+  }
   const int ei = cpi >= 0 ? elc[cpi] : elem[i];
   const float* vci = vdw_c + ei * TM_MAX_ELE;
   const float* vqi = vdw_q + ei * TM_MAX_ELE;
@@ -185,6 +223,14 @@ coulomb_kernel(int N, const float4* __restrict__ xq, const int* __restrict__ ele
   auto load = [&](int p, bool valid, int mapped) {
     const int q = valid ? p : 0;
     Cand c;
+    if constexpr (RAW) {
+      const double* p3 = raw.pos + 3 * (long)q;
+      c.x = make_float4((float)p3[0], (float)p3[1], (float)p3[2],
+                        (float)((double)raw.qraw[q] - mean));
+      c.e = elem[q];
+      c.m = mi;
+      return c;
+    }
     c.x = mapped ? xqc[q] : xq[q];
     c.e = mapped ? elc[q] : elem[q];
     c.m = (MOLC && mapped) ? grid.molc[q] : mi;
@@ -589,6 +635,24 @@ int tm_mol_sum_f64(int B, const int* mol_start, int C, const double* in, int ldi
 
 namespace {
 
+CoulArgs coul_args(const double* consts, double rc_ee, double width, int add_ecc, int has_vdw,
+                   int nele, const double* c6, const double* r0) {
+  CoulArgs a;
+  a.alpha = (float)consts[0]; a.r_sr = (float)consts[1]; a.r_lr = (float)consts[2];
+  a.zz = (float)consts[3]; a.yy = (float)consts[4]; a.shift = (float)consts[5];
+  a.ea = (float)consts[6];
+  a.lin = (float)(consts[3] / consts[2] + consts[4]);
+  a.rc2 = (float)(rc_ee * rc_ee);
+  a.inv_width = (float)(1.0 / width);
+  a.add_ecc = add_ecc;
+  a.has_vdw = has_vdw;
+  for (int e = 0; e < TM_MAX_ELE; ++e) {
+    a.c6[e] = e < nele ? (float)c6[e] : 0.f;
+    a.r0[e] = e < nele ? (float)r0[e] : 0.f;
+  }
+  return a;
+}
+
 // The per-molecule sums of tm_mol_sums; `work` (may be null) is the block
 // partials and completion counter of the many-block path for one system.
 int mol_sums_impl(const char* name, int B, const int* mol_start, int n_total, int nsrc,
@@ -737,19 +801,7 @@ int tm_coulomb(int N, const float* xq, const int* elem, const int* mol, const in
                tm_range_bound(rc_ee, cs, nc, periodic), C_RANGES);
   }
   if (N == 0) return TM_OK;
-  CoulArgs a;
-  a.alpha = (float)consts[0]; a.r_sr = (float)consts[1]; a.r_lr = (float)consts[2];
-  a.zz = (float)consts[3]; a.yy = (float)consts[4]; a.shift = (float)consts[5];
-  a.ea = (float)consts[6];
-  a.lin = (float)(consts[3] / consts[2] + consts[4]);
-  a.rc2 = (float)(rc_ee * rc_ee);
-  a.inv_width = (float)(1.0 / width);
-  a.add_ecc = add_ecc;
-  a.has_vdw = has_vdw;
-  for (int e = 0; e < TM_MAX_ELE; ++e) {
-    a.c6[e] = e < nele ? (float)c6[e] : 0.f;
-    a.r0[e] = e < nele ? (float)r0[e] : 0.f;
-  }
+  const CoulArgs a = coul_args(consts, rc_ee, width, add_ecc, has_vdw, nele, c6, r0);
   CellGrid g;
   g.cell_start = cell_start; g.cell_atoms = cell_atoms; g.cell_of = cell_of;
   g.cell_pos = cell_pos; g.posc = nullptr; g.molc = molc;
@@ -764,11 +816,30 @@ int tm_coulomb(int N, const float* xq, const int* elem, const int* mol, const in
                                                          (float4*)xqc, elc);
     TM_LAUNCH_CHECK();
   }
-  auto k = (cell_atoms != nullptr && molc != nullptr) ? coulomb_kernel<true>
-                                                      : coulomb_kernel<false>;
+  auto k = (cell_atoms != nullptr && molc != nullptr) ? coulomb_kernel<true, false>
+                                                      : coulomb_kernel<false, false>;
   k<<<tm_div_up(N, C_WAVES), C_WAVES * 64, 0, s>>>(N, (const float4*)xq, elem,
                                                    (const float4*)xqc, elc, mol, mol_start, box, g,
-                                                   a, phi, grad, eatom, flags);
+                                                   a, phi, grad, eatom, flags, RawCharges{});
+  TM_LAUNCH_CHECK();
+  return TM_OK;
+}
+
+int tm_coulomb_raw(int N, int B, const float* qraw, const double* pos, const int* elem,
+                   const int* mol, const int* mol_start, const double* box, int periodic,
+                   const double* consts, double rc_ee, double width, int add_ecc, int has_vdw,
+                   int nele, const double* c6, const double* r0, double* qmean, float* xq, double* q,
+                   double* qx, double* phi, double* grad, double* eatom, int* flags, void* stream) {
+  TM_REQUIRE(N >= 0 && B >= 0, "tm_coulomb_raw: negative size");
+  TM_REQUIRE(nele > 0 && nele <= TM_MAX_ELE, "tm_coulomb_raw: bad nele");
+  const int waves = std::max(N, B);
+  if (waves == 0) return TM_OK;
+  const CoulArgs a = coul_args(consts, rc_ee, width, add_ecc, has_vdw, nele, c6, r0);
+  CellGrid g{};
+  g.periodic = periodic;
+  coulomb_kernel<false, true><<<tm_div_up(waves, C_WAVES), C_WAVES * 64, 0, (hipStream_t)stream>>>(
+      N, nullptr, elem, nullptr, nullptr, mol, mol_start, box, g, a, phi, grad, eatom, flags,
+      RawCharges{qraw, pos, qmean, q, qx, (float4*)xq, B});
   TM_LAUNCH_CHECK();
   return TM_OK;
 }

@@ -418,25 +418,31 @@ class BPEEEngine:
         (to record timing events on the launch stream)."""
         key = (pos.data_ptr(), self._raw_stream())
         st = self._stream
-        # One system: the mean of the raw charges is formed inside the charges
-        # launch (each block sums it).  A batch of many small molecules takes
-        # one block per molecule in a reduction launch first instead, since a
-        # block would otherwise step through every molecule it touches.
-        ms = None
-        if ws.B == 1:
-            ms = ws.mol_start
-        else:
-            self._call(ws, "tm_mol_sum_f32", key, lambda: (
-                ws.B, _P(ws.mol_start), 1, _P(ws.qraw), 1, _P(ws.qmean), 1, _P(ws.red), ws.N, st()))
-        if ws.use_cells:   # charges written straight into cell order for the sweep
-            self._call(ws, "tm_charges", key, lambda: (
-                ws.N, _P(ws.mol), _P(ms), _P(ws.qmean), _P(ws.qraw), _P(pos), None, _P(ws.q),
-                _P(ws.qx), _P(ws.cell_pos), _P(ws.elem), _P(ws.xqc), _P(ws.elc), st()))
-        else:
-            self._call(ws, "tm_charges", key, lambda: (
-                ws.N, _P(ws.mol), _P(ms), _P(ws.qmean), _P(ws.qraw), _P(pos), _P(ws.xq), _P(ws.q),
-                _P(ws.qx), None, None, None, None, st()))
-        table = self._cl_table() if (ws.use_cells and self.coulomb_tables) else None
+        if not ws.use_cells:
+            # molecules: charges and sweep in one launch
+            add_ecc = int(bool(PARAMS["AddEcc"]))
+            if timer is not None:
+                timer[0]()
+            self._call(ws, "tm_coulomb_raw", key + (add_ecc,), lambda: (
+                ws.N, ws.B, _P(ws.qraw), _P(pos), _P(ws.elem), _P(ws.mol), _P(ws.mol_start),
+                _P(ws.box), ws.periodic, self.dsf.ctypes.data_as(_lib.P), self.model.ee_off,
+                self.vdw_width, add_ecc, int(self.model.has_vdw), self.nele,
+                self.c6.ctypes.data_as(_lib.P), self.r0.ctypes.data_as(_lib.P), _P(ws.qmean),
+                _P(ws.xq), _P(ws.q), _P(ws.qx), _P(ws.phi), _P(ws.gradc), _P(ws.eatom),
+                _P(ws.flags), st()))
+            if timer is not None:
+                timer[1]()
+            self._call(ws, "tm_mol_sum_f64", key, lambda: (
+                ws.B, _P(ws.mol_start), 1, _P(ws.phi), 1, _P(ws.phimean), 1, _P(ws.red), ws.N,
+                st()))
+            return
+        # One system (a cell grid is only set up for one): the mean of the raw
+        # charges is formed inside the charges launch (each block sums it), and
+        # charges are written straight into cell order for the sweep.
+        self._call(ws, "tm_charges", key, lambda: (
+            ws.N, _P(ws.mol), _P(ws.mol_start), _P(ws.qmean), _P(ws.qraw), _P(pos), None, _P(ws.q),
+            _P(ws.qx), _P(ws.cell_pos), _P(ws.elem), _P(ws.xqc), _P(ws.elc), st()))
+        table = self._cl_table() if self.coulomb_tables else None
         if timer is not None:
             timer[0]()
         if table is not None:
@@ -452,7 +458,7 @@ class BPEEEngine:
 
             def coul_args():
                 g = self._grid_args(ws)
-                return (ws.N, None if ws.use_cells else _P(ws.xq), _P(ws.elem), _P(ws.mol),
+                return (ws.N, None, _P(ws.elem), _P(ws.mol),
                         _P(ws.mol_start), _P(ws.box), g[0], g[1], g[2], g[3], g[5], g[6], g[7],
                         g[8], g[9], g[10], g[11], g[12], g[13], g[14], ws.periodic,
                         self.dsf.ctypes.data_as(_lib.P), self.model.ee_off, self.vdw_width,
