@@ -267,6 +267,15 @@ int tm_fm_loss(int B, const int* mol_start, const float* eps, const double* E_re
 int tm_force_gather(int N, int ldr, const int* ncnt, const int* rev, const float* wslot,
                     const double* extra, double scale, double* grad, double* force,
                     void* stream);
+/* tm_force_gather and tm_mol_sums (of all N atoms; scratch needed for one system
+ * of more than 2048 atoms) in one launch, bit-identical to the two calls. */
+int tm_force_gather_sums(int N, int ldr, const int* ncnt, const int* rev, const float* wslot,
+                         const double* extra, double scale, double* grad, double* force, int B,
+                         const int* mol_start, int nsrc, const void* const* in, const int* f64,
+                         const int* cols, const int* ld, double* const* out, double* scratch,
+                         void* stream);
+/* Per-molecule total energy out[m] = bp[m] + ext[2m] + ext[2m+1]. */
+int tm_total_energy(int B, const double* bp, const double* ext, double* out, void* stream);
 /* tm_force_gather followed by tm_vv_kick_drift with the gathered force (scale
  * = JOULEPERHARTREE gives the force tm_vv_kick takes), in one launch and
  * bit-identical to the two calls: one MD step of VelocityVerletStep

@@ -22,6 +22,7 @@
 #include <mutex>
 
 #include "tm_cells.h"
+#include "tm_sums.h"
 
 namespace {
 
@@ -412,104 +413,17 @@ sum_last_block_kernel(int n, int C, const T* __restrict__ in, int ldin, double* 
     __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Several per-molecule column sums in one launch.  Source k is an [N, ld[k]]
-// array (float64 when f64[k], else float32) of which the first cols[k]
-// columns are summed; columns are numbered across sources in order.
-constexpr int SUMS_MAX_SRC = 4, SUMS_MAX_COL = 16;
-struct SumSrc {
-  const void* in[SUMS_MAX_SRC];
-  double* out[SUMS_MAX_SRC];
-  int f64[SUMS_MAX_SRC], cols[SUMS_MAX_SRC], ld[SUMS_MAX_SRC];
-  int nsrc, ctot;
-};
-
-__device__ __forceinline__ double src_val(const SumSrc& S, int k, long a, int c) {
-  return S.f64[k] ? ((const double*)S.in[k])[a * S.ld[k] + c]
-                  : (double)((const float*)S.in[k])[a * S.ld[k] + c];
+// Several per-molecule column sums in one launch (tm_sums.h).
+__global__ void __launch_bounds__(256) sums_last_block_kernel(int n, SumCols S, double* work) {
+  __shared__ SumsLds L;
+  sums_by_blocks(S, n, blockIdx.x, gridDim.x, work, L);
 }
 
-// one large system: block k sums atoms [1024 k, 1024 (k + 1)) of every column;
-// the last block to finish sums the partials in block order (as
-// sum_last_block_kernel) and resets the counter
-__global__ void __launch_bounds__(256)
-sums_last_block_kernel(int n, SumSrc S, double* work) {
-  __shared__ double part[SUMS_MAX_COL][4];
-  __shared__ double stage[256];
-  __shared__ int last;
-  unsigned int* counter = reinterpret_cast<unsigned int*>(work);
-  double* partial = work + 1;
-  const int k = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int lo = k * 1024, hi = min(n, lo + 1024);
-  int cg = 0;
-  for (int q = 0; q < S.nsrc; ++q) {
-    for (int c = 0; c < S.cols[q]; ++c, ++cg) {
-      double v[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) v[u] = src_val(S, q, min(lo + u * 256 + tid, n - 1), c);
-      double acc = 0.0;
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (lo + u * 256 + tid < hi) acc += v[u];
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
-      if (lane == 0) part[cg][wv] = acc;
-    }
-  }
-  __syncthreads();
-  const int C = S.ctot;
-  if (tid < C) partial[(long)k * C + tid] = ((part[tid][0] + part[tid][1]) + part[tid][2]) + part[tid][3];
-  __syncthreads();
-  if (tid == 0) {
-    const unsigned int done =
-        __hip_atomic_fetch_add(counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-    last = done == gridDim.x - 1;
-  }
-  __syncthreads();
-  if (!last) return;
-  __threadfence();
-  // partials [nb][C] staged 256 at a time; thread c < C adds column c in block order
-  const int tot_n = (int)gridDim.x * C;
-  double tot = 0.0;
-  for (int e0 = 0; e0 < tot_n; e0 += 256) {
-    stage[tid] = e0 + tid < tot_n ? partial[e0 + tid] : 0.0;
-    __syncthreads();
-    if (tid < C) {
-      const int e1 = min(e0 + 256, tot_n);
-      for (int e = e0 + ((tid - e0 % C) + C) % C; e < e1; e += C) tot += stage[e - e0];
-    }
-    __syncthreads();
-  }
-  if (tid < C) {
-    int q = 0, c = tid;
-    while (c >= S.cols[q]) { c -= S.cols[q]; ++q; }
-    S.out[q][c] = tot;
-  }
-  if (tid == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// one block per molecule, every column; fixed reduction tree
 template <int NT>
 __global__ void __launch_bounds__(NT)
-sums_per_mol_kernel(const int* __restrict__ mol_start, SumSrc S) {
-  __shared__ double part[NT / 64];
-  const int m = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int lo = mol_start[m], hi = mol_start[m + 1];
-  for (int q = 0; q < S.nsrc; ++q) {
-    for (int c = 0; c < S.cols[q]; ++c) {
-      double acc = 0.0;
-      for (int a = lo + tid; a < hi; a += NT) acc += src_val(S, q, a, c);
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
-      if (lane == 0) part[wv] = acc;
-      __syncthreads();
-      if (tid == 0) {
-        double v = 0.0;
-        for (int w = 0; w < NT / 64; ++w) v += part[w];
-        S.out[q][(long)m * S.cols[q] + c] = v;
-      }
-      __syncthreads();
-    }
-  }
+sums_per_mol_kernel(const int* __restrict__ mol_start, SumCols S) {
+  __shared__ SumsLds L;
+  sums_of_molecule<NT>(S, mol_start, blockIdx.x, L);
 }
 
 template <class T>
@@ -658,24 +572,9 @@ CoulArgs coul_args(const double* consts, double rc_ee, double width, int add_ecc
 int mol_sums_impl(const char* name, int B, const int* mol_start, int n_total, int nsrc,
                   const void* const* in, const int* f64, const int* cols, const int* ld,
                   double* const* out, double* work, void* stream) {
-  TM_REQUIRE(B >= 0 && n_total >= 0 && nsrc > 0 && nsrc <= SUMS_MAX_SRC, "%s: bad sizes", name);
-  SumSrc S;
-  S.nsrc = nsrc;
-  S.ctot = 0;
-  for (int k = 0; k < SUMS_MAX_SRC; ++k) {
-    const bool on = k < nsrc;
-    S.in[k] = on ? in[k] : nullptr;
-    S.out[k] = on ? out[k] : nullptr;
-    S.f64[k] = on ? f64[k] : 0;
-    S.cols[k] = on ? cols[k] : 0;
-    S.ld[k] = on ? ld[k] : 0;
-    if (on) {
-      TM_REQUIRE(cols[k] > 0 && ld[k] >= cols[k] && in[k] != nullptr && out[k] != nullptr,
-                 "%s: bad source %d", name, k);
-      S.ctot += cols[k];
-    }
-  }
-  TM_REQUIRE(S.ctot <= SUMS_MAX_COL, "%s: %d columns above %d", name, S.ctot, SUMS_MAX_COL);
+  SumCols S;
+  const int st = sum_cols(name, B, n_total, nsrc, in, f64, cols, ld, out, &S);
+  if (st) return st;
   if (B == 0) return TM_OK;
   hipStream_t s = (hipStream_t)stream;
   if (B == 1 && n_total > 2048 && work != nullptr) {

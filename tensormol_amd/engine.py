@@ -483,16 +483,9 @@ class BPEEEngine:
         (device float64 arrays, ke may be None) also advances a Velocity Verlet
         state in the same launch as the gather: the kick of this step with the
         new forces, then the drift of the next (x is updated in place)."""
-        self._need_rev(ws, pos)
+        self._adjoint_slots(ws, pos)
         key = (pos.data_ptr(), self._raw_stream())
         st = self._stream
-        sym = self.model.sym
-        self._call(ws, "tm_sym_adjoint#energy", key, lambda: (
-            ws.N, _P(pos), _P(ws.box), _P(ws.mol), _P(ws.elem), _P(ws.nbr), _P(ws.ncnt),
-            _P(ws.rseg), _P(ws.ang), _P(ws.acnt), _P(ws.aseg), self.ldr, self.lda, self.nele,
-            sym.nr_r, sym.eta, sym.zeta, sym.rr, sym.ra, _lib.fptr(self.sym_rs_r),
-            _lib.fptr(self.sym_rs_a), _lib.fptr(self.sym_th), _P(ws.JE), _P(ws.JQ), None,
-            _P(ws.phi), _P(ws.phimean), self.D, _P(ws.wslot), st()))
         if vv is None:
             self._call(ws, "tm_force_gather#energy", key, lambda: (
                 ws.N, self.ldr, _P(ws.ncnt), _P(ws.rev), _P(ws.wslot), _P(ws.gradc),
@@ -504,6 +497,19 @@ class BPEEEngine:
                 ws.N, self.ldr, _P(ws.ncnt), _P(ws.rev), _P(ws.wslot), _P(ws.gradc),
                 JOULEPERHARTREE, _P(ws.grad), _P(ws.force), float(dt), _P(m), _P(v), _P(a),
                 _P(ke), _P(x), st()))
+
+    def _adjoint_slots(self, ws, pos):
+        """The descriptor adjoint of the energy: one gradient per neighbour slot."""
+        self._need_rev(ws, pos)
+        key = (pos.data_ptr(), self._raw_stream())
+        st = self._stream
+        sym = self.model.sym
+        self._call(ws, "tm_sym_adjoint#energy", key, lambda: (
+            ws.N, _P(pos), _P(ws.box), _P(ws.mol), _P(ws.elem), _P(ws.nbr), _P(ws.ncnt),
+            _P(ws.rseg), _P(ws.ang), _P(ws.acnt), _P(ws.aseg), self.ldr, self.lda, self.nele,
+            sym.nr_r, sym.eta, sym.zeta, sym.rr, sym.ra, _lib.fptr(self.sym_rs_r),
+            _lib.fptr(self.sym_rs_a), _lib.fptr(self.sym_th), _P(ws.JE), _P(ws.JQ), None,
+            _P(ws.phi), _P(ws.phimean), self.D, _P(ws.wslot), st()))
 
     def descriptor_jvp(self, ws, pos, du, out):
         """out[:N, :D] = dG/dx . du (float32) for per-atom displacements du
@@ -532,23 +538,35 @@ class BPEEEngine:
         L.tm_force_gather(ws.N, self.ldr, _P(ws.ncnt), _P(ws.rev), _P(ws.wslot), None, 1.0,
                           _P(grad), None, st)
 
-    def reductions(self, ws):
-        """Per-molecule BP energy, Coulomb/vdW energies and dipole in one launch."""
+    def _sums_args(self, ws):
+        """(sources, inputs, types, columns, strides, outputs) of the closing sums."""
         key = (ws.eps.data_ptr(), ws.eatom.data_ptr(), ws.qx.data_ptr(), ws.Ebp.data_ptr(),
                ws.Eext.data_ptr(), ws.dipole.data_ptr())
-        arr = getattr(ws, "_sums_args", None)
+        arr = getattr(ws, "_sums", None)
         if arr is None or arr[0] != key:
             c = _lib.ctypes
             srcs = ((ws.eps, 0, 1, 1, ws.Ebp), (ws.eatom, 1, 2, 2, ws.Eext), (ws.qx, 1, 3, 3, ws.dipole))
-            arr = (key, (c.c_void_p * 3)(*[t.data_ptr() for t, *_ in srcs]),
-                   (c.c_int * 3)(*[f for _, f, _, _, _ in srcs]),
-                   (c.c_int * 3)(*[k for _, _, k, _, _ in srcs]),
-                   (c.c_int * 3)(*[ld for _, _, _, ld, _ in srcs]),
-                   (c.c_void_p * 3)(*[o.data_ptr() for *_, o in srcs]))
-            ws._sums_args = arr
-        _, ins, f64, cols, ld, outs = arr
-        self.lib.tm_mol_sums(ws.B, _P(ws.mol_start), ws.N, 3, ins, f64, cols, ld, outs, _P(ws.red),
+            arr = (key, (3, (c.c_void_p * 3)(*[t.data_ptr() for t, *_ in srcs]),
+                         (c.c_int * 3)(*[f for _, f, _, _, _ in srcs]),
+                         (c.c_int * 3)(*[k for _, _, k, _, _ in srcs]),
+                         (c.c_int * 3)(*[ld for _, _, _, ld, _ in srcs]),
+                         (c.c_void_p * 3)(*[o.data_ptr() for *_, o in srcs])))
+            ws._sums = arr
+        return arr[1]
+
+    def reductions(self, ws):
+        """Per-molecule BP energy, Coulomb/vdW energies and dipole in one launch."""
+        self.lib.tm_mol_sums(ws.B, _P(ws.mol_start), ws.N, *self._sums_args(ws), _P(ws.red),
                              self._stream())
+
+    def _forces_and_sums(self, ws, pos):
+        """adjoint() and reductions() with the force gather and the sums in one launch."""
+        self._adjoint_slots(ws, pos)
+        sums = self._sums_args(ws)
+        key = (pos.data_ptr(), self._raw_stream()) + ws._sums[0]
+        self._call(ws, "tm_force_gather_sums", key, lambda: (
+            ws.N, self.ldr, _P(ws.ncnt), _P(ws.rev), _P(ws.wslot), _P(ws.gradc), JOULEPERHARTREE,
+            _P(ws.grad), _P(ws.force), ws.B, _P(ws.mol_start), *sums, _P(ws.red), self._stream()))
 
     def run(self, ws, pos, forces=True, check=None):
         """Enqueue one full evaluation for positions pos (cuda float64 [N,3]).
@@ -562,8 +580,9 @@ class BPEEEngine:
         self.networks(ws)
         self.electrostatics(ws, pos)
         if forces:
-            self.adjoint(ws, pos)
-        self.reductions(ws)
+            self._forces_and_sums(ws, pos)
+        else:
+            self.reductions(ws)
         if self.check_overflow if check is None else check:
             self.check_flags(ws)
 
@@ -579,7 +598,9 @@ class BPEEEngine:
 
     def energy_tensor(self, ws):
         """Per-molecule total energy as a device tensor (no host copy)."""
-        return ws.Ebp[:ws.B] + ws.Eext[:ws.B, 0] + ws.Eext[:ws.B, 1]
+        E = torch.empty(ws.B, dtype=torch.float64, device=ws.Ebp.device)
+        self.lib.tm_total_energy(ws.B, _P(ws.Ebp), _P(ws.Eext), _P(E), self._stream())
+        return E
 
 
 class NeighbourOverflow(RuntimeError):
