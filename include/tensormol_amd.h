@@ -213,8 +213,9 @@ int tm_train_elem(int op, int M, int H, int ld, float alpha, const float* s, con
 int tm_rows(int scatter, int M, int cols, const int* idx, const float* in, int ldi, float* out,
             int ldo, void* stream);
 
-/* One row gather / scatter of a grouped call; fields as tm_rows' arguments;
- * out_bf16: out is BF16 (the FP32 input rounded to nearest even). */
+/* One row gather / scatter of a grouped call; fields as tm_rows' arguments (idx
+ * NULL: row r itself); out_bf16: out is BF16 (the FP32 input rounded to nearest
+ * even). */
 typedef struct tm_rows_group {
   int M, cols;
   const int* idx;
@@ -226,7 +227,7 @@ typedef struct tm_rows_group {
 } tm_rows_group;
 
 /* ngroups tm_rows calls (groups: host array; the per-element row sets of one
- * step) in one launch per 16 of them. */
+ * step) in one launch per 32 of them. */
 int tm_rows_grouped(int ngroups, const tm_rows_group* groups, int scatter, void* stream);
 
 /* out[0 .. n) = BF16 of in (round to nearest even) for ngroups arrays (host

@@ -858,26 +858,65 @@ __global__ void rows_kernel(int scatter, int M, int cols, const int* __restrict_
   else out[(long)r * ldo + c] = in[(long)idx[r] * ldi + c];
 }
 
-// rows_kernel over several (idx, in, out) sets at once, one per blockIdx.y.
+// rows_kernel over several (idx, in, out) sets at once; idx NULL: row r itself.
+// A block takes four rows, a wave each, or 256 rows of a single column; set g's
+// blocks start at block0[g].  Rows that allow it go in 16-byte loads, three in
+// flight per lane: 10,398 descriptor rows of 768 and eight columns as BF16
+// 13.9 -> 11.3 us, the rows and the weights (a launch of 8.3 us of their own
+// before) 13.0 -> 15.1.
+constexpr int MAXR = 32;
 struct RowsBatch {
-  tm_rows_group r[MAXG];
+  int block0[MAXR];
+  tm_rows_group r[MAXR];
   int scatter;
 };
 
-// Four rows per 256-thread block, 64 lanes per row walking its columns.
-__global__ void rows_grouped_kernel(const RowsBatch rb) {
-  const tm_rows_group& d = rb.r[blockIdx.y];
-  const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
+__global__ void __launch_bounds__(256) rows_grouped_kernel(const RowsBatch rb) {
+  int g = 0;
+#pragma unroll
+  for (int k = 1; k < MAXR; ++k) g += (int)blockIdx.x >= rb.block0[k] ? 1 : 0;
+  const tm_rows_group& d = rb.r[g];
+  const int block = (int)blockIdx.x - rb.block0[g];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int cols = d.cols;
+  const int r = cols == 1 ? block * 256 + (int)threadIdx.x : block * 4 + w;
   if (r >= d.M) return;
-  const long src = rb.scatter ? (long)r * d.ldi : (long)d.idx[r] * d.ldi;
-  const long dst = rb.scatter ? (long)d.idx[r] * d.ldo : (long)r * d.ldo;
-  if (d.out_bf16) {
-    unsigned short* out = static_cast<unsigned short*>(d.out);
-    for (int c = threadIdx.x & 63; c < d.cols; c += 64)
-      out[dst + c] = (unsigned short)bf16_bits(d.in[src + c]);
-  } else {
-    float* out = static_cast<float*>(d.out);
-    for (int c = threadIdx.x & 63; c < d.cols; c += 64) out[dst + c] = d.in[src + c];
+  const long at = d.idx != nullptr ? d.idx[r] : r;
+  const float* in = d.in + (rb.scatter ? (long)r : at) * d.ldi;
+  const long dst = (rb.scatter ? at : (long)r) * d.ldo;
+  unsigned short* oh = static_cast<unsigned short*>(d.out) + dst;
+  float* of = static_cast<float*>(d.out) + dst;
+  if (cols == 1) {
+    if (d.out_bf16) oh[0] = (unsigned short)bf16_bits(in[0]);
+    else of[0] = in[0];
+    return;
+  }
+  const uintptr_t out = d.out_bf16 ? reinterpret_cast<uintptr_t>(oh) << 1 : reinterpret_cast<uintptr_t>(of);
+  const bool wide = cols % 4 == 0 && ((reinterpret_cast<uintptr_t>(in) | out) & 15) == 0;
+  if (wide) {
+    for (int c0 = 0; c0 < cols; c0 += 768) {
+      float4 v[3];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const int c = c0 + 4 * (lane + 64 * k);
+        if (c < cols) v[k] = *reinterpret_cast<const float4*>(in + c);
+      }
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const int c = c0 + 4 * (lane + 64 * k);
+        if (c >= cols) break;
+        if (d.out_bf16)
+          *reinterpret_cast<uint2*>(oh + c) = make_uint2(bf16_bits(v[k].x) | (bf16_bits(v[k].y) << 16),
+                                                         bf16_bits(v[k].z) | (bf16_bits(v[k].w) << 16));
+        else
+          *reinterpret_cast<float4*>(of + c) = v[k];
+      }
+    }
+    return;
+  }
+  for (int c = lane; c < cols; c += 64) {
+    if (d.out_bf16) oh[c] = (unsigned short)bf16_bits(in[c]);
+    else of[c] = in[c];
   }
 }
 
@@ -1125,16 +1164,20 @@ int tm_rows_grouped(int ngroups, const tm_rows_group* groups, int scatter, void*
     RowsBatch rb;
     rb.scatter = scatter;
     int n = 0;
-    int most = 0;
-    for (; g0 < ngroups && n < MAXG; ++g0) {
+    long blocks = 0;
+    for (; g0 < ngroups && n < MAXR; ++g0) {
       const tm_rows_group& q = groups[g0];
       TM_REQUIRE(q.M >= 0 && q.cols >= 0, "tm_rows_grouped: negative size (set %d)", g0);
       if ((long)q.M * q.cols == 0) continue;
+      const long more = tm_div_up(q.M, q.cols == 1 ? 256 : 4);
+      if (blocks + more > 0x7fffffffl) break;   // the next launch's
+      rb.block0[n] = (int)blocks;
       rb.r[n++] = q;
-      most = std::max(most, q.M);
+      blocks += more;
     }
     if (n == 0) continue;
-    rows_grouped_kernel<<<dim3(tm_div_up(most, 4), n), 256, 0, (hipStream_t)stream>>>(rb);
+    for (int k = n; k < MAXR; ++k) rb.block0[k] = 0x7fffffff;
+    rows_grouped_kernel<<<(int)blocks, 256, 0, (hipStream_t)stream>>>(rb);
     TM_LAUNCH_CHECK();
   }
   return TM_OK;

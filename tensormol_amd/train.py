@@ -272,13 +272,6 @@ class ForceMatchingTrainer:
         self.eng.lib.tm_rows_grouped(len(sets), _ctypes.cast(arr, _ctypes.c_void_p), scatter,
                                      self.eng._stream())
 
-    def _cast(self, pairs):
-        """One tm_cast_bf16_grouped call: each (FP32 tensor, BF16 tensor) pair."""
-        arr = (_lib.CastGroup * len(pairs))(
-            *[_lib.CastGroup(x.data_ptr(), y.data_ptr(), x.numel()) for x, y in pairs])
-        self.eng.lib.tm_cast_bf16_grouped(len(pairs), _ctypes.cast(arr, _ctypes.c_void_p),
-                                          self.eng._stream())
-
     def _mfma_step(self, tb, pos, check=True, views=False):
         """(L, E, F, gradients in parameters() order) of the BF16 MFMA path.
         Each GEMM stage runs for every element in one grouped launch, with
@@ -301,10 +294,12 @@ class ForceMatchingTrainer:
         # per-element GEMMs below write every row of these through their row maps
         eps = torch.empty(N, 1, **f32)
         J = torch.empty(N, D, **f32)
-        # this step's weights as BF16 (one launch), then the descriptors as BF16 rows
-        self._cast([(prm[l][0], b["Wb"][l]) for b, prm in items for l in range(4)])
+        # this step's weights and the descriptors' rows as BF16, in one launch
+        whole = lambda W: (1, W.numel()) if W.shape[1] == 1 else tuple(W.shape)
         self._grows([(b["M"], D, ad(b["idx"]), ad(ws.G), D, ad(b["X0"]), b["ldx"], 1)
-                     for b, _ in items], 0)
+                     for b, _ in items] +
+                    [(*whole(W), None, ad(W), whole(W)[1], ad(Wb), whole(W)[1], 1)
+                     for b, prm in items for (W, _), Wb in zip(prm, b["Wb"])], 0)
         # forward: z_l = h_{l-1} W_l + b_l, h_l = act(z_l), s_l = act'(z_l); the
         # last layer also starts the J chain, zd_3 = s_3 w_4 (rows M.. of ZZ3)
         layers = (("X0", "H1", "S1", "ZT1"), ("H1", "H2", "S2", "ZT2"), ("H2", "H3", "S3", "ZT3"))
@@ -319,10 +314,6 @@ class ForceMatchingTrainer:
                     g.update(x1=ad(prm[3][0]), out2=ad(b["ZZ3"], M, ldh))
                 grp.append(g)
             self._ggemm(grp, 0, 0, 1, io=1 | 2 | 8)   # H_l, zd_3 BF16; s_l FP32
-        # atom energies y = h_3 w_4 + b_4, written to each atom's row of eps
-        self._ggemm([dict(M=b["M"], N=1, K=H, A=ad(b["H3"]), lda=b["ldh"], B=ad(b["Wb"][3]),
-                          ldb=1, C=ad(eps), ldc=1, bias=ad(prm[3][1]), crow=ad(b["idx"]))
-                     for b, prm in items], 0, 0, 0)
         # J chain: hd_{l-1} = zd_l W_l^T, zd_{l-1} = s_{l-1} hd_{l-1}, J = zd_1 W_1^T
         for (l, zz_in, hd, sk, zz_out) in ((2, "ZZ3", "HD2", "S2", "ZZ2"),
                                            (1, "ZZ2", "HD1", "S1", "ZZ1")):
@@ -330,9 +321,13 @@ class ForceMatchingTrainer:
                               B=ad(b["Wb"][l]), ldb=H, C=ad(b[hd]), ldc=b["ldh"], s=ad(b[sk]),
                               aux=ad(b[zz_out], b["M"], b["ldh"])) for b, prm in items], 0, 1, 2,
                         io=1 | 4)   # hd FP32, zd BF16
-        # J rows written to each atom's row of J
+        # J rows written to each atom's row of J, and in the same launch the atom
+        # energies y = h_3 w_4 + b_4 to each atom's row of eps (w_4 is one row of W^T)
         self._ggemm([dict(M=b["M"], N=D, K=H, A=ad(b["ZZ1"], b["M"], b["ldh"]), lda=b["ldh"],
                           B=ad(b["Wb"][0]), ldb=H, C=ad(J), ldc=D, crow=ad(b["idx"]))
+                     for b, prm in items] +
+                    [dict(M=b["M"], N=1, K=H, A=ad(b["H3"]), lda=b["ldh"], B=ad(b["Wb"][3]),
+                          ldb=H, C=ad(eps), ldc=1, bias=ad(prm[3][1]), crow=ad(b["idx"]))
                      for b, prm in items], 0, 1, 0)
         f64 = dict(dtype=torch.float64, device=self.device)
         grad = torch.empty(N, 3, **f64)
@@ -347,7 +342,7 @@ class ForceMatchingTrainer:
                            P(tb.F_ref), P(tb.w_f), P(E), P(ybar), P(gg), P(part), P(Lt),
                            eng._stream())
         L = Lt[0]
-        F = -grad
+        F = None if views else -grad   # step() has no use for the forces
         V = torch.empty(N, D, **f32)
         eng.descriptor_jvp(ws, pos, gg, V)
         self._grows([(b["M"], D, ad(b["idx"]), ad(V), D, ad(b["X0"], b["M"], b["ldx"]), b["ldx"],
