@@ -35,11 +35,14 @@ constexpr int GT = 128;       // C tile edge per workgroup (four waves of 64 x 6
 constexpr int GK = 64;        // K per staged step (two v_mfma_f32_16x16x32_bf16 deep)
 constexpr int LROW = GK + 8;  // LDS row of a staged operand, in bf16 (144 B, padded)
 constexpr int MAXG = 16;      // GEMMs per grouped launch
-constexpr int MINSTEPS = 16;  // K steps below which a split is not made shorter
-// 128 x 128 tiles below which 64 x 128 ones are used (four per CU).  Softplus
-// epilogue, N = K = 512: 2,560 rows (80 tiles) 18.9 -> 13.3 us, 10,240 (320)
-// 27.5 -> 23.6, 20,480 (640) 41.3 -> 37.2; 40,960 (1,280) 66.4 against 69.3.
-constexpr int HALF_UNITS = 1024;
+// K steps below which a split is not made shorter: a training step of 10,398
+// atoms takes 607 us with 10, 600 with 16, 597 with 24 (fewer partial sums).
+constexpr int MINSTEPS = 24;
+// 128 x 128 tiles below which 64 x 128 ones are used (two per CU).  Softplus
+// epilogue, N = K = 512: 2,560 rows (80 tiles) 18.5 -> 12.4 us, 10,240 (320)
+// 26.2 -> 22.4; 20,480 (640) 33.7 against 34.9, 10,240 x 768 (480, plain) 18.9
+// against 20.5.
+constexpr int HALF_UNITS = 448;
 constexpr int NXCD = 8;       // XCDs; workgroups are dealt to them round-robin
 
 enum { EPI_STORE = 0, EPI_SOFTPLUS = 1, EPI_TANGENT = 2, EPI_REVERSE = 3 };
@@ -451,14 +454,17 @@ __global__ void __launch_bounds__(256) gemm_bf16_kernel(const GemmBatch gb) {
 // load latency per row), 2-byte loads of the operand stored across k another
 // third, and the first instructions' chain of scalar loads 2 us.  Here each
 // epilogue is its own kernel with branch-free buffer accesses and the next
-// rows' inputs in flight, operands load in 16-byte chunks two K steps ahead,
-// and a launch of few tiles uses 64 x 128 ones (HALF_UNITS).  10,240 rows,
-// N = K = 512: plain 27.7 -> 17.2 us, softplus 33.8 -> 23, tangent 32.2 ->
-// 18.4, reverse 31.0 -> 21.7; the weight-gradient launch of 10,398 atoms
-// 259 -> 124 us, of which 40 came from units that run split by split, so that
+// rows' inputs in flight, and operands load in 16-byte chunks ahead of their
+// step.  128-row tiles stage one step at a time and their C tile in two parts,
+// which lets three workgroups share a CU (two with double buffers: 45.1
+// against 37.2 us for 40,960 x 512 x 512, plain); 64-row tiles run where there
+// are too few tiles for that and keep two steps in flight each.  10,240 rows,
+// N = K = 512: plain 27.7 -> 16.9 us, softplus 33.8 -> 22.4, tangent 32.2 ->
+// 18.5, reverse 31.0 -> 21.5; the weight-gradient launch of 10,398 atoms
+// 259 -> 105 us, of which 40 came from units that run split by split, so that
 // every XCD gets the same share of GEMMs with unequal K.  What is left is the
-// issue of loads, LDS stores and LDS reads by one or two workgroups per CU
-// (a step's MFMAs are a quarter of its time) and launch latency.
+// issue of loads, LDS stores and LDS reads (a step's MFMAs are a quarter of
+// its time) and launch latency.
 //
 // LDS image of a staged operand: S[row][k] in BF16, 128 bytes per row, so an
 // MFMA fragment (8 consecutive k of one row) is one 16-byte read.  Chunk c (16
@@ -584,14 +590,16 @@ __device__ __forceinline__ void buf_st4(__amdgpu_buffer_rsrc_t b, unsigned e, bo
 }
 
 template <bool TA, bool TB, int EPI, int GM>
-__global__ void __launch_bounds__(256, GM == GT ? 2 : 3) gemm_wide_kernel(const GemmBatch gb) {
-  // two staged K steps of A (GM rows) and B, and after the K loop the C tile
+__global__ void __launch_bounds__(256, 3) gemm_wide_kernel(const GemmBatch gb) {
+  // NBUF staged K steps of A (GM rows) and B, and after the K loop GM / NH rows
+  // of the C tile
+  constexpr int NBUF = GM == GT ? 1 : 2, NH = GM == GT ? 2 : 1;
   constexpr int AOP = GM * GK, BOP = GT * GK;   // elements of a staged operand
   constexpr int MI = GM / 32;                   // 16-row blocks per wave
-  constexpr int CB = GM * CLD * 4, OB = 4 * (AOP + BOP);
+  constexpr int CB = GM / NH * CLD * 4, OB = NBUF * 2 * (AOP + BOP);
   __shared__ __align__(16) unsigned char lds[CB > OB ? CB : OB];
   unsigned short* As = reinterpret_cast<unsigned short*>(lds);
-  unsigned short* Bs = As + 2 * AOP;
+  unsigned short* Bs = As + NBUF * AOP;
   const Unit un = unit_of(gb);
   if (un.gi < 0) return;
   const GemmDev& g = gb.g[un.gi];
@@ -601,36 +609,37 @@ __global__ void __launch_bounds__(256, GM == GT ? 2 : 3) gemm_wide_kernel(const 
   const int k_begin = split * g.kchunk;
   const int nsteps = max(min(g.K - k_begin, g.kchunk) + GK - 1, 0) / GK;
   const int wm = (w >> 1) * (GM / 2), wn = (w & 1) * 64;
-  WideStage<!TA, GM> sa[2];
-  WideStage<TB, GT> sb[2];
+  WideStage<!TA, GM> sa[NBUF];
+  WideStage<TB, GT> sb[NBUF];
   sa[0].init(reinterpret_cast<const unsigned short*>(g.A), g.lda, M, m0, g.K, k_begin, tid);
   sb[0].init(reinterpret_cast<const unsigned short*>(g.B), g.ldb, N, n0, g.K, k_begin, tid);
-  sa[1] = sa[0];
-  sb[1] = sb[0];
   auto load = [&](int step, auto& xa, auto& xb) {
     const unsigned kill = step < nsteps ? 0u : OOB;
     xa.load(step, kill);
     xb.load(step, kill);
+    __builtin_amdgcn_sched_barrier(0);   // in this order: the waits count loads in flight
   };
   load(0, sa[0], sb[0]);
-  __builtin_amdgcn_sched_barrier(0);   // in this order: the waits count loads in flight
-  load(1, sa[1], sb[1]);
-  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (NBUF == 2) {
+    sa[1] = sa[0];
+    sb[1] = sb[0];
+    load(1, sa[1], sb[1]);
+  }
   floatx4 acc[MI][4];
 #pragma unroll
   for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-  // 16-row blocks of this wave's quadrant that hold output; the others only
-  // feed rows and columns that are not stored
-  const int nj = (N - n0 - wn + 15) >> 4, mi = nj > 0 ? min((M - m0 - wm + 15) >> 4, MI) : 0;
+  // a wave whose quadrant holds no output stages and waits like the others
+  const bool active = m0 + wm < M && n0 + wn < N;
   const int fr = lane & 15, fc = lane >> 4;
-  // One K step from LDS buffer b.
-  auto multiply = [&](int b, auto full) {
+  // The K step in LDS buffer b.
+  auto multiply = [&](int b) {
     const unsigned short* Ab = As + b * AOP;
     const unsigned short* Bb = Bs + b * BOP;
 #pragma unroll
     for (int kk = 0; kk < GK / 8; kk += 4) {
+      if (GM == GT && kk > 0) __builtin_amdgcn_sched_barrier(0);   // fragments of one half at a time
       uint4 fa[MI], fb[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j)
@@ -639,44 +648,32 @@ __global__ void __launch_bounds__(256, GM == GT ? 2 : 3) gemm_wide_kernel(const 
       for (int i = 0; i < MI; ++i)
         fa[i] = *reinterpret_cast<const uint4*>(&Ab[lds_at(wm + 16 * i + fr, kk + fc)]);
 #pragma unroll
-      for (int i = 0; i < MI; ++i) {
-        if (full || i < mi) {
+      for (int i = 0; i < MI; ++i)
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                __builtin_bit_cast(bf16x8, fb[j]), __builtin_bit_cast(bf16x8, fa[i]), acc[i][j], 0,
-                0, 0);
-        }
-      }
+        for (int j = 0; j < 4; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8, fb[j]), __builtin_bit_cast(bf16x8, fa[i]), acc[i][j], 0, 0,
+              0);
     }
   };
-  // The waves of a workgroup may take different branches here: they meet at
-  // the same number of barriers.
-  auto kloop = [&](auto full) {
-    for (int step = 0; step < nsteps; step += 2) {
-      sa[0].store(As, tid);
-      sb[0].store(Bs, tid);
+  for (int step = 0; step < nsteps; step += NBUF) {
+#pragma unroll
+    for (int b = 0; b < NBUF; ++b) {
+      sa[b].store(As + b * AOP, tid);
+      sb[b].store(Bs + b * BOP, tid);
       __syncthreads();
-      load(step + 2, sa[0], sb[0]);
-      __builtin_amdgcn_sched_barrier(0);
-      multiply(0, full);
-      sa[1].store(As + AOP, tid);
-      sb[1].store(Bs + BOP, tid);
-      __syncthreads();
-      load(step + 3, sa[1], sb[1]);
-      __builtin_amdgcn_sched_barrier(0);
-      if (step + 1 < nsteps) multiply(1, full);
+      load(step + b + NBUF, sa[b], sb[b]);
+      if (active && (b == 0 || step + b < nsteps)) multiply(b);
+      if (NBUF == 1) __syncthreads();   // every wave is done with the staged operands
     }
-  };
-  if (mi == MI) kloop(std::true_type{});
-  else kloop(std::false_type{});
+  }
   // Epilogue (the formulas: epilogue_tile).  The C tile goes through LDS;
   // thread t takes columns 4 (t % 32) .. + 3 of rows t / 32 + 8 r, ER rows at
   // a time.  The row-indexed inputs of the next ER rows are in flight while
   // these are computed and stored; the first are requested before the tile is
   // in LDS.  Rows past the last lie outside the buffers: they read zero and
   // write nothing.
-  constexpr int ER = 4, NB = GM / 8 / ER;
+  constexpr int ER = EPI == EPI_REVERSE ? 2 : 4, NB = GM / 8 / ER;
   constexpr bool HAS_S = EPI == EPI_TANGENT || EPI == EPI_REVERSE;
   const int c = (tid & 31) * 4, n = n0 + c, row = tid >> 5, io = gb.io;
   const long ldc = g.ldc, left = (long)(M - 1 - m0) * ldc + N;   // elements from row m0 on
@@ -709,7 +706,6 @@ __global__ void __launch_bounds__(256, GM == GT ? 2 : 3) gemm_wide_kernel(const 
         q.ym[j] = has_out2 ? g.x2[min(m0 + row + 8 * (ER * b + j), M - 1)] : 0.f;
     }
   };
-  int crow[EPI == EPI_STORE ? GM / 8 : 1];
   if (n < N) {
     fetch(cur, 0);
 #pragma unroll
@@ -717,76 +713,84 @@ __global__ void __launch_bounds__(256, GM == GT ? 2 : 3) gemm_wide_kernel(const 
       if (g.bias != nullptr && n + k < N) bv[k] = g.bias[n + k];
       if (has_out2) wv[k] = g.x1[n + k];
     }
-    if (EPI == EPI_STORE && g.crow != nullptr) {
-#pragma unroll
-      for (int r = 0; r < GM / 8; ++r) crow[r] = g.crow[min(m0 + row + 8 * r, M - 1)];
-    }
   }
-  __syncthreads();   // every wave is done with the staged operands
   float* Cs = reinterpret_cast<float*>(lds);
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      *reinterpret_cast<floatx4*>(&Cs[(wm + 16 * i + fr) * CLD + wn + 16 * j + fc * 4]) = acc[i][j];
-  __syncthreads();
-  if (n >= N) return;
   const float* Ct = Cs + row * CLD + c;
-  if constexpr (EPI == EPI_STORE) {
-    float* C = g.C + (long)split * g.cstride;
-    const bool half = (io & 2) != 0;
-    if (g.crow == nullptr && g.vec_out && n + 4 <= N) {
-      const __amdgpu_buffer_rsrc_t bc = obuf(C, 2);
-#pragma unroll 4
-      for (int r = 0; r < GM / 8; ++r) {
-        const float4 f = *reinterpret_cast<const float4*>(Ct + r * 8 * CLD);
-        const float o[4] = {f.x + bv[0], f.y + bv[1], f.z + bv[2], f.w + bv[3]};
-        buf_st4(bc, e0 + r * estep, half, o);
-      }
-    } else {   // a row map, or columns that do not take 16-byte stores
-      const int nv = min(4, N - n);
-#pragma unroll
-      for (int r = 0; r < GM / 8; ++r) {
-        const int m = m0 + row + 8 * r;
-        if (m >= M) break;
-        const long o = (long)(g.crow != nullptr ? crow[r] : m) * ldc + n;
-        const float4 f = *reinterpret_cast<const float4*>(Ct + r * 8 * CLD);
-        const float v[4] = {f.x + bv[0], f.y + bv[1], f.z + bv[2], f.w + bv[3]};
-        if (half) st4h(reinterpret_cast<unsigned short*>(C), o, nv, g.vec_out != 0, v);
-        else st4(C, o, nv, g.vec_out != 0, v);
-      }
-    }
-    return;
-  }
   const float a = gb.alpha, ia = 1.0f / a;
-  const __amdgpu_buffer_rsrc_t bc = obuf(g.C, 2), ba = obuf(g.aux, 4), bo = obuf(g.out2, 8);
+  float* Cp = EPI == EPI_STORE ? g.C + (long)split * g.cstride : g.C;
+  const __amdgpu_buffer_rsrc_t bc = obuf(Cp, 2), ba = obuf(g.aux, 4), bo = obuf(g.out2, 8);
   const bool hc = (io & 2) != 0, ha = (io & 4) != 0, ho = (io & 8) != 0;
+  if (NBUF == 2) __syncthreads();   // every wave is done with the staged operands
 #pragma unroll 1
-  for (int b = 0; b < NB; ++b) {
-    if (HAS_S && b + 1 < NB) fetch(nxt, b + 1);
+  for (int h = 0; h < NH; ++h) {      // NH 2: the rows of waves 2 h and 2 h + 1
+    constexpr int HR = GM / 8 / NH;   // a thread's rows of a part
+    int crow[HR];
+    if (EPI == EPI_STORE && g.crow != nullptr && n < N) {
 #pragma unroll
-    for (int j = 0; j < ER; ++j) {
-      const unsigned e = e0 + (unsigned)(ER * b + j) * estep;
-      const float4 f = *reinterpret_cast<const float4*>(Ct + (ER * b + j) * 8 * CLD);
-      const float v[4] = {f.x, f.y, f.z, f.w};
-      float sv[4], u1[4], u2[4], r0[4], r1[4], r2[4];
-      if (HAS_S) { sv[0] = cur.s[j].x; sv[1] = cur.s[j].y; sv[2] = cur.s[j].z; sv[3] = cur.s[j].w; }
-      if (EPI == EPI_REVERSE) {
-        u1[0] = cur.u1[j].x; u1[1] = cur.u1[j].y; u1[2] = cur.u1[j].z; u1[3] = cur.u1[j].w;
-        u2[0] = cur.u2[j].x; u2[1] = cur.u2[j].y; u2[2] = cur.u2[j].z; u2[3] = cur.u2[j].w;
-      }
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        if constexpr (EPI == EPI_SOFTPLUS) softplus_epi(v[k], bv[k], wv[k], a, ia, r0[k], r1[k], r2[k]);
-        else if constexpr (EPI == EPI_TANGENT)
-          tangent_epi(v[k], sv[k], cur.ym[j], wv[k], a, r0[k], r1[k], r2[k]);
-        else r0[k] = reverse_epi(v[k], sv[k], u1[k], u2[k], a);
-      }
-      if (EPI != EPI_TANGENT || g.C != nullptr) buf_st4(bc, e, hc, r0);
-      if (EPI != EPI_REVERSE) buf_st4(ba, e, ha, r1);
-      if (has_out2) buf_st4(bo, e, ho, r2);
+      for (int r = 0; r < HR; ++r) crow[r] = g.crow[min(m0 + row + 8 * (HR * h + r), M - 1)];
     }
-    if (HAS_S) cur = nxt;
+    if (h > 0) __syncthreads();   // the first part is read
+    if (NH == 1 || (w >> 1) == h) {
+      const int wr = NH == 1 ? wm : 0;
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          *reinterpret_cast<floatx4*>(&Cs[(wr + 16 * i + fr) * CLD + wn + 16 * j + fc * 4]) = acc[i][j];
+    }
+    __syncthreads();
+    if (n >= N) continue;
+    if constexpr (EPI == EPI_STORE) {
+      if (g.crow == nullptr && g.vec_out && n + 4 <= N) {
+#pragma unroll
+        for (int r = 0; r < HR; ++r) {
+          const float4 f = *reinterpret_cast<const float4*>(Ct + r * 8 * CLD);
+          const float o[4] = {f.x + bv[0], f.y + bv[1], f.z + bv[2], f.w + bv[3]};
+          buf_st4(bc, e0 + (HR * h + r) * estep, hc, o);
+        }
+      } else {   // a row map, or columns that do not take 16-byte stores
+        const int nv = min(4, N - n);
+#pragma unroll
+        for (int r = 0; r < HR; ++r) {
+          const int m = m0 + row + 8 * (HR * h + r);
+          if (m >= M) break;
+          const long o = (long)(g.crow != nullptr ? crow[r] : m) * ldc + n;
+          const float4 f = *reinterpret_cast<const float4*>(Ct + r * 8 * CLD);
+          const float v[4] = {f.x + bv[0], f.y + bv[1], f.z + bv[2], f.w + bv[3]};
+          if (hc) st4h(reinterpret_cast<unsigned short*>(Cp), o, nv, g.vec_out != 0, v);
+          else st4(Cp, o, nv, g.vec_out != 0, v);
+        }
+      }
+    } else {
+#pragma unroll 1
+      for (int b = h * NB / NH; b < (h + 1) * NB / NH; ++b) {
+        if (HAS_S && b + 1 < NB) fetch(nxt, b + 1);
+#pragma unroll
+        for (int j = 0; j < ER; ++j) {
+          const unsigned e = e0 + (unsigned)(ER * b + j) * estep;
+          const float4 f = *reinterpret_cast<const float4*>(Ct + (ER * (b - h * NB / NH) + j) * 8 * CLD);
+          const float v[4] = {f.x, f.y, f.z, f.w};
+          float sv[4], u1[4], u2[4], r0[4], r1[4], r2[4];
+          if (HAS_S) { sv[0] = cur.s[j].x; sv[1] = cur.s[j].y; sv[2] = cur.s[j].z; sv[3] = cur.s[j].w; }
+          if (EPI == EPI_REVERSE) {
+            u1[0] = cur.u1[j].x; u1[1] = cur.u1[j].y; u1[2] = cur.u1[j].z; u1[3] = cur.u1[j].w;
+            u2[0] = cur.u2[j].x; u2[1] = cur.u2[j].y; u2[2] = cur.u2[j].z; u2[3] = cur.u2[j].w;
+          }
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            if constexpr (EPI == EPI_SOFTPLUS)
+              softplus_epi(v[k], bv[k], wv[k], a, ia, r0[k], r1[k], r2[k]);
+            else if constexpr (EPI == EPI_TANGENT)
+              tangent_epi(v[k], sv[k], cur.ym[j], wv[k], a, r0[k], r1[k], r2[k]);
+            else r0[k] = reverse_epi(v[k], sv[k], u1[k], u2[k], a);
+          }
+          if (EPI != EPI_TANGENT || g.C != nullptr) buf_st4(bc, e, hc, r0);
+          if (EPI != EPI_REVERSE) buf_st4(ba, e, ha, r1);
+          if (has_out2) buf_st4(bo, e, ho, r2);
+        }
+        if (HAS_S) cur = nxt;
+      }
+    }
   }
 }
 
