@@ -16,9 +16,7 @@
 //    The grid is shifted so that a node falls on the elu matching radius,
 //    where K's second derivative jumps.  A pair costs two table reads and ten
 //    FMAs for both energies and both derivatives instead of the erfc / exp /
-//    reciprocal chains.  The tables are read through the L1 cache (16 KiB for
-//    two elements); copies in LDS cost more waves than they save (86-91
-//    against 84-86 us on the 12,288-atom box).
+//    reciprocal chains.  Small tables are copied to LDS (CT_LDS_TABLE).
 //  - Candidates as a list (tm_sweep_list) instead of a search over ranges.
 //  - Sums.  Each lane sums its pairs in float32 (a few tens per centre) and
 //    the lane sums are added in float64 in a fixed butterfly, instead of a
@@ -31,7 +29,8 @@
 // from the host, a queue that wraps instead of moving its rest to the front
 // and table reads that return under the next chunk's tests took the box from
 // 94 to 84 us, the open 24,000-atom sphere from 133 to 119 us (charges and the
-// mean potential included).
+// mean potential included); a candidate list that holds a round whole and
+// tables in LDS, to 77 and 116.
 #include <math.h>
 
 #include "tm_cells.h"
@@ -39,11 +38,22 @@
 namespace {
 
 constexpr double CL_BOHRPERA = 1.889725989;
-constexpr int CT_WAVES = 4;
 constexpr int CT_RANGES = 480;   // stencils of more ranges are refused (tm_coulomb's bound)
-constexpr int CT_LIST = 448;     // candidate list per wave
 constexpr int CT_QCAP = 128;     // compacted pair queue per wave (a ring)
 constexpr int CL_TABLE_MAX = 3072;   // float4 table entries (48 KiB)
+// Tables of up to this many entries (16 KiB, two elements) are copied to LDS,
+// where 64 lanes read 64 different entries at once; the L1 cache serves them a
+// line at a time.  Eight waves share a copy, so that three workgroups fit a CU:
+// box 80.7 -> 76.9 us.  Larger ones stay in memory: copied, the sphere's 44 KiB
+// leave one workgroup per CU (117 -> 137 us).
+constexpr int CT_LDS_TABLE = 1024;
+// Candidate list per wave: 64 rows of a stencil hold 500 on average on the box.
+// With 448 entries most rounds went in two parts (83.6 us, sphere 123), 640:
+// 82.1 (117), 768: 80.4 (116).
+template <bool LT>
+struct CtShape {
+  static constexpr int WAVES = LT ? 8 : 4, LIST = LT ? 576 : 768;
+};
 
 struct ClArgs {
   float rc2;       // cutoff (A), squared
@@ -73,7 +83,9 @@ struct PairTab {
   float4 d, C, V;
   float t, ir;
 
-  __device__ __forceinline__ void begin(const ClArgs& a, const float4* __restrict__ tab,
+  // at(byte): entry of the tables at that offset
+  template <class At>
+  __device__ __forceinline__ void begin(const ClArgs& a, At at,
                                         unsigned vo, float4 dq) {
     d = dq;
     // r_A = sqrt(s + 1e-27), the reference's regulariser (RawSymFunc.py:1330)
@@ -82,8 +94,8 @@ struct PairTab {
     const float u = fmaf(s * ir, a.inv_h, a.u0);
     const int k = max(0, min((int)u, a.nint - 1));
     t = u - (float)k;
-    C = ld16(tab, 16u * (unsigned)k);
-    V = ld16(tab, vo + 16u * (unsigned)k);
+    C = at(16u * (unsigned)k);
+    V = at(vo + 16u * (unsigned)k);
   }
 
   __device__ __forceinline__ void finish(const ClArgs& a, float qi, ClAcc& acc) const {
@@ -102,16 +114,23 @@ struct PairTab {
   }
 };
 
-template <bool PERIODIC>
-__global__ void __launch_bounds__(CT_WAVES * 64)
+template <bool PERIODIC, bool LT>
+__global__ void __launch_bounds__(CtShape<LT>::WAVES * 64)
 coulomb_tab_kernel(int N, const float4* __restrict__ xqc, const int* __restrict__ elc,
                    const double* __restrict__ box, CellGrid grid, ClArgs a,
                    const float4* __restrict__ tab, double* __restrict__ phi,
                    double* __restrict__ grad, double* __restrict__ eatom) {
+  constexpr int CT_WAVES = CtShape<LT>::WAVES;
   __shared__ float4 qx[CT_WAVES][CT_QCAP];
-  __shared__ int qe[CT_WAVES][CT_QCAP];
-  __shared__ ListLds<CT_LIST> list[CT_WAVES];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  __shared__ unsigned char qe[CT_WAVES][CT_QCAP];
+  __shared__ ListLds<CtShape<LT>::LIST> list[CT_WAVES];
+  __shared__ float4 ltab[LT ? CT_LDS_TABLE : 1];
+  if constexpr (LT) {
+    const int nt = (1 + a.nele * (a.nele + 1) / 2) * a.nint;   // at most CT_LDS_TABLE
+    for (int t = threadIdx.x; t < nt; t += CT_WAVES * 64) ltab[t] = tab[t];
+    __syncthreads();
+  }
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int cpi = blockIdx.x * CT_WAVES + w;   // centre, in cell order
   if (cpi >= N) return;   // wave-level synchronisation only below
   const int i = grid.cell_atoms[cpi];
@@ -121,12 +140,12 @@ coulomb_tab_kernel(int N, const float4* __restrict__ xqc, const int* __restrict_
     iLx = 1.0f / Lx; iLy = 1.0f / Ly; iLz = 1.0f / Lz;
   }
   const float4 pi = xqc[cpi];
-  // vdW table of the centre with element e: field e of 6 bits (at most 37 tables)
+  // vdW table of the centre with element e: byte e (at most 37 tables)
   const int ei = elc[cpi] & (TM_MAX_ELE - 1);
   unsigned long long vtab = 0;
   for (int e = 0; e < a.nele; ++e) {
     const int lo = min(ei, e), hi = max(ei, e);
-    vtab |= (unsigned long long)(1 + lo * a.nele - lo * (lo - 1) / 2 + (hi - lo)) << (6 * e);
+    vtab |= (unsigned long long)(1 + lo * a.nele - lo * (lo - 1) / 2 + (hi - lo)) << (8 * e);
   }
   ClAcc acc = {0.f, 0.f, 0.f, 0.f, 0.f};
   int qn = 0, qh = 0;   // queue length and head (0 or 64), wave-uniform
@@ -135,13 +154,18 @@ coulomb_tab_kernel(int N, const float4* __restrict__ xqc, const int* __restrict_
   auto begin = [&]() {
     const float4 d = qx[w][qh + lane];
     const int e = qe[w][qh + lane];
-    pair.begin(a, tab, ((unsigned)(vtab >> (6 * e)) & 63u) * (16u * (unsigned)a.nint), d);
+    const unsigned vo = __umul24((unsigned)(vtab >> (8 * e)) & 255u, 16u * (unsigned)a.nint);
+    if constexpr (LT) pair.begin(a, [&](unsigned byte) { return ltab[byte >> 4]; }, vo, d);
+    else pair.begin(a, [&](unsigned byte) { return ld16(tab, byte); }, vo, d);
   };
   struct Cand {
     float4 x;
     int e;
   };
-  auto load = [&](int p) { return Cand{ld16(xqc, 16u * (unsigned)p), elc[(unsigned)p]}; };
+  auto load = [&](int p) {
+    return Cand{ld16(xqc, 16u * (unsigned)p),
+                *reinterpret_cast<const int*>(reinterpret_cast<const char*>(elc) + 4u * (unsigned)p)};
+  };
   auto visit = [&](int p, bool valid, const Cand& c) {
     float4 d;
     d.x = c.x.x - pi.x;
@@ -153,13 +177,13 @@ coulomb_tab_kernel(int N, const float4* __restrict__ xqc, const int* __restrict_
       d.z = cl_min_image(d.z, Lz, iLz);
     }
     d.w = c.x.w;
-    // bitwise and: every test is evaluated, no branches
-    const bool ok = valid & (p != cpi) & (d.x * d.x + d.y * d.y + d.z * d.z < a.rc2);
-    const unsigned long long bal = __ballot(ok);
+    const bool near = d.x * d.x + d.y * d.y + d.z * d.z < a.rc2;
+    const bool ok = near && p != cpi && valid;
+    const unsigned long long bal = __builtin_amdgcn_ballot_w64(ok);
     if (ok) {
       const int q = (qh + qn + tm_lanes_below(bal)) & (CT_QCAP - 1);
       qx[w][q] = d;
-      qe[w][q] = c.e & (TM_MAX_ELE - 1);
+      qe[w][q] = (unsigned char)(c.e & (TM_MAX_ELE - 1));
     }
     qn += __popcll(bal);
     __syncwarp();
@@ -336,8 +360,11 @@ int tm_coulomb_tab(int N, const double* box, const int* cell_start, const int* c
   g.org[0] = (float)ox; g.org[1] = (float)oy; g.org[2] = (float)oz;
   g.periodic = periodic;
   tm_set_stencil(g, (float)rc_ee);
-  const auto k = periodic ? coulomb_tab_kernel<true> : coulomb_tab_kernel<false>;
-  k<<<tm_div_up(N, CT_WAVES), CT_WAVES * 64, 0, (hipStream_t)stream>>>(
+  const bool lt = ntab * nint <= CT_LDS_TABLE;
+  const auto k = periodic ? (lt ? coulomb_tab_kernel<true, true> : coulomb_tab_kernel<true, false>)
+                          : (lt ? coulomb_tab_kernel<false, true> : coulomb_tab_kernel<false, false>);
+  const int waves = lt ? CtShape<true>::WAVES : CtShape<false>::WAVES;
+  k<<<tm_div_up(N, waves), waves * 64, 0, (hipStream_t)stream>>>(
       N, (const float4*)xqc, elc, box, g, a, (const float4*)table, phi, grad, eatom);
   TM_LAUNCH_CHECK();
   return TM_OK;
