@@ -415,7 +415,7 @@ def run_train(args):
         "fp32_mlp": {k_: (round(v, 4) if isinstance(v, float) else v) for k_, v in out["fp32"].items()},
         "loss_first_last_bf16": [out["bf16"]["loss_first"], out["bf16"]["loss_last"]],
         "weight_grad_rel_err_vs_fp64": errs,
-        "roofline": {"bound": "mfma", "kernel": "gemm_bf16_kernel",
+        "roofline": {"bound": "mfma", "kernel": "gemm_wide_kernel",
                      "achieved": round(gtf, 2), "peak": 2500.0, "unit": "TFLOP/s",
                      "frac": round(gtf / 2500.0, 4), "traffic": None,
                      "flops_per_step": bf["gemm_flops_per_step"],
