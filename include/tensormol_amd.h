@@ -104,6 +104,16 @@ int tm_sym_forward(int N, const double* pos, const double* box, const int* mol, 
                    float eta, float zeta, float rr, float ra, const float* rs_r,
                    const float* rs_a, const float* thetas, float* G, int ldg, int* rev,
                    int* flags, void* stream);
+/* tm_sym_forward that also writes each atom's descriptors as a BF16 row (to
+ * nearest even) at the address places[4 i]; places: device int64 [N][4] =
+ * addresses of atom i's BF16 descriptor row, its BF16 tangent row, its float and
+ * its BF16 slot of dLoss/dy (the last three written by tm_sym_jvp_rows). */
+int tm_sym_forward_rows(int N, const double* pos, const double* box, const int* mol, const int* elem,
+                   const int* nbr, const int* ncnt, const int* rseg, const int* ang,
+                   const int* acnt, const int* aseg, int ldr, int lda, int nele, int nr,
+                   float eta, float zeta, float rr, float ra, const float* rs_r,
+                   const float* rs_a, const float* thetas, float* G, int ldg, int* rev,
+                   int* flags, const long* places, void* stream);
 
 /* Descriptor adjoint (replaces tf.gradients through the descriptor graph,
  * TFMolInstanceDirect.py:5761): with g_i = gE_i + u_i * gQ_i (gQ may be NULL),
@@ -134,6 +144,14 @@ int tm_sym_jvp(int N, const double* pos, const double* box, const int* mol, cons
                const int* aseg, int ldr, int lda, int nele, int nr, float eta, float zeta,
                float rr, float ra, const float* rs_r, const float* rs_a, const float* thetas,
                const double* du, float* V, int ldg, void* stream);
+/* tm_sym_jvp with the tangent as BF16 rows and ybar [N] copied to its slots
+ * (places as in tm_sym_forward_rows); no float V. */
+int tm_sym_jvp_rows(int N, const double* pos, const double* box, const int* mol, const int* elem,
+               const int* nbr, const int* ncnt, const int* rseg, const int* ang, const int* acnt,
+               const int* aseg, int ldr, int lda, int nele, int nr, float eta, float zeta,
+               float rr, float ra, const float* rs_r, const float* rs_a, const float* thetas,
+               const double* du, const float* ybar, const long* places,
+                    void* stream);
 
 /* ---- training-step MLP kernels ------------------------------------------
  * The MLP half of the force-matching step's second-order graph

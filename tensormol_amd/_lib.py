@@ -27,9 +27,11 @@ SIGNATURES = {
     "tm_triples": [I, I, I, I, P, P, P, P, P, P, P],
     "tm_pairs": [I, P, P, P, P, P, P, P, P, P, P, P, I, I, I, D, D, D, D, D, D, I, D, D, I, P, P, P, P, P],
     "tm_sym_forward": [I, P, P, P, P, P, P, P, P, P, P, I, I, I, I, F, F, F, F, P, P, P, P, I, P, P, P],
+    "tm_sym_forward_rows": [I, P, P, P, P, P, P, P, P, P, P, I, I, I, I, F, F, F, F, P, P, P, P, I, P, P, P, P],
     "tm_sym_adjoint": [I, P, P, P, P, P, P, P, P, P, P, I, I, I, I, F, F, F, F, P, P, P, P, P, P,
                        P, P, I, P, P],
     "tm_sym_jvp": [I, P, P, P, P, P, P, P, P, P, P, I, I, I, I, F, F, F, F, P, P, P, P, P, I, P],
+    "tm_sym_jvp_rows": [I, P, P, P, P, P, P, P, P, P, P, I, I, I, I, F, F, F, F, P, P, P, P, P, P, P],
     "tm_force_gather": [I, I, P, P, P, P, D, P, P, P],
     "tm_force_gather_sums": [I, I, P, P, P, P, D, P, P, I, P, I, P, P, P, P, P, P, P],
     "tm_total_energy": [I, P, P, P, P],

@@ -207,10 +207,9 @@ __device__ __forceinline__ float group_sum8(const float (&v)[8], int g) {
 // 76 -> 64; descriptors of 10,398 chain atoms 61 -> 36 and their tangent
 // 74 -> 47.  Reading the next pair's first triples ahead and keeping the pairs'
 // ranges per lane gained nothing.
-template <class Stage, class Term>
+template <class Out, class Stage, class Term>
 __device__ __forceinline__ void angular_pass(int lane, int nele, int nelep, int av, int ntrip,
-                                             float scale, float* __restrict__ out, Stage stage,
-                                             Term term) {
+                                             float scale, Out put, Stage stage, Term term) {
   const int g = lane & 7;
   float acc[NA];
 #pragma unroll
@@ -262,17 +261,30 @@ __device__ __forceinline__ void angular_pass(int lane, int nele, int nelep, int 
 #pragma unroll
         for (int s = 0; s < NA; ++s) acc[s] = 0.f;
       }
-      out[p * 64 + lane] = scale * x;
+      put(p * 64 + lane, scale * x);
       T = Te;
       ++p;
       if (++eb == nele) eb = ++ea;
     }
     __syncwarp();
   }
-  for (; p < nelep; ++p) out[p * 64 + lane] = 0.f;
+  for (; p < nelep; ++p) put(p * 64 + lane, 0.f);
 }
 
-template <int ZI, int RC>
+// A training step's GEMMs read descriptors and tangents as BF16 rows in element
+// order.  With ROWS the kernels below write those rows themselves (rounded to
+// nearest even): places[4 i ..] = addresses of atom i's descriptor row, its
+// tangent row, its float and its BF16 slot of dLoss/dy.
+// Copying them from FP32 arrays afterwards took launches of 15 and 11 us on
+// 10,398 atoms with 768 descriptors, bound by memory, where these kernels are
+// bound by instructions and have the bandwidth to spare: training step 600 ->
+// 576 us.  The descriptors are written in FP32 as well, for whoever reads them.
+__device__ __forceinline__ unsigned short bf16_of(float x) {
+  return __builtin_bit_cast(unsigned short, (__bf16)x);
+}
+
+
+template <int ZI, int RC, bool ROWS>
 __global__ void __launch_bounds__(SYM_WAVES * 64)
 sym_fwd_kernel(int N, const double* __restrict__ pos, const double* __restrict__ box,
                const int* __restrict__ mol, const int* __restrict__ elem,
@@ -280,7 +292,7 @@ sym_fwd_kernel(int N, const double* __restrict__ pos, const double* __restrict__
                const int* __restrict__ rseg, const int* __restrict__ ang,
                const int* __restrict__ acnt, const int* __restrict__ aseg, int ldr, int lda,
                SymArgs a, float* __restrict__ G, int ldg, int* __restrict__ rev,
-               int* __restrict__ flags) {
+               int* __restrict__ flags, const long* __restrict__ places) {
   __shared__ RowLdsFwd<RC> L;
   __shared__ float4 tq[SYM_WAVES][64];        // per triple: (cos theta, sin theta, fc_j fc_k, -)
   __shared__ float4 tR[SYM_WAVES][64][NA / 4];   // per triple: exp(-eta (ravg - Rs_s)^2), s = 0..7
@@ -299,6 +311,12 @@ sym_fwd_kernel(int N, const double* __restrict__ pos, const double* __restrict__
   load_row<RC>(i, w, lane, pos, box, mol, jq, n, a, L, [](int, int, const float4&) {});
   __syncwarp();
   float* Gi = G + (long)i * ldg;
+  unsigned short* Xi = nullptr;
+  if constexpr (ROWS) Xi = reinterpret_cast<unsigned short*>(places[4l * i]);
+  auto put = [&](int f, float v) {
+    Gi[f] = v;
+    if constexpr (ROWS) Xi[f] = bf16_of(v);
+  };
   // ---------------- radial: lane = (half h, shell s)
   {
     const int h = lane >> 5, s = lane & 31;
@@ -315,7 +333,7 @@ sym_fwd_kernel(int N, const double* __restrict__ pos, const double* __restrict__
           acc += __expf(-a.eta * x * x) * L.fc[w][q];
         }
         acc += __shfl_xor(acc, 32, 64);
-        if (h == 0 && ss < a.nr) Gi[e * a.nr + ss] = acc;
+        if (h == 0 && ss < a.nr) put(e * a.nr + ss, acc);
       }
     }
   }
@@ -324,7 +342,8 @@ sym_fwd_kernel(int N, const double* __restrict__ pos, const double* __restrict__
   // theta point and adds it times R_s to the shells.
   const float ct = a.cos_t[lane >> 3], st = a.sin_t[lane >> 3];
   angular_pass(
-      lane, a.nele, a.nelep, av, m * (m - 1) / 2, a.two_1mz, Gi + a.nele * a.nr,
+      lane, a.nele, a.nelep, av, m * (m - 1) / 2, a.two_1mz,
+      [&](int f, float v) { put(a.nele * a.nr + f, v); },
       [&](int ja, int kb) {
         const int qj = apos[w][ja], qk = apos[w][kb];
         float4 dj = L.d[w][qj], dk = L.d[w][qk];
@@ -733,14 +752,15 @@ struct JvpLds {
   float dfc[SYM_WAVES][RC];    // d fc_r / dr
 };
 
-template <int ZI, int RC>
+template <int ZI, int RC, bool ROWS>
 __global__ void __launch_bounds__(SYM_WAVES * 64)
 sym_jvp_kernel(int N, const double* __restrict__ pos, const double* __restrict__ box,
                const int* __restrict__ mol, const int* __restrict__ elem,
                const int* __restrict__ nbr, const int* __restrict__ ncnt,
                const int* __restrict__ rseg, const int* __restrict__ ang,
                const int* __restrict__ acnt, const int* __restrict__ aseg, int ldr, int lda,
-               SymArgs a, const double* __restrict__ du, float* __restrict__ V, int ldg) {
+               SymArgs a, const double* __restrict__ du, float* __restrict__ V, int ldg,
+               const float* __restrict__ ybar, const long* __restrict__ places) {
   // the forward's row (the angular cutoff and its derivative are formed per
   // triple), which with the per-triple staging below fits 4 waves per SIMD
   __shared__ RowLdsFwd<RC> L;
@@ -769,7 +789,22 @@ sym_jvp_kernel(int N, const double* __restrict__ pos, const double* __restrict__
     T.dfc[w][q] = -0.5f * kr * __sinf(kr * d.w);
   });
   __syncwarp();
-  float* Vi = V + (long)i * ldg;
+  float* Vi = nullptr;
+  unsigned short* Xi = nullptr;
+  if constexpr (ROWS) {
+    Xi = reinterpret_cast<unsigned short*>(places[4l * i + 1]);
+    if (lane == 0) {
+      const float y = ybar[i];
+      *reinterpret_cast<float*>(places[4l * i + 2]) = y;
+      *reinterpret_cast<unsigned short*>(places[4l * i + 3]) = bf16_of(y);
+    }
+  } else {
+    Vi = V + (long)i * ldg;
+  }
+  auto put = [&](int f, float v) {
+    if constexpr (ROWS) Xi[f] = bf16_of(v);
+    else Vi[f] = v;
+  };
   // ---------------- radial: lane = (half h, shell s)
   {
     const int h = lane >> 5, s = lane & 31;
@@ -787,7 +822,7 @@ sym_jvp_kernel(int N, const double* __restrict__ pos, const double* __restrict__
                  T.t[w][q].w;
         }
         acc += __shfl_xor(acc, 32, 64);
-        if (h == 0 && ss < a.nr) Vi[e * a.nr + ss] = acc;
+        if (h == 0 && ss < a.nr) put(e * a.nr + ss, acc);
       }
     }
   }
@@ -799,7 +834,8 @@ sym_jvp_kernel(int N, const double* __restrict__ pos, const double* __restrict__
   // tangents of cos theta, ravg and fc_j fc_k).
   const float ct = a.cos_t[lane >> 3], st = a.sin_t[lane >> 3];
   angular_pass(
-      lane, a.nele, a.nelep, av, m * (m - 1) / 2, a.two_1mz, Vi + a.nele * a.nr,
+      lane, a.nele, a.nelep, av, m * (m - 1) / 2, a.two_1mz,
+      [&](int f, float v) { put(a.nele * a.nr + f, v); },
       [&](int ja, int kb) {
         const int qj = apos[w][ja], qk = apos[w][kb];
         float4 dj = L.d[w][qj], dk = L.d[w][qk];
@@ -873,16 +909,13 @@ int fill_args(SymArgs& a, int nele, int nr, float eta, float zeta, float rr, flo
 
 }  // namespace
 
-extern "C" {
-
-// Host-side parameter arrays (rs_r[nr], rs_a[8], thetas[8]) are read on the
-// host and passed to the kernels by value.
-int tm_sym_forward(int N, const double* pos, const double* box, const int* mol, const int* elem,
+template <bool ROWS>
+static int sym_forward(int N, const double* pos, const double* box, const int* mol, const int* elem,
                    const int* nbr, const int* ncnt, const int* rseg, const int* ang,
                    const int* acnt, const int* aseg, int ldr, int lda, int nele, int nr,
                    float eta, float zeta, float rr, float ra, const float* rs_r,
                    const float* rs_a, const float* thetas, float* G, int ldg, int* rev,
-                   int* flags, void* stream) {
+                   int* flags, const long* places, void* stream) {
   SymArgs a;
   int st = fill_args(a, nele, nr, eta, zeta, rr, ra, rs_r, rs_a, thetas);
   if (st) return st;
@@ -893,13 +926,64 @@ int tm_sym_forward(int N, const double* pos, const double* box, const int* mol, 
   if (N == 0) return TM_OK;
   hipStream_t s = (hipStream_t)stream;
   // rows up to 128 entries stage in the smaller LDS layout (more waves per CU)
-  auto k = ldr <= 128 ? (a.zeta_int == 8 ? sym_fwd_kernel<8, 128> : sym_fwd_kernel<0, 128>)
-                      : (a.zeta_int == 8 ? sym_fwd_kernel<8, 256> : sym_fwd_kernel<0, 256>);
+  decltype(&sym_fwd_kernel<0, 128, ROWS>) k =
+      ldr <= 128 ? (a.zeta_int == 8 ? sym_fwd_kernel<8, 128, ROWS> : sym_fwd_kernel<0, 128, ROWS>)
+                 : (a.zeta_int == 8 ? sym_fwd_kernel<8, 256, ROWS> : sym_fwd_kernel<0, 256, ROWS>);
   k<<<tm_div_up(N, SYM_WAVES), SYM_WAVES * 64, 0, s>>>(N, pos, box, mol, elem, nbr, ncnt, rseg,
                                                        ang, acnt, aseg, ldr, lda, a, G, ldg, rev,
-                                                       flags);
+                                                       flags, places);
   TM_LAUNCH_CHECK();
   return TM_OK;
+}
+
+template <bool ROWS>
+static int sym_jvp(int N, const double* pos, const double* box, const int* mol, const int* elem,
+               const int* nbr, const int* ncnt, const int* rseg, const int* ang, const int* acnt,
+               const int* aseg, int ldr, int lda, int nele, int nr, float eta, float zeta,
+               float rr, float ra, const float* rs_r, const float* rs_a, const float* thetas,
+               const double* du, float* V, int ldg,
+               const float* ybar, const long* places, void* stream) {
+  SymArgs a;
+  int st = fill_args(a, nele, nr, eta, zeta, rr, ra, rs_r, rs_a, thetas);
+  if (st) return st;
+  TM_REQUIRE(ROWS || ldg >= a.D, "tm_sym_jvp: ldg %d < D %d", ldg, a.D);
+  TM_REQUIRE(ldr > 0 && ldr <= MAX_ROW && lda > 0 && lda <= ldr,
+             "tm_sym_jvp: strides %d/%d (need 0 < lda <= ldr <= %d)", ldr, lda, MAX_ROW);
+  if (N == 0) return TM_OK;
+  hipStream_t s = (hipStream_t)stream;
+  decltype(&sym_jvp_kernel<0, 128, ROWS>) k =
+      ldr <= 128 ? (a.zeta_int == 8 ? sym_jvp_kernel<8, 128, ROWS> : sym_jvp_kernel<0, 128, ROWS>)
+                 : (a.zeta_int == 8 ? sym_jvp_kernel<8, 256, ROWS> : sym_jvp_kernel<0, 256, ROWS>);
+  k<<<tm_div_up(N, SYM_WAVES), SYM_WAVES * 64, 0, s>>>(N, pos, box, mol, elem, nbr, ncnt, rseg,
+                                                       ang, acnt, aseg, ldr, lda, a, du, V, ldg,
+                                                       ybar, places);
+  TM_LAUNCH_CHECK();
+  return TM_OK;
+}
+
+extern "C" {
+
+// Host-side parameter arrays (rs_r[nr], rs_a[8], thetas[8]) are read on the
+// host and passed to the kernels by value.
+int tm_sym_forward(int N, const double* pos, const double* box, const int* mol, const int* elem,
+                   const int* nbr, const int* ncnt, const int* rseg, const int* ang,
+                   const int* acnt, const int* aseg, int ldr, int lda, int nele, int nr,
+                   float eta, float zeta, float rr, float ra, const float* rs_r,
+                   const float* rs_a, const float* thetas, float* G, int ldg, int* rev,
+                   int* flags, void* stream) {
+  return sym_forward<false>(N, pos, box, mol, elem, nbr, ncnt, rseg, ang, acnt, aseg, ldr, lda, nele, nr, eta,
+                     zeta, rr, ra, rs_r, rs_a, thetas, G, ldg, rev, flags, nullptr, stream);
+}
+
+int tm_sym_forward_rows(int N, const double* pos, const double* box, const int* mol, const int* elem,
+                   const int* nbr, const int* ncnt, const int* rseg, const int* ang,
+                   const int* acnt, const int* aseg, int ldr, int lda, int nele, int nr,
+                   float eta, float zeta, float rr, float ra, const float* rs_r,
+                   const float* rs_a, const float* thetas, float* G, int ldg, int* rev,
+                   int* flags, const long* places, void* stream) {
+  TM_REQUIRE(places != nullptr, "tm_sym_forward_rows: places missing");
+  return sym_forward<true>(N, pos, box, mol, elem, nbr, ncnt, rseg, ang, acnt, aseg, ldr, lda, nele, nr, eta,
+                     zeta, rr, ra, rs_r, rs_a, thetas, G, ldg, rev, flags, places, stream);
 }
 
 int tm_sym_adjoint(int N, const double* pos, const double* box, const int* mol, const int* elem,
@@ -937,20 +1021,19 @@ int tm_sym_jvp(int N, const double* pos, const double* box, const int* mol, cons
                const int* aseg, int ldr, int lda, int nele, int nr, float eta, float zeta,
                float rr, float ra, const float* rs_r, const float* rs_a, const float* thetas,
                const double* du, float* V, int ldg, void* stream) {
-  SymArgs a;
-  int st = fill_args(a, nele, nr, eta, zeta, rr, ra, rs_r, rs_a, thetas);
-  if (st) return st;
-  TM_REQUIRE(ldg >= a.D, "tm_sym_jvp: ldg %d < D %d", ldg, a.D);
-  TM_REQUIRE(ldr > 0 && ldr <= MAX_ROW && lda > 0 && lda <= ldr,
-             "tm_sym_jvp: strides %d/%d (need 0 < lda <= ldr <= %d)", ldr, lda, MAX_ROW);
-  if (N == 0) return TM_OK;
-  hipStream_t s = (hipStream_t)stream;
-  auto k = ldr <= 128 ? (a.zeta_int == 8 ? sym_jvp_kernel<8, 128> : sym_jvp_kernel<0, 128>)
-                      : (a.zeta_int == 8 ? sym_jvp_kernel<8, 256> : sym_jvp_kernel<0, 256>);
-  k<<<tm_div_up(N, SYM_WAVES), SYM_WAVES * 64, 0, s>>>(N, pos, box, mol, elem, nbr, ncnt, rseg,
-                                                       ang, acnt, aseg, ldr, lda, a, du, V, ldg);
-  TM_LAUNCH_CHECK();
-  return TM_OK;
+  return sym_jvp<false>(N, pos, box, mol, elem, nbr, ncnt, rseg, ang, acnt, aseg, ldr, lda, nele, nr, eta,
+                     zeta, rr, ra, rs_r, rs_a, thetas, du, V, ldg, nullptr, nullptr, stream);
+}
+
+int tm_sym_jvp_rows(int N, const double* pos, const double* box, const int* mol, const int* elem,
+               const int* nbr, const int* ncnt, const int* rseg, const int* ang, const int* acnt,
+               const int* aseg, int ldr, int lda, int nele, int nr, float eta, float zeta,
+               float rr, float ra, const float* rs_r, const float* rs_a, const float* thetas,
+               const double* du, const float* ybar, const long* places,
+                    void* stream) {
+  TM_REQUIRE(ybar != nullptr && places != nullptr, "tm_sym_jvp_rows: ybar or places missing");
+  return sym_jvp<true>(N, pos, box, mol, elem, nbr, ncnt, rseg, ang, acnt, aseg, ldr, lda, nele, nr, eta,
+                     zeta, rr, ra, rs_r, rs_a, thetas, du, nullptr, 0, ybar, places, stream);
 }
 
 int tm_force_gather(int N, int ldr, const int* ncnt, const int* rev, const float* wslot,

@@ -523,6 +523,33 @@ class BPEEEngine:
                             sym.ra, _lib.fptr(self.sym_rs_r), _lib.fptr(self.sym_rs_a),
                             _lib.fptr(self.sym_th), _P(du), _P(out), self.D, self._stream())
 
+    def _sym_args(self, ws, pos):
+        """Leading arguments of the descriptor launches."""
+        sym = self.model.sym
+        return (ws.N, _P(pos), _P(ws.box), _P(ws.mol), _P(ws.elem), _P(ws.nbr), _P(ws.ncnt),
+                _P(ws.rseg), _P(ws.ang), _P(ws.acnt), _P(ws.aseg), self.ldr, self.lda, self.nele,
+                sym.nr_r, sym.eta, sym.zeta, sym.rr, sym.ra, _lib.fptr(self.sym_rs_r),
+                _lib.fptr(self.sym_rs_a), _lib.fptr(self.sym_th))
+
+    def descriptor_rows(self, ws, pos, places):
+        """descriptors() that also writes them as BF16 rows to the addresses
+        places[:, 0] (cuda int64 [N, 4], see tm_sym_forward_rows)."""
+        assert places.dtype == torch.int64 and places.is_contiguous()
+        assert places.shape[0] >= ws.N and places.shape[1] == 4
+        self.lib.tm_sym_forward_rows(*self._sym_args(ws, pos), _P(ws.G), self.D, _P(ws.rev),
+                                     _P(ws.flags), _P(places), self._stream())
+        ws.rev_ok = True
+
+    def descriptor_jvp_rows(self, ws, pos, du, ybar, places):
+        """descriptor_jvp() as BF16 rows at places[:, 1], with ybar (cuda float32
+        [N]) copied to places[:, 2] (float32) and places[:, 3] (BF16)."""
+        assert du.dtype == torch.float64 and du.is_contiguous() and du.shape[0] >= ws.N
+        assert ybar.dtype == torch.float32 and ybar.is_contiguous() and ybar.numel() >= ws.N
+        assert places.dtype == torch.int64 and places.is_contiguous()
+        assert places.shape[0] >= ws.N and places.shape[1] == 4
+        self.lib.tm_sym_jvp_rows(*self._sym_args(ws, pos), _P(du), _P(ybar), _P(places),
+                                 self._stream())
+
     def descriptor_vjp(self, ws, pos, gE, grad):
         """grad[:N] = (dG/dx)^T gE: the per-atom gradient of sum_i gE_i . G_i
         (gE cuda float32 [N, D]); the BP-only adjoint (no charge branch)."""

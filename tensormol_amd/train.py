@@ -245,6 +245,15 @@ class ForceMatchingTrainer:
             b["nsplit"] = ns
             b["work"] = [torch.zeros(ns * (D + 1) * H, **f32), torch.zeros(ns * (H + 1) * H, **f32),
                          torch.zeros(ns * (H + 1) * H, **f32), torch.zeros(ns * (H + 1), **f32)]
+        # where the descriptor kernels write each atom's rows and dLoss/dy
+        places = torch.zeros(tb.N, 4, dtype=torch.int64, device=dev)
+        for e, b in bufs.items():
+            k = torch.arange(b["M"], dtype=torch.int64, device=dev)
+            places[tb.idx[e]] = torch.stack(
+                [b["X0"].data_ptr() + 2 * ldx * k, b["X0"].data_ptr() + 2 * ldx * (b["M"] + k),
+                 b["YB"].data_ptr() + 4 * k, b["YBb"].data_ptr() + 2 * k], dim=1)
+        assert sum(b["M"] for b in bufs.values()) == tb.N
+        tb._places = places
         tb._mfma = bufs
         return bufs
 
@@ -283,9 +292,10 @@ class ForceMatchingTrainer:
         eng.build_lists(ws, pos)
         if check:
             eng.check_flags(ws)
-        eng.descriptors(ws, pos)
         N, D = tb.N, eng.D
         bufs = self._mfma_buffers(tb)
+        # descriptors, and their rows as BF16 in element order (rows ..M of X0)
+        eng.descriptor_rows(ws, pos, tb._places)
         items = [(b, self.params[e]) for e, b in bufs.items()]
         H = items[0][0]["H"]
         ad = lambda t, rows=0, ld=0: t.data_ptr() + t.element_size() * rows * ld   # row `rows`
@@ -294,11 +304,9 @@ class ForceMatchingTrainer:
         # per-element GEMMs below write every row of these through their row maps
         eps = torch.empty(N, 1, **f32)
         J = torch.empty(N, D, **f32)
-        # this step's weights and the descriptors' rows as BF16, in one launch
+        # this step's weights as BF16, in one launch
         whole = lambda W: (1, W.numel()) if W.shape[1] == 1 else tuple(W.shape)
-        self._grows([(b["M"], D, ad(b["idx"]), ad(ws.G), D, ad(b["X0"]), b["ldx"], 1)
-                     for b, _ in items] +
-                    [(*whole(W), None, ad(W), whole(W)[1], ad(Wb), whole(W)[1], 1)
+        self._grows([(*whole(W), None, ad(W), whole(W)[1], ad(Wb), whole(W)[1], 1)
                      for b, prm in items for (W, _), Wb in zip(prm, b["Wb"])], 0)
         # forward: z_l = h_{l-1} W_l + b_l, h_l = act(z_l), s_l = act'(z_l); the
         # last layer also starts the J chain, zd_3 = s_3 w_4 (rows M.. of ZZ3)
@@ -343,13 +351,8 @@ class ForceMatchingTrainer:
                            eng._stream())
         L = Lt[0]
         F = None if views else -grad   # step() has no use for the forces
-        V = torch.empty(N, D, **f32)
-        eng.descriptor_jvp(ws, pos, gg, V)
-        self._grows([(b["M"], D, ad(b["idx"]), ad(V), D, ad(b["X0"], b["M"], b["ldx"]), b["ldx"],
-                      1) for b, _ in items] +
-                    [(b["M"], 1, ad(b["idx"]), ad(ybar), 1, ad(b["YB"]), 1, 0) for b, _ in items] +
-                    [(b["M"], 1, ad(b["idx"]), ad(ybar), 1, ad(b["YBb"]), 1, 1) for b, _ in items],
-                    0)
+        # the tangent V as rows M.. of X0, ybar as YB and rows ..M of YBb
+        eng.descriptor_jvp_rows(ws, pos, gg, ybar, tb._places)
         # tangent along V: zt_l = ht_{l-1} W_l, ht_l = s_l zt_l (rows M.. of H_l);
         # the last layer also starts the reverse pass,
         # zb_3 = s_3 ybar w_4 + a s_3 (1 - s_3) zt_3 w_4 (rows ..M of ZZ3)
