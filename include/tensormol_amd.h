@@ -50,6 +50,12 @@ int tm_cell_build(int N, const double* pos, const int* mol, double ox, double oy
                   double cx, double cy, double cz, int nx, int ny, int nz, int periodic,
                   int* cell_of, int* cell_count, int* cell_start, int* cell_fill, int* cell_atoms,
                   int* cell_pos, double* posc, int* molc, int* flags, void* stream);
+/* tm_zero_i32(8, flags) and tm_cell_build without a launch for the clearing:
+ * flags (8 ints) then hold what this build raised. */
+int tm_cell_build_fresh(int N, const double* pos, const int* mol, double ox, double oy, double oz,
+                  double cx, double cy, double cz, int nx, int ny, int nz, int periodic,
+                  int* cell_of, int* cell_count, int* cell_start, int* cell_fill, int* cell_atoms,
+                  int* cell_pos, double* posc, int* molc, int* flags, void* stream);
 
 /* Builds, for every atom i, the full (DoPerms=1) list of neighbours j with
  * squared distance s < s_r and marks those with s < s_a.  s_r/s_a are the

@@ -22,6 +22,7 @@ SIGNATURES = {
     "tm_version": [],
     "tm_zero_i32": [I, P, P],
     "tm_cell_build": [I, P, P, D, D, D, D, D, D, I, I, I, I, P, P, P, P, P, P, P, P, P, P],
+    "tm_cell_build_fresh": [I, P, P, D, D, D, D, D, D, I, I, I, I, P, P, P, P, P, P, P, P, P, P],
     "tm_nl_build": [I, P, P, P, P, P, P, P, P, P, P, P, I, I, I, D, D, D, D, D, D, I, I, D, D, D, I, I, P, P, P,
                     P, P, P, P, P, P],
     "tm_triples": [I, I, I, I, P, P, P, P, P, P, P],

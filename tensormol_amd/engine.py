@@ -337,7 +337,7 @@ class BPEEEngine:
         accumulate them, and a check after the replay sees every step's."""
         key = (pos.data_ptr(), self._raw_stream())
         ws.rev_ok = False   # the mirror slots are filled by the next descriptor forward
-        if clear_flags:
+        if clear_flags and not ws.use_cells:
             self._call(ws, "tm_zero_i32", key, lambda: (8, _P(ws.flags), self._stream()))
         if ws.use_cells:
             def cell_args():
@@ -346,7 +346,8 @@ class BPEEEngine:
                         n[2], ws.periodic, _P(ws.cell_of), _P(ws.cell_count), _P(ws.cell_start),
                         _P(ws.cell_fill), _P(ws.cell_atoms), _P(ws.cell_pos), _P(ws.posc),
                         _P(ws.molc), _P(ws.flags), self._stream())
-            self._call(ws, "tm_cell_build", key, cell_args)
+            self._call(ws, "tm_cell_build_fresh" if clear_flags else "tm_cell_build", key,
+                       cell_args)
         self._call(ws, "tm_nl_build", key, lambda: (
             ws.N, _P(pos), _P(ws.elem), _P(ws.mol), _P(ws.mol_start), _P(ws.box),
             *self._grid_args(ws), ws.periodic, self.nele, self.model.sym.rr, self.s_r, self.s_a,
