@@ -68,6 +68,28 @@ def xcd_order(til):
     return out
 
 
+def with_readers(til, ncu):
+    """An XCD-ordered table with one reader per XCD and weight blob appended
+    (segment -2 - s: the workgroup only streams the weights of segment s into
+    its XCD's L2, ahead of the tiles), where tiles and readers have a CU each.
+    Past that the readers would take turns with tiles, and enough tiles share
+    a blob that they read ahead for each other."""
+    if len(til) == 0:
+        return til
+    s = til[:, 0].reshape(-1, NXCD)
+    new = s >= 0
+    new[1:] &= s[1:] != s[:-1]                     # a run's tiles are sorted by segment
+    k = np.cumsum(new, axis=0)
+    c = int(k[-1].max())
+    if len(til) + c * NXCD > ncu:
+        return til
+    out = np.zeros((c, NXCD, 2), dtype=np.int32)
+    out[:, :, 0] = -1
+    t, x = np.nonzero(new)
+    out[k[t, x] - 1, x, 0] = -2 - s[t, x]
+    return np.concatenate([til, out.reshape(-1, 2)])
+
+
 class MFMAWeights:
     def __init__(self, engine, precision):
         if precision not in MODES:
@@ -149,7 +171,7 @@ class MFMAWeights:
         halves[1::2, 1] += 32
         rows = seg[halves[:, 0], 3] if len(halves) else np.zeros(0, np.int32)
         t32 = halves[halves[:, 1] < rows] if len(halves) else halves
-        t64x, t32x = xcd_order(head), xcd_order(t32)
+        t64x, t32x = xcd_order(head), with_readers(xcd_order(t32), self.ncu)
         if upload is None:
             dev = self.engine.device
             upload = lambda a, out=None: torch.from_numpy(a).to(dev)
