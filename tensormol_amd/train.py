@@ -284,8 +284,9 @@ class ForceMatchingTrainer:
     def _mfma_step(self, tb, pos, check=True, views=False):
         """(L, E, F, gradients in parameters() order) of the BF16 MFMA path.
         Each GEMM stage runs for every element in one grouped launch, with
-        the elementwise steps between them in the GEMM epilogues; the row
-        gathers and scatters of every element also take one launch each.
+        the elementwise steps between them in the GEMM epilogues; descriptors
+        and tangents come as BF16 rows in element order from their kernels, and
+        J and the atom energies leave through row maps.
         views=True returns the gradients as views of the batch's buffers (the
         next step overwrites them) instead of copies."""
         eng, ws = self.eng, tb.ws
