@@ -86,7 +86,7 @@ struct RangeLds {
   int mark[64];   // range starts inside the current chunk, tagged with the chunk's base
 };
 
-// A centre's cell and its offset inside the cell.
+// A centre's cell and its offset inside the cell, in [0, cs] on an open grid.
 struct CellCentre {
   int c[3];
   float f[3];
@@ -106,7 +106,14 @@ __device__ __forceinline__ CellCentre tm_centre(const CellGrid& g, int cell, dou
     // wrapped in FP64, so unwrapped coordinates keep their precision; the
     // offset lies within a cell of a multiple of the length, so the nearest one is it
     if (g.periodic && g.nc[d] >= 3) u -= g.len[d] * rint(u * g.inv_len[d]);
-    o.f[d] = (float)u;   // offset inside the centre's cell
+    float f = (float)u;   // offset inside the centre's cell
+    // A centre outside an open grid sits in an edge cell: it is taken to that
+    // cell's face.  Taking centre and candidate into the grid never makes them
+    // further apart, so with the centre there all distances to bands of cells
+    // and the range along x bound the true ones from below; its own band, for
+    // one, can hold atoms that are as far outside.
+    if (!g.periodic) f = fminf(fmaxf(f, 0.f), g.cs[d]);
+    o.f[d] = f;
   }
   return o;
 }
