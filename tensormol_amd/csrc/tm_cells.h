@@ -45,8 +45,10 @@ constexpr float TM_TRIM_MARGIN = 2e-3f;
 
 // Stencil of cutoff rc over the grid.  Computed once per launch: with the
 // integer divisions and the ceilings of a cutoff in cells it cost each wave
-// about half of its instructions per 64 rows.
+// about half of its instructions per 64 rows.  Without a grid its sizes mean
+// nothing (callers may pass zeros) and are not looked at.
 inline void tm_set_stencil(CellGrid& g, float rc) {
+  if (g.cell_atoms == nullptr) return;
   for (int d = 0; d < 3; ++d) {
     // a band further out is at least ceil(rc / cs) cells away.  An axis counts
     // as wrapped two bands before it is, which decides the order of its rows
@@ -58,7 +60,7 @@ inline void tm_set_stencil(CellGrid& g, float rc) {
   }
   g.ny = g.full[1] ? g.nc[1] : 2 * g.k[1] + 1;
   g.nrow = g.ny * (g.full[2] ? g.nc[2] : 2 * g.k[2] + 1);
-  g.magic = (unsigned)((0x100000000ull + (unsigned)g.ny - 1) / (unsigned)g.ny);
+  g.magic = g.ny > 1 ? (unsigned)((0x100000000ull + (unsigned)g.ny - 1) / (unsigned)g.ny) : 0u;
   const float rcm = rc + TM_TRIM_MARGIN;
   g.rc2 = rcm * rcm;
   g.inv_cs0 = 1.0f / g.cs[0];

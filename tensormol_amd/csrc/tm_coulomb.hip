@@ -701,7 +701,7 @@ int tm_coulomb(int N, const float* xq, const int* elem, const int* mol, const in
   }
   if (N == 0) return TM_OK;
   const CoulArgs a = coul_args(consts, rc_ee, width, add_ecc, has_vdw, nele, c6, r0);
-  CellGrid g;
+  CellGrid g{};
   g.cell_start = cell_start; g.cell_atoms = cell_atoms; g.cell_of = cell_of;
   g.cell_pos = cell_pos; g.posc = nullptr; g.molc = molc;
   g.nc[0] = nx; g.nc[1] = ny; g.nc[2] = nz;

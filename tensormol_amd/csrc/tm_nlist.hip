@@ -562,7 +562,7 @@ static CellGrid make_grid(const int* cell_start, const int* cell_atoms, const in
                           const int* cell_pos, const double* posc, const int* molc, int nx, int ny,
                           int nz, double csx, double csy, double csz, double ox, double oy,
                           double oz, int periodic, double rc) {
-  CellGrid g;
+  CellGrid g{};
   g.cell_start = cell_start; g.cell_atoms = cell_atoms; g.cell_of = cell_of;
   g.cell_pos = cell_pos; g.posc = posc; g.molc = molc;
   g.nc[0] = nx; g.nc[1] = ny; g.nc[2] = nz;
