@@ -32,6 +32,15 @@ _P = _lib.ptr
 # largest table (float4 entries, 48 KiB) the tabulated Coulomb sweep accepts
 CL_TABLE_ENTRIES = 3072
 
+# Batches of molecules whose Coulomb sweep forms the charges itself
+# (tm_coulomb_raw): up to this many candidates, sum n^2, plus 150 per atom.  It
+# saves two launches, some 7 us, but each candidate takes FP64 loads and each
+# atom a sum over its molecule.  Electrostatics from raw charges / from charges
+# formed first (us): 15 molecules of 256 atoms 11.2 / 17.6, 92 of 256 33.8 / 33.6,
+# 600 of 100 54.6 / 51.0, 10 of 1,000 38.0 / 37.8, 2 of 3,000 51.3 / 46.7, 6 of
+# 3,000 108 / 88.  Of 60 to 3,000 atoms the two meet between 8 and 11 million.
+RAW_SWEEP_WORK = 9_000_000
+
 
 def nl_threshold(rc):
     """First float64 s for which sqrt(s) + 1e-13 < rc is false (MolEmb.cpp:1214-1218).
@@ -188,7 +197,7 @@ class BPEEEngine:
         ws.Eext = torch.zeros(B, 2, **f64)
         ws.dipole = torch.zeros(B, 3, **f64)
         ws.mlp_ws = None
-        ws.use_cells = False
+        ws.use_cells = ws.raw_sweep = False
         return ws
 
     def set_topology(self, ws, Z, mol_start, boxes=None, margin=4.0, pos0=None, stager=None):
@@ -249,6 +258,8 @@ class BPEEEngine:
         ws.JQ = ws.J2[N * self.D:2 * N * self.D].view(N, self.D)
         # cell grid for one large system
         ws.use_cells = (B == 1 and N > 256)
+        sizes = np.diff(ms)
+        ws.raw_sweep = not ws.use_cells and int((sizes * sizes).sum()) + 150 * N <= RAW_SWEEP_WORK
         if ws.use_cells:
             self._setup_grid(ws, pos0, margin)
             ws.xqc = torch.zeros(max(1, N), 4, dtype=torch.float32, device=dev)
@@ -419,8 +430,8 @@ class BPEEEngine:
         (to record timing events on the launch stream)."""
         key = (pos.data_ptr(), self._raw_stream())
         st = self._stream
-        if not ws.use_cells:
-            # molecules: charges and sweep in one launch
+        if ws.raw_sweep:
+            # small molecules: charges and sweep in one launch
             add_ecc = int(bool(PARAMS["AddEcc"]))
             if timer is not None:
                 timer[0]()
@@ -437,13 +448,25 @@ class BPEEEngine:
                 ws.B, _P(ws.mol_start), 1, _P(ws.phi), 1, _P(ws.phimean), 1, _P(ws.red), ws.N,
                 st()))
             return
-        # One system (a cell grid is only set up for one): the mean of the raw
-        # charges is formed inside the charges launch (each block sums it), and
-        # charges are written straight into cell order for the sweep.
-        self._call(ws, "tm_charges", key, lambda: (
-            ws.N, _P(ws.mol), _P(ws.mol_start), _P(ws.qmean), _P(ws.qraw), _P(pos), None, _P(ws.q),
-            _P(ws.qx), _P(ws.cell_pos), _P(ws.elem), _P(ws.xqc), _P(ws.elc), st()))
-        table = self._cl_table() if self.coulomb_tables else None
+        # One system: the mean of the raw charges is formed inside the charges
+        # launch (each block sums it).  A batch of molecules takes one block per
+        # molecule in a reduction launch first instead, since a block would
+        # otherwise step through every molecule it touches.
+        ms = None
+        if ws.B == 1:
+            ms = ws.mol_start
+        else:
+            self._call(ws, "tm_mol_sum_f32", key, lambda: (
+                ws.B, _P(ws.mol_start), 1, _P(ws.qraw), 1, _P(ws.qmean), 1, _P(ws.red), ws.N, st()))
+        if ws.use_cells:   # charges written straight into cell order for the sweep
+            self._call(ws, "tm_charges", key, lambda: (
+                ws.N, _P(ws.mol), _P(ms), _P(ws.qmean), _P(ws.qraw), _P(pos), None, _P(ws.q),
+                _P(ws.qx), _P(ws.cell_pos), _P(ws.elem), _P(ws.xqc), _P(ws.elc), st()))
+        else:
+            self._call(ws, "tm_charges", key, lambda: (
+                ws.N, _P(ws.mol), _P(ms), _P(ws.qmean), _P(ws.qraw), _P(pos), _P(ws.xq), _P(ws.q),
+                _P(ws.qx), None, None, None, None, st()))
+        table = self._cl_table() if (ws.use_cells and self.coulomb_tables) else None
         if timer is not None:
             timer[0]()
         if table is not None:
@@ -459,7 +482,7 @@ class BPEEEngine:
 
             def coul_args():
                 g = self._grid_args(ws)
-                return (ws.N, None, _P(ws.elem), _P(ws.mol),
+                return (ws.N, None if ws.use_cells else _P(ws.xq), _P(ws.elem), _P(ws.mol),
                         _P(ws.mol_start), _P(ws.box), g[0], g[1], g[2], g[3], g[5], g[6], g[7],
                         g[8], g[9], g[10], g[11], g[12], g[13], g[14], ws.periodic,
                         self.dsf.ctypes.data_as(_lib.P), self.model.ee_off, self.vdw_width,
