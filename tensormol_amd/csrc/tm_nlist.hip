@@ -44,6 +44,15 @@ __device__ __forceinline__ double sq_dist_nocontract(double xi, double yi, doubl
   return s;
 }
 
+__device__ __forceinline__ double sq_dist_nocontract(double xi, double yi, double zi, double xj,
+                                                     double yj, double zj) {
+#pragma clang fp contract(off)
+  const double dx = xi - xj, dy = yi - yj, dz = zi - zj;
+  double s = dx * dx + dy * dy;
+  s = s + dz * dz;
+  return s;
+}
+
 // The same with the reciprocal edges (0 for open boundaries).  The image it
 // picks differs only where a separation is half an edge to the last digit, for
 // which the two images are equally far.
@@ -94,9 +103,12 @@ nl_rows_kernel(int N, const double* __restrict__ pos, const int* __restrict__ el
     iLz = Lz > 0.0 ? 1.0 / Lz : 0.0;
   }
   int count = 0;   // wave-uniform
-  // candidate j at (x, y, z); self and other molecules are not taken
+  // candidate j at (x, y, z); self and other molecules are not taken.  Without
+  // boxes the images' FP64 operations, half of a test, are left out.
   auto test = [&](double x, double y, double z, int j, bool take) {
-    const double s = sq_dist_nocontract(xi, yi, zi, x, y, z, Lx, Ly, Lz, iLx, iLy, iLz);
+    const double s = box != nullptr
+                         ? sq_dist_nocontract(xi, yi, zi, x, y, z, Lx, Ly, Lz, iLx, iLy, iLz)
+                         : sq_dist_nocontract(xi, yi, zi, x, y, z);
     const bool ok = take & (s < s_r);
     const unsigned long long bal = __ballot(ok);
     const int slot = count + tm_lanes_below(bal);
