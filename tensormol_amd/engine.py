@@ -649,6 +649,9 @@ class BPEEEngine:
 
     def energy_tensor(self, ws):
         """Per-molecule total energy as a device tensor (no host copy)."""
+        if not ws.Ebp.is_cuda or torch.cuda.current_device() != ws.Ebp.device.index:
+            # the launch below goes to the current device
+            return ws.Ebp[:ws.B] + ws.Eext[:ws.B, 0] + ws.Eext[:ws.B, 1]
         E = torch.empty(ws.B, dtype=torch.float64, device=ws.Ebp.device)
         self.lib.tm_total_energy(ws.B, _P(ws.Ebp), _P(ws.Eext), _P(E), self._stream())
         return E
