@@ -35,6 +35,7 @@ struct CellGrid {
   int ny, nrow;            // stencil rows per z layer, and in all
   unsigned magic;          // ceil(2^32 / ny): t / ny = (t magic) >> 32 for the row numbers here (ny > 1)
   double len[3], inv_len[3];   // axis lengths nc cs and their reciprocals
+  float flo[3], fhi[3];    // bounds of a centre's offset inside its cell (tm_centre)
   float rc2, inv_cs0;      // squared trimmed cutoff, 1 / cs[0]
 };
 
@@ -57,6 +58,8 @@ inline void tm_set_stencil(CellGrid& g, float rc) {
     g.full[d] = g.periodic && (2 * ((int)ceilf(rc / g.cs[d]) + 1) + 1 >= g.nc[d]);
     g.len[d] = (double)g.nc[d] * (double)g.cs[d];
     g.inv_len[d] = 1.0 / g.len[d];
+    g.flo[d] = g.periodic ? -g.cs[d] : 0.f;
+    g.fhi[d] = !g.periodic ? g.cs[d] : (g.nc[d] < 3 ? 2.f : 1.5f) * g.cs[d];
   }
   g.ny = g.full[1] ? g.nc[1] : 2 * g.k[1] + 1;
   g.nrow = g.ny * (g.full[2] ? g.nc[2] : 2 * g.k[2] + 1);
@@ -88,11 +91,23 @@ struct RangeLds {
   int mark[64];   // range starts inside the current chunk, tagged with the chunk's base
 };
 
-// A centre's cell and its offset inside the cell, in [0, cs] on an open grid.
+// A centre's cell and its offset inside the cell.
+//
+// A centre outside an open grid sits in an edge cell and is taken to that
+// cell's face.  Taking centre and candidate into the grid never makes them
+// further apart, so with the centre there all distances to bands of cells and
+// the range along x bound the true ones from below; its own band, for one, can
+// hold atoms that are as far outside.
+// PERIODIC 1 or 0: what the grid is, where the kernel knows it; -1: the bounds
+// come with the grid, one instruction per axis (a branch on g.periodic cost the
+// periodic rows 0.5 us).  A periodic grid's bounds lie outside every offset a
+// coordinate has (which is off by a whole cell only on axes of one or two) and
+// hold those that have lost their digits near the grid.
 struct CellCentre {
   int c[3];
   float f[3];
 };
+template <int PERIODIC = -1>
 __device__ __forceinline__ CellCentre tm_centre(const CellGrid& g, int cell, double px, double py,
                                                 double pz) {
   CellCentre o;
@@ -100,22 +115,18 @@ __device__ __forceinline__ CellCentre tm_centre(const CellGrid& g, int cell, dou
   o.c[1] = (cell / g.nc[0]) % g.nc[1];
   o.c[2] = cell / (g.nc[0] * g.nc[1]);
   const double p[3] = {px, py, pz};
+  const bool periodic = PERIODIC < 0 ? g.periodic : PERIODIC;
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
     double u = p[d] - (double)g.org[d];
-    if (g.periodic && g.nc[d] < 3) u -= g.len[d] * floor(u / g.len[d]);
+    if (periodic && g.nc[d] < 3) u -= g.len[d] * floor(u / g.len[d]);
     u -= (double)o.c[d] * (double)g.cs[d];
     // wrapped in FP64, so unwrapped coordinates keep their precision; the
     // offset lies within a cell of a multiple of the length, so the nearest one is it
-    if (g.periodic && g.nc[d] >= 3) u -= g.len[d] * rint(u * g.inv_len[d]);
-    float f = (float)u;   // offset inside the centre's cell
-    // A centre outside an open grid sits in an edge cell: it is taken to that
-    // cell's face.  Taking centre and candidate into the grid never makes them
-    // further apart, so with the centre there all distances to bands of cells
-    // and the range along x bound the true ones from below; its own band, for
-    // one, can hold atoms that are as far outside.
-    if (!g.periodic) f = fminf(fmaxf(f, 0.f), g.cs[d]);
-    o.f[d] = f;
+    if (periodic && g.nc[d] >= 3) u -= g.len[d] * rint(u * g.inv_len[d]);
+    o.f[d] = (float)u;   // offset inside the centre's cell
+    if (PERIODIC == 0) o.f[d] = __builtin_amdgcn_fmed3f(o.f[d], 0.f, g.cs[d]);
+    if (PERIODIC < 0) o.f[d] = __builtin_amdgcn_fmed3f(o.f[d], g.flo[d], g.fhi[d]);
   }
   return o;
 }

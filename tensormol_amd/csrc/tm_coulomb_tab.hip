@@ -197,8 +197,9 @@ coulomb_tab_kernel(int N, const float4* __restrict__ xqc, const int* __restrict_
       __syncwarp();
     }
   };
-  tm_sweep_list(grid, tm_centre(grid, grid.cell_of[i], (double)pi.x, (double)pi.y, (double)pi.z),
-                list[w], lane, load, visit);
+  tm_sweep_list(
+      grid, tm_centre<PERIODIC>(grid, grid.cell_of[i], (double)pi.x, (double)pi.y, (double)pi.z),
+      list[w], lane, load, visit);
   if (pending) pair.finish(a, pi.w, acc);
   if (lane < qn) {
     begin();

@@ -77,6 +77,9 @@ __device__ __forceinline__ double sq_dist_nocontract(double xi, double yi, doubl
 // atoms, divisions by the box edges, a search over ranges and block barriers
 // made it 20.6 us for the 12,288-atom box; now 18.6, lists and descriptors
 // 64.6 -> 61.0.
+// BOX false (no boxes): the images' FP64 operations, half of a test, are left
+// out.  A kernel of its own: a branch cost the periodic rows 0.8 us.
+template <bool BOX>
 __global__ void __launch_bounds__(NL_WAVES * 64)
 nl_rows_kernel(int N, const double* __restrict__ pos, const int* __restrict__ elem,
                const int* __restrict__ mol, const int* __restrict__ mol_start,
@@ -96,18 +99,16 @@ nl_rows_kernel(int N, const double* __restrict__ pos, const int* __restrict__ el
   const int mi = mol[i];
   const double xi = pos[3 * (long)i], yi = pos[3 * (long)i + 1], zi = pos[3 * (long)i + 2];
   double Lx = 0, Ly = 0, Lz = 0, iLx = 0, iLy = 0, iLz = 0;
-  if (box != nullptr) {
+  if constexpr (BOX) {
     Lx = box[3 * mi]; Ly = box[3 * mi + 1]; Lz = box[3 * mi + 2];
     iLx = Lx > 0.0 ? 1.0 / Lx : 0.0;
     iLy = Ly > 0.0 ? 1.0 / Ly : 0.0;
     iLz = Lz > 0.0 ? 1.0 / Lz : 0.0;
   }
   int count = 0;   // wave-uniform
-  // candidate j at (x, y, z); self and other molecules are not taken.  Without
-  // boxes the images' FP64 operations, half of a test, are left out.
+  // candidate j at (x, y, z); self and other molecules are not taken
   auto test = [&](double x, double y, double z, int j, bool take) {
-    const double s = box != nullptr
-                         ? sq_dist_nocontract(xi, yi, zi, x, y, z, Lx, Ly, Lz, iLx, iLy, iLz)
+    const double s = BOX ? sq_dist_nocontract(xi, yi, zi, x, y, z, Lx, Ly, Lz, iLx, iLy, iLz)
                          : sq_dist_nocontract(xi, yi, zi, x, y, z);
     const bool ok = take & (s < s_r);
     const unsigned long long bal = __ballot(ok);
@@ -633,7 +634,8 @@ int tm_nl_build(int N, const double* pos, const int* elem, const int* mol, const
   hipStream_t s = (hipStream_t)stream;
   CellGrid g = make_grid(cell_start, cell_atoms, cell_of, cell_pos, posc, molc, nx, ny, nz, csx, csy,
                          csz, ox, oy, oz, periodic, rc);
-  nl_rows_kernel<<<tm_div_up(N, NL_WAVES), NL_WAVES * 64, 0, s>>>(
+  const auto rows = box != nullptr ? nl_rows_kernel<true> : nl_rows_kernel<false>;
+  rows<<<tm_div_up(N, NL_WAVES), NL_WAVES * 64, 0, s>>>(
       N, pos, elem, mol, mol_start, box, g, nele, s_r, s_a, ldr, lda, nbr, ncnt, rseg,
       ang, acnt, aseg, flags);
   TM_LAUNCH_CHECK();
