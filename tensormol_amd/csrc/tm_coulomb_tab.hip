@@ -55,6 +55,19 @@ struct CtShape {
   static constexpr int WAVES = LT ? 8 : 4, LIST = LT ? 576 : 768;
 };
 
+// Whether workgroups of eight waves share a CU's LDS with their tables, for nb
+// of them on ncu CUs.  Where they leave the last of up to four rounds at most
+// half full, four-wave workgroups that read the tables from memory spread more
+// evenly (LDS / memory, us; periodic water): 3,000 atoms 40.3 / 37.2, 3,600 41.1
+// / 42.6, 4,320 49.5 / 45.5, 4,680 52.5 / 47.6, 5,616 52.4 / 53.2, 6,591 66.5 /
+// 58.1, 7,644 62.5 / 68.3, 8,820 66.4 / 67.8, 10,800 75.0 / 74.2, 12,288 76.8 /
+// 82.4.  Open systems, whose waves differ more, gain nothing: 3,000 27.2 / 27.2,
+// 5,000 31.3 / 31.9.
+inline bool ct_lds_tables(long nb, long ncu) {
+  const long rest = nb % ncu;
+  return nb <= ncu || nb >= 4 * ncu || rest == 0 || 2 * rest > ncu;
+}
+
 struct ClArgs {
   float rc2;       // cutoff (A), squared
   float inv_h;     // intervals per A
@@ -361,7 +374,13 @@ int tm_coulomb_tab(int N, const double* box, const int* cell_start, const int* c
   g.org[0] = (float)ox; g.org[1] = (float)oy; g.org[2] = (float)oz;
   g.periodic = periodic;
   tm_set_stencil(g, (float)rc_ee);
-  const bool lt = ntab * nint <= CT_LDS_TABLE;
+  bool lt = ntab * nint <= CT_LDS_TABLE;
+  if (lt && periodic) {
+    int dev = 0, ncu = 0;
+    TM_HIP_CHECK(hipGetDevice(&dev));
+    TM_HIP_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    lt = ct_lds_tables(tm_div_up(N, CtShape<true>::WAVES), ncu);
+  }
   const auto k = periodic ? (lt ? coulomb_tab_kernel<true, true> : coulomb_tab_kernel<true, false>)
                           : (lt ? coulomb_tab_kernel<false, true> : coulomb_tab_kernel<false, false>);
   const int waves = lt ? CtShape<true>::WAVES : CtShape<false>::WAVES;
