@@ -190,7 +190,9 @@ coulomb_tab_kernel(int N, const float4* __restrict__ xqc, const int* __restrict_
       d.z = cl_min_image(d.z, Lz, iLz);
     }
     d.w = c.x.w;
-    const bool near = d.x * d.x + d.y * d.y + d.z * d.z < a.rc2;
+    // written out: left to the compiler, the loop's copies fused it in two ways,
+    // and a pair at the cutoff's last digit counted in one and not in another
+    const bool near = fmaf(d.z, d.z, fmaf(d.x, d.x, d.y * d.y)) < a.rc2;
     const bool ok = near && p != cpi && valid;
     const unsigned long long bal = __builtin_amdgcn_ballot_w64(ok);
     if (ok) {
