@@ -240,17 +240,6 @@ __device__ inline int tm_build_ranges(int i, const CellGrid& g, RangeLds<CAP>& R
   return __builtin_amdgcn_readfirstlane(carry);   // the same in every lane
 }
 
-// Position (in cell order) of the t-th candidate: binary search in pre.
-template <int CAP>
-__device__ __forceinline__ int tm_candidate(const RangeLds<CAP>& R, int nr, int t) {
-  int lo = 0, hi = nr;   // find r with pre[r] <= t < pre[r+1]
-  while (hi - lo > 1) {
-    int mid = (lo + hi) >> 1;
-    if (R.pre[mid] <= t) lo = mid; else hi = mid;
-  }
-  return R.lo[lo] + (t - R.pre[lo]);
-}
-
 // Cell-order position of candidate base + lane of a sweep over the ranges in R
 // (0 for base + lane >= total), and r0 advanced from the range holding
 // candidate base to the range holding base + 64.  Call with base = 0, 64,

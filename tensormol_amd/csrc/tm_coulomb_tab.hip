@@ -38,7 +38,9 @@
 namespace {
 
 constexpr double CL_BOHRPERA = 1.889725989;
-constexpr int CT_RANGES = 480;   // stencils of more ranges are refused (tm_coulomb's bound)
+// Stencils of more ranges are refused: tm_coulomb's bound, so that both sweeps
+// take the same grids.  The list here would hold any number.
+constexpr int CT_RANGES = 480;
 constexpr int CT_QCAP = 128;     // compacted pair queue per wave (a ring)
 constexpr int CL_TABLE_MAX = 3072;   // float4 table entries (48 KiB)
 // Tables of up to this many entries (16 KiB, two elements) are copied to LDS,
@@ -358,9 +360,8 @@ int tm_coulomb_tab(int N, const double* box, const int* cell_start, const int* c
   const int nc[3] = {nx, ny, nz};
   const int need = tm_range_bound(rc_ee, cs, nc, periodic);
   TM_REQUIRE(need <= CT_RANGES,
-             "tm_coulomb_tab: cells of %.2f A are too small for a %.1f A cutoff (a sweep "
-             "could need %d candidate ranges, room for %d)", fmin(csx, fmin(csy, csz)), rc_ee,
-             need, CT_RANGES);
+             "tm_coulomb_tab: cells of %.2f A are too small for a %.1f A cutoff (a sweep of "
+             "%d candidate ranges, at most %d)", fmin(csx, fmin(csy, csz)), rc_ee, need, CT_RANGES);
   if (N == 0) return TM_OK;
   ClArgs a;
   a.rc2 = (float)(rc_ee * rc_ee);

@@ -29,7 +29,7 @@ namespace {
 
 constexpr int NL_WAVES = 4;           // waves per block, one centre per wave
 constexpr int NL_LDS_CAP = 256;       // candidate buffer per wave
-constexpr int NL_RANGES = 192;        // stencil ranges of a 4.6 A sweep over ~2.3 A cells
+constexpr int NL_RANGES = 192;        // finer grids than this many stencil ranges are refused
 constexpr int NL_LIST = 256;          // candidate list per wave
 
 __device__ __forceinline__ double sq_dist_nocontract(double xi, double yi, double zi, double xj,
@@ -69,8 +69,8 @@ __device__ __forceinline__ double sq_dist_nocontract(double xi, double yi, doubl
   return s;
 }
 
-// One wavefront per centre: candidates from the molecule or from the cell list
-// (their loads one chunk ahead), kept ones as (atom, near) until the sweep is
+// One wavefront per centre: candidates from the molecule, or from the cell list
+// with their loads one chunk ahead; kept ones as (atom, near) until the sweep is
 // over, then their elements in one round of loads, a rank sort and the segment
 // counts.  What bounds it: a chain of five dependent loads and some 700 vector
 // instructions per centre.  Elements read chunk by chunk behind the cell's
